@@ -2,13 +2,12 @@
  * og_bin.c -- one-time build of the binned pull's edge layout (og_bin.h)
  * from a PageRank plan whose rows keep the reference's in-neighbour order.
  *
- * Host: the rows are packed into bins (from the plan's row offsets), the
- * rows of more than OG_BIN_CAP in-edges are cut into pieces, and, once the
- * device has sorted the edges into tiles, the tiles are ordered segment by
- * segment (the gather's source order) and every quad of 16 sources gets
- * its run of entries.
- * Device: the (bin, segment) keys, their stable radix sort, the entries'
- * source and slot indices, and the tile boundaries.
+ * Device: the runs of equal in-degree of the (in-degree-ordered) rows; the
+ * tiles' sizes by a histogram of each bin's segments and their places by
+ * prefix sums; then each bin's entries, sources and quads.
+ * Host: the rows are packed into bins run by run, the rows of more than
+ * OG_BIN_CAP in-edges are cut into pieces, and each segment's sources into
+ * work items.
  */
 #include <stdio.h>
 #include <stdlib.h>
@@ -78,13 +77,6 @@ static void *og_vec_push(og_vec *v)
         v->cap = c;
     }
     return (char *)v->p + (v->n++) * v->elem;
-}
-
-static int og_bits(uint64_t x)
-{
-    int b = 0;
-    while (b < 64 && (1ull << b) <= x) b++;
-    return b;
 }
 
 /* Device copy of a host array (NULL and error set on failure). */
@@ -208,6 +200,166 @@ out:
     return rc;
 }
 
+/* Runs of equal in-degree of the rows [0, Z): (first row, in-degree),
+ * ascending by row; what the packing of rows into bins needs of the row
+ * offsets.  A relabelled plan orders its rows by in-degree, so there are at
+ * most about sqrt(2 E) runs and the device lists them; a plan in original
+ * order (relabel 0) has its row offsets read back instead. */
+typedef struct
+{
+    uint32_t row, deg;
+} og_bin_run;
+
+static int og_bin_run_cmp(const void *a, const void *b)
+{
+    const uint32_t x = ((const og_bin_run *)a)->row, y = ((const og_bin_run *)b)->row;
+    return x < y ? -1 : x > y;
+}
+
+static int og_bin_runs(const og_plan *pl, og_vec *runs)
+{
+    const uint32_t Z = pl->Z;
+    hipStream_t s = og_stream();
+    int rc = -1;
+    if (pl->relabel)
+    {
+        uint64_t cap = 64;
+        while (cap * cap < 2ull * pl->E) cap += cap / 8;
+        cap += 64;
+        uint32_t *d = og_dalloc(16 + cap * sizeof(og_bin_run));
+        og_bin_run *h = (og_bin_run *)malloc(16 + cap * sizeof(og_bin_run));
+        uint32_t n = 0;
+        if (!h) og_set_error("out of host memory");
+        if (d && h && !og_launch_fill_u32(d, 0, 4, s) &&
+            !og_launch_bin_runs(pl->row_ptr, Z, d + 4, (uint32_t)cap, d, s) &&
+            !og_hip_check(og_copy(h, d, 16 + cap * sizeof(og_bin_run), hipMemcpyDeviceToHost), "D2H row runs"))
+        {
+            n = *(const uint32_t *)h;
+            if (n <= cap)
+            {
+                const og_bin_run *r = (const og_bin_run *)((const char *)h + 16);
+                rc = 0;
+                for (uint32_t i = 0; i < n && !rc; i++)
+                {
+                    og_bin_run *o = (og_bin_run *)og_vec_push(runs);
+                    if (o) *o = r[i];
+                    else { og_set_error("out of host memory"); rc = -1; }
+                }
+                if (!rc) qsort(runs->p, runs->n, sizeof(og_bin_run), og_bin_run_cmp);
+            }
+        }
+        og_dfree(d);
+        free(h);
+        if (!rc || n <= cap) return rc;
+    }
+    uint32_t *rp = (uint32_t *)malloc(((size_t)Z + 1) * 4);
+    if (!rp) { og_set_error("out of host memory"); return -1; }
+    rc = og_hip_check(og_copy(rp, pl->row_ptr, ((size_t)Z + 1) * 4, hipMemcpyDeviceToHost), "D2H row_ptr");
+    for (uint32_t r = 0; r < Z && !rc; r++)
+    {
+        const uint32_t d = rp[r + 1] - rp[r];
+        if (r && d == ((og_bin_run *)runs->p)[runs->n - 1].deg) continue;
+        og_bin_run *o = (og_bin_run *)og_vec_push(runs);
+        if (!o) { og_set_error("out of host memory"); rc = -1; break; }
+        o->row = r;
+        o->deg = d;
+    }
+    free(rp);
+    return rc;
+}
+
+/* Long rows (more than OG_BIN_CAP in-edges) and bins: first the pieces of
+ * the long rows (OG_BIN_CAP in-edges each, in CSR order), then consecutive
+ * rows of one kind (thread rows, wavefront rows of more than OG_BIN_WAVE_ROW
+ * in-edges) with at most OG_BIN_CAP in-edges and OG_BIN_RPT * OG_BIN_THREADS
+ * rows together. */
+typedef struct
+{
+    uint32_t row, deg, bin;
+} og_bin_long;
+
+static int og_bin_long_cmp(const void *a, const void *b)
+{
+    const og_bin_long *x = (const og_bin_long *)a, *y = (const og_bin_long *)b;
+    if (x->deg != y->deg) return x->deg > y->deg ? -1 : 1;
+    return x->row < y->row ? -1 : x->row > y->row;
+}
+
+static int og_bin_pack(const og_plan *pl, const og_vec *runs, og_vec *bins, og_vec *longs)
+{
+    const og_bin_run *run = (const og_bin_run *)runs->p;
+    const uint32_t Z = pl->Z;
+    uint32_t pos = 0;
+    for (size_t i = 0; i < runs->n; i++)
+    {
+        const uint32_t r1 = i + 1 < runs->n ? run[i + 1].row : Z, deg = run[i].deg;
+        if (deg <= OG_BIN_CAP)
+        {
+            pos += (r1 - run[i].row) * deg;
+            continue;
+        }
+        for (uint32_t r = run[i].row; r < r1; r++, pos += deg)
+        {
+            og_bin_long *l = (og_bin_long *)og_vec_push(longs);
+            if (!l) return -1;
+            l->row = r;
+            l->deg = deg;
+            l->bin = (uint32_t)bins->n;
+            for (uint32_t p0 = 0; p0 < deg; p0 += OG_BIN_CAP)
+            {
+                og_bin_desc *d = (og_bin_desc *)og_vec_push(bins);
+                if (!d) return -1;
+                memset(d, 0, sizeof(*d));
+                d->row0 = r;
+                d->row1 = (uint32_t)longs->n - 1;
+                d->pos0 = pos + p0;
+                d->kind = OG_BIN_PIECE;
+                d->cnt = deg - p0 < OG_BIN_CAP ? deg - p0 : OG_BIN_CAP;
+            }
+        }
+    }
+    og_bin_desc *d = NULL;   /* the open bin (the last one) */
+    pos = 0;
+    for (size_t i = 0; i < runs->n; i++)
+    {
+        const uint32_t r1 = i + 1 < runs->n ? run[i + 1].row : Z, deg = run[i].deg;
+        const uint32_t kind = deg > OG_BIN_WAVE_ROW ? OG_BIN_WAVE_ROWS : OG_BIN_THREAD_ROWS;
+        uint32_t r = run[i].row;
+        if (deg > OG_BIN_CAP)
+        {
+            pos += (r1 - r) * deg;
+            d = NULL;
+            continue;
+        }
+        while (r < r1)
+        {
+            uint32_t room = 0;
+            if (d && d->kind == kind)
+            {
+                room = (OG_BIN_CAP - d->cnt) / deg;
+                const uint32_t rows = OG_BIN_RPT * OG_BIN_THREADS - (d->row1 - d->row0);
+                if (room > rows) room = rows;
+            }
+            if (!room)
+            {
+                d = (og_bin_desc *)og_vec_push(bins);
+                if (!d) return -1;
+                memset(d, 0, sizeof(*d));
+                d->row0 = d->row1 = r;
+                d->pos0 = pos;
+                d->kind = kind;
+                continue;
+            }
+            if (room > r1 - r) room = r1 - r;
+            d->row1 += room;
+            d->cnt += room * deg;
+            pos += room * deg;
+            r += room;
+        }
+    }
+    return 0;
+}
+
 int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
 {
     *out = NULL;
@@ -223,118 +375,40 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
         return -1;
     }
     og_bin_plan *b = (og_bin_plan *)calloc(1, sizeof(og_bin_plan));
-    uint32_t *rp = (uint32_t *)malloc(((size_t)N + 1) * 4);
-    og_vec bins = {NULL, 0, 0, sizeof(og_bin_desc)};
-    uint32_t *long_rows = NULL, *long_list = NULL, *long_bin_rowordered = NULL, *long_bin = NULL;
-    uint32_t *tseg = NULL, *tbin = NULL, *tstart = NULL, *tcnt = NULL, *tent = NULL, *order = NULL;
-    uint32_t *seg_cnt = NULL, *tsrc = NULL, *seg_src = NULL, *qent = NULL;
-    og_vec items = {NULL, 0, 0, sizeof(og_bin_item)};
-    uint32_t *key_a = NULL, *val_a = NULL, *key_b = NULL, *val_b = NULL;
-    void *scratch = NULL, *d_tseg = NULL, *d_tbin = NULL, *d_tstart = NULL, *d_tent = NULL, *d_tcnt = NULL;
-    void *d_tsrc = NULL;
+    og_vec runs = {NULL, 0, 0, sizeof(og_bin_run)}, bins = {NULL, 0, 0, sizeof(og_bin_desc)};
+    og_vec longs = {NULL, 0, 0, sizeof(og_bin_long)}, items = {NULL, 0, 0, sizeof(og_bin_item)};
+    uint32_t *ids = NULL, *seg_src = NULL, *rp = NULL;
+    uint32_t *d_quads = NULL, *d_bin_quads = NULL, *d_seg = NULL;
+    void *scratch = NULL;
     hipStream_t s = og_stream();
     int rc = -1;
-    if (!b || !rp)
+    if (!b)
     {
         og_set_error("out of host memory");
         goto done;
     }
-    if (og_hip_check(og_copy(rp, pl->row_ptr, ((size_t)N + 1) * 4, hipMemcpyDeviceToHost), "D2H row_ptr"))
-        goto done;
-
+    if (og_bin_runs(pl, &runs)) goto done;
+    if (og_bin_pack(pl, &runs, &bins, &longs))
     {
-        /* ---- long rows, longest first; their pieces first in the bin
-         * list (bins of OG_BIN_CAP in-edges each, in CSR order) ---- */
-        uint32_t n_long = 0;
-        for (uint32_t r = 0; r < Z; r++)
-            if (rp[r + 1] - rp[r] > OG_BIN_CAP) n_long++;
-        long_rows = (uint32_t *)malloc((size_t)(n_long + 1) * 4);
-        long_list = (uint32_t *)malloc((size_t)(n_long + 1) * 4);
-        long_bin_rowordered = (uint32_t *)malloc((size_t)(n_long + 1) * 4);
-        long_bin = (uint32_t *)malloc((size_t)(n_long + 1) * 4);
-        if (!long_rows || !long_list || !long_bin_rowordered || !long_bin)
-        {
-            og_set_error("out of host memory");
-            goto done;
-        }
-        uint32_t k = 0;
-        for (uint32_t r = 0; r < Z; r++)
-            if (rp[r + 1] - rp[r] > OG_BIN_CAP)
-            {
-                const uint32_t deg = rp[r + 1] - rp[r];
-                long_bin_rowordered[k] = (uint32_t)bins.n;
-                for (uint32_t p0 = 0; p0 < deg; p0 += OG_BIN_CAP)
-                {
-                    og_bin_desc *d = (og_bin_desc *)og_vec_push(&bins);
-                    if (!d) { og_set_error("out of host memory"); goto done; }
-                    memset(d, 0, sizeof(*d));
-                    d->row0 = r;
-                    d->row1 = k;
-                    d->pos0 = rp[r] + p0;
-                    d->kind = OG_BIN_PIECE;
-                    d->cnt = deg - p0 < OG_BIN_CAP ? deg - p0 : OG_BIN_CAP;
-                }
-                long_rows[k++] = r;
-            }
-        b->d.first_bin = (uint32_t)bins.n;
+        og_set_error("out of host memory");
+        goto done;
+    }
+    {
+        const uint32_t n_long = (uint32_t)longs.n, n_edge_bins = (uint32_t)bins.n;
         b->n_edges = E;
-        for (uint32_t i = 0; i < n_long; i++) b->long_terms += rp[long_rows[i] + 1] - rp[long_rows[i]];
-        uint32_t *lord = (uint32_t *)malloc((size_t)(n_long + 1) * 4);
-        if (!lord) { og_set_error("out of host memory"); goto done; }
-        for (uint32_t i = 0; i < n_long; i++) lord[i] = i;
-        for (uint32_t i = 1; i < n_long; i++)   /* insertion sort: few long rows */
-        {
-            uint32_t x = lord[i], dx = rp[long_rows[x] + 1] - rp[long_rows[x]];
-            int j = (int)i - 1;
-            while (j >= 0 && rp[long_rows[lord[j]] + 1] - rp[long_rows[lord[j]]] < dx)
-            {
-                lord[j + 1] = lord[j];
-                j--;
-            }
-            lord[j + 1] = x;
-        }
+        b->d.first_bin = 0;
+        for (uint32_t q = 0; q < n_edge_bins && ((og_bin_desc *)bins.p)[q].kind == OG_BIN_PIECE; q++) b->d.first_bin++;
+        /* the long rows, longest first, and each one's first piece */
+        if (n_long) qsort(longs.p, n_long, sizeof(og_bin_long), og_bin_long_cmp);
+        ids = (uint32_t *)malloc((size_t)(n_long + 1) * 8);
+        if (!ids) { og_set_error("out of host memory"); goto done; }
         for (uint32_t i = 0; i < n_long; i++)
         {
-            long_list[i] = long_rows[lord[i]];
-            long_bin[i] = long_bin_rowordered[lord[i]];
+            const og_bin_long *l = (const og_bin_long *)longs.p + i;
+            ids[i] = l->row;
+            ids[n_long + i] = l->bin;
+            b->long_terms += l->deg;
         }
-        free(lord);
-
-        /* ---- bins: consecutive rows of one kind (thread rows, wavefront
-         * rows of more than OG_BIN_WAVE_ROW in-edges) with at most
-         * OG_BIN_CAP in-edges and OG_BIN_RPT * OG_BIN_THREADS rows together
-         * (the long rows have their pieces already) ---- */
-        uint32_t r = 0;
-        while (r < Z)
-        {
-            const uint32_t deg = rp[r + 1] - rp[r];
-            if (deg > OG_BIN_CAP)
-            {
-                r++;
-                continue;
-            }
-            const uint32_t kind = deg > OG_BIN_WAVE_ROW ? OG_BIN_WAVE_ROWS : OG_BIN_THREAD_ROWS;
-            const uint32_t r0 = r;
-            uint32_t tot = 0;
-            while (r < Z)
-            {
-                const uint32_t dr = rp[r + 1] - rp[r];
-                const uint32_t kr = dr > OG_BIN_WAVE_ROW ? OG_BIN_WAVE_ROWS : OG_BIN_THREAD_ROWS;
-                if (kr != kind || dr > OG_BIN_CAP || tot + dr > OG_BIN_CAP || r - r0 == OG_BIN_RPT * OG_BIN_THREADS)
-                    break;
-                tot += dr;
-                r++;
-            }
-            og_bin_desc *d = (og_bin_desc *)og_vec_push(&bins);
-            if (!d) { og_set_error("out of host memory"); goto done; }
-            memset(d, 0, sizeof(*d));
-            d->row0 = r0;
-            d->row1 = r;
-            d->pos0 = rp[r0];
-            d->kind = kind;
-            d->cnt = tot;
-        }
-        const uint32_t n_edge_bins = (uint32_t)bins.n;
         /* rows without in-edges: epilogue-only bins, last */
         for (uint32_t r0 = Z; r0 < N; r0 += OG_BIN_ZERO_ROWS)
         {
@@ -343,12 +417,12 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
             memset(d, 0, sizeof(*d));
             d->row0 = r0;
             d->row1 = N - r0 < OG_BIN_ZERO_ROWS ? N : r0 + OG_BIN_ZERO_ROWS;
-            d->pos0 = rp[r0];
+            d->pos0 = E;
             d->kind = OG_BIN_THREAD_ROWS;
         }
         b->n_zero_bins = (uint32_t)bins.n - n_edge_bins;
         const uint32_t n_seg = (N + OG_BIN_SEG - 1) / OG_BIN_SEG;
-        if ((uint64_t)n_edge_bins * n_seg > 0xFFFFFFFFull)
+        if ((uint64_t)n_edge_bins * n_seg > 0xFFFF0000ull)
         {
             og_set_error("binned pull: graph too large for 32-bit tile keys");
             goto done;
@@ -359,152 +433,66 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
         b->d.n_bins_live = (uint32_t)bins.n;
         b->d.n_long = n_long;
 
-        /* ---- device: (bin, segment) keys of the CSR positions, stable sort,
-         * tile starts ---- */
-        og_bin_desc *hb = (og_bin_desc *)bins.p;
+        /* ---- device: the tiles' sizes in quads (16 entries), segment by
+         * segment; prefix sums give each tile's place among the sources and
+         * each bin's among the entries ---- */
+        const uint32_t n_cells = n_edge_bins * n_seg;
         b->mem_bins = og_bin_upload(bins.p, bins.n * sizeof(og_bin_desc));
-        key_a = og_dalloc(((size_t)E + 1) * 4);
-        val_a = og_dalloc(((size_t)E + 1) * 4);
-        key_b = og_dalloc(((size_t)E + 1) * 4);
-        val_b = og_dalloc(((size_t)E + 1) * 4);
-        size_t sb = og_radix_scratch_bytes(E), sc2 = og_scan_scratch_bytes(E);
-        scratch = og_dalloc(sb > sc2 ? sb : sc2);
-        if (!b->mem_bins || !key_a || !val_a || !key_b || !val_b || !scratch) goto done;
-        og_bin_desc *d_bins = (og_bin_desc *)b->mem_bins;
-        if (og_launch_bin_keys(d_bins, n_edge_bins, pl->cols, n_seg, key_b, val_b, s)) goto done;
-        int in_b = 0;
-        const uint32_t kbits = (uint32_t)og_bits((uint64_t)n_edge_bins * n_seg - 1);
-        if (og_radix_sort_pairs(key_b, val_b, key_a, val_a, key_b, val_b, E, kbits ? kbits : 1, scratch, s, &in_b))
-            goto done;
-        uint32_t *K = in_b ? key_b : key_a, *V = in_b ? val_b : val_a;
-        uint32_t *flag = in_b ? key_a : key_b, *fscan = in_b ? val_a : val_b;
-        if (og_launch_bin_flags(K, E, d_bins, n_seg, flag, s) || og_scan_exclusive(flag, fscan, E, scratch, s))
-            goto done;
-        uint32_t n_tiles = 0;
-        if (og_hip_check(og_copy(&n_tiles, fscan + E, 4, hipMemcpyDeviceToHost), "D2H tiles")) goto done;
-        b->n_tiles = n_tiles;
-        d_tseg = og_dalloc((size_t)n_tiles * 4);
-        d_tbin = og_dalloc((size_t)n_tiles * 4);
-        d_tstart = og_dalloc((size_t)n_tiles * 4);
-        if (!d_tseg || !d_tbin || !d_tstart) goto done;
-        if (og_launch_bin_tiles(K, E, n_seg, fscan, (uint32_t *)d_tseg, (uint32_t *)d_tbin, (uint32_t *)d_tstart, s))
-            goto done;
-        tseg = (uint32_t *)malloc((size_t)n_tiles * 4 + 4);
-        tbin = (uint32_t *)malloc((size_t)n_tiles * 4 + 4);
-        tstart = (uint32_t *)malloc((size_t)n_tiles * 4 + 4);
-        tcnt = (uint32_t *)malloc((size_t)n_tiles * 4 + 4);
-        tent = (uint32_t *)malloc((size_t)n_tiles * 4 + 4);
-        order = (uint32_t *)malloc((size_t)n_tiles * 4 + 4);
-        seg_cnt = (uint32_t *)calloc((size_t)n_seg + 1, 4);
-        tsrc = (uint32_t *)malloc((size_t)n_tiles * 4 + 4);
+        d_quads = og_dalloc(((size_t)n_cells + 1) * 4);
+        d_bin_quads = og_dalloc(((size_t)n_edge_bins + 1) * 4);
+        d_seg = og_dalloc(((size_t)n_seg + 1) * 4);
+        const size_t sc = og_scan_scratch_bytes(n_cells), sb = og_scan_scratch_bytes(n_edge_bins);
+        scratch = og_dalloc(sc > sb ? sc : sb);
         seg_src = (uint32_t *)malloc(((size_t)n_seg + 1) * 4);
-        if (!tseg || !tbin || !tstart || !tcnt || !tent || !order || !seg_cnt || !tsrc || !seg_src)
+        if (!seg_src) { og_set_error("out of host memory"); goto done; }
+        if (!b->mem_bins || !d_quads || !d_bin_quads || !d_seg || !scratch) goto done;
+        og_bin_desc *d_bins = (og_bin_desc *)b->mem_bins;
+        if (og_launch_bin_count(d_bins, n_edge_bins, pl->cols, n_seg, d_quads, d_bin_quads, s) ||
+            og_scan_exclusive(d_quads, d_quads, n_cells, scratch, s) ||
+            og_scan_exclusive(d_bin_quads, d_bin_quads, n_edge_bins, scratch, s) ||
+            og_launch_bin_place(d_bins, n_edge_bins, b->d.n_bins, d_bin_quads, d_quads, n_seg, d_seg, s) ||
+            og_hip_check(og_copy(seg_src, d_seg, ((size_t)n_seg + 1) * 4, hipMemcpyDeviceToHost), "D2H segments"))
+            goto done;
+        const uint64_t ent = (uint64_t)seg_src[n_seg] * OG_BIN_TILE_ALIGN;
+        if (ent + OG_BIN_SPARE > 0xFFFFFFFFull)
         {
-            og_set_error("out of host memory");
+            og_set_error("binned pull: graph too large for 32-bit entries");
             goto done;
         }
-        if (og_hip_check(og_copy(tseg, d_tseg, (size_t)n_tiles * 4, hipMemcpyDeviceToHost), "D2H tile seg") ||
-            og_hip_check(og_copy(tbin, d_tbin, (size_t)n_tiles * 4, hipMemcpyDeviceToHost), "D2H tile bin") ||
-            og_hip_check(og_copy(tstart, d_tstart, (size_t)n_tiles * 4, hipMemcpyDeviceToHost), "D2H tile start"))
-            goto done;
-
-        /* ---- host: tile sizes, their padded entry ranges, bins' entries ---- */
-        uint64_t ent = 0;
-        uint32_t bprev = 0xFFFFFFFFu;
-        for (uint32_t t = 0; t < n_tiles; t++)
-        {
-            tcnt[t] = (t + 1 < n_tiles ? tstart[t + 1] : E) - tstart[t];
-            if (tbin[t] != bprev)
-            {
-                if (bprev != 0xFFFFFFFFu) hb[bprev].ent1 = (uint32_t)ent;
-                bprev = tbin[t];
-                hb[bprev].ent0 = (uint32_t)ent;
-            }
-            tent[t] = (uint32_t)ent;
-            ent += (tcnt[t] + OG_BIN_TILE_ALIGN - 1) / OG_BIN_TILE_ALIGN * OG_BIN_TILE_ALIGN;
-            if (ent + OG_BIN_SPARE > 0xFFFFFFFFull)
-            {
-                og_set_error("binned pull: graph too large for 32-bit entries");
-                goto done;
-            }
-        }
-        if (bprev != 0xFFFFFFFFu) hb[bprev].ent1 = (uint32_t)ent;
-        for (uint32_t q = n_edge_bins; q < bins.n; q++) hb[q].ent0 = hb[q].ent1 = (uint32_t)ent;
         b->n_ent = ent + OG_BIN_SPARE;   /* spare entries past the last tile */
         b->d.n_ent = (uint32_t)ent;
-        /* the tiles segment by segment (bins ascending), and each tile's
-         * first entry in that order: where the gather reads its sources */
-        for (uint32_t t = 0; t < n_tiles; t++) seg_cnt[tseg[t] + 1]++;
-        for (uint32_t q = 0; q < n_seg; q++) seg_cnt[q + 1] += seg_cnt[q];
-        {
-            uint32_t *fill = (uint32_t *)malloc(((size_t)n_seg + 1) * 4);
-            if (!fill) { og_set_error("out of host memory"); goto done; }
-            memcpy(fill, seg_cnt, ((size_t)n_seg + 1) * 4);
-            for (uint32_t t = 0; t < n_tiles; t++) order[fill[tseg[t]]++] = t;
-            free(fill);
-        }
-        {
-            uint64_t f = 0;
-            for (uint32_t q = 0; q < n_seg; q++)
-            {
-                seg_src[q] = (uint32_t)f;
-                for (uint32_t i = seg_cnt[q]; i < seg_cnt[q + 1]; i++)
-                {
-                    tsrc[order[i]] = (uint32_t)f;
-                    f += (tcnt[order[i]] + OG_BIN_TILE_ALIGN - 1) / OG_BIN_TILE_ALIGN * OG_BIN_TILE_ALIGN;
-                }
-            }
-            seg_src[n_seg] = (uint32_t)f;   /* == ent */
-        }
         b->mem_src = og_dalloc(b->n_ent * 2);
         b->mem_pos = og_dalloc(b->n_ent * 2);
         b->mem_val = og_dalloc(b->n_ent * 4);
-        b->mem_long_row = og_bin_upload(long_list, (size_t)n_long * 4);
-        b->mem_long_bin = og_bin_upload(long_bin, (size_t)n_long * 4);
+        b->mem_qent = og_dalloc(ent / OG_BIN_TILE_ALIGN * 4);
+        b->mem_long_row = og_bin_upload(ids, (size_t)n_long * 4);
+        b->mem_long_bin = og_bin_upload(ids + n_long, (size_t)n_long * 4);
         b->mem_ticket = og_dalloc(256);
-        d_tent = og_bin_upload(tent, (size_t)n_tiles * 4);
-        d_tcnt = og_bin_upload(tcnt, (size_t)n_tiles * 4);
-        d_tsrc = og_bin_upload(tsrc, (size_t)n_tiles * 4);
-        if (!b->mem_src || !b->mem_pos || !b->mem_val || !b->mem_long_row || !b->mem_long_bin || !b->mem_ticket ||
-            !d_tent || !d_tcnt || !d_tsrc ||
-            og_hip_check(og_copy(d_bins, hb, bins.n * sizeof(og_bin_desc), hipMemcpyHostToDevice), "H2D bins"))
+        if (!b->mem_src || !b->mem_pos || !b->mem_val || !b->mem_qent || !b->mem_long_row || !b->mem_long_bin ||
+            !b->mem_ticket)
             goto done;
-        if (og_launch_bin_fill(K, V, E, d_bins, n_seg, pl->cols, fscan, (const uint32_t *)d_tstart,
-                               (const uint32_t *)d_tent, (const uint32_t *)d_tsrc, (uint16_t *)b->mem_src,
-                               (uint16_t *)b->mem_pos, s) ||
-            og_launch_bin_pads((const uint32_t *)d_tent, (const uint32_t *)d_tsrc, (const uint32_t *)d_tcnt, n_tiles,
-                               (uint16_t *)b->mem_src, (uint16_t *)b->mem_pos, s) ||
-            og_hip_check(hipMemsetAsync((uint16_t *)b->mem_src + ent, 0, OG_BIN_SPARE * 2, s), "memset slack") ||
-            og_hip_check(hipStreamSynchronize(s), "sync bin layout"))
+        if (og_launch_bin_fill(d_bins, n_edge_bins, pl->cols, n_seg, d_quads, (uint16_t *)b->mem_src,
+                               (uint16_t *)b->mem_pos, (uint32_t *)b->mem_qent, s) ||
+            og_launch_fill_u32((uint32_t *)((uint16_t *)b->mem_src + ent), 0, OG_BIN_SPARE / 2, s))
             goto done;
-        og_dfree(key_a); og_dfree(val_a); og_dfree(key_b); og_dfree(val_b); og_dfree(scratch);
-        key_a = val_a = key_b = val_b = NULL;
-        scratch = NULL;
 
-        /* ---- host: each quad's first entry (a tile's padded sources are
-         * whole quads), and the work items: each segment's sources in runs
-         * of at most OG_BIN_ITEM_SRC ---- */
-        const uint64_t n_quads = ent / OG_BIN_TILE_ALIGN;
-        qent = (uint32_t *)malloc(n_quads * 4 + 4);
-        if (!qent) { og_set_error("out of host memory"); goto done; }
-        for (uint32_t t = 0; t < n_tiles; t++)
-        {
-            const uint32_t P = (tcnt[t] + OG_BIN_TILE_ALIGN - 1) / OG_BIN_TILE_ALIGN * OG_BIN_TILE_ALIGN;
-            for (uint32_t k = 0; k < P; k += OG_BIN_TILE_ALIGN) qent[(tsrc[t] + k) / OG_BIN_TILE_ALIGN] = tent[t] + k;
-        }
+        /* ---- host: the work items: each segment's sources in runs of at
+         * most OG_BIN_ITEM_SRC ---- */
         for (uint32_t q = 0; q < n_seg; q++)
-            for (uint32_t f0 = seg_src[q]; f0 < seg_src[q + 1]; f0 += OG_BIN_ITEM_SRC)
+        {
+            const uint64_t end = (uint64_t)seg_src[q + 1] * OG_BIN_TILE_ALIGN;
+            for (uint64_t f0 = (uint64_t)seg_src[q] * OG_BIN_TILE_ALIGN; f0 < end; f0 += OG_BIN_ITEM_SRC)
             {
                 og_bin_item *it = (og_bin_item *)og_vec_push(&items);
                 if (!it) { og_set_error("out of host memory"); goto done; }
                 it->seg = q;
-                it->f0 = f0;
-                it->f1 = seg_src[q + 1] - f0 < OG_BIN_ITEM_SRC ? seg_src[q + 1] : f0 + OG_BIN_ITEM_SRC;
+                it->f0 = (uint32_t)f0;
+                it->f1 = (uint32_t)(end - f0 < OG_BIN_ITEM_SRC ? end : f0 + OG_BIN_ITEM_SRC);
                 it->pad = 0;
             }
-        b->mem_qent = og_bin_upload(qent, n_quads * 4);
+        }
         b->mem_items = og_bin_upload(items.p, items.n * sizeof(og_bin_item));
-        if (!b->mem_qent || !b->mem_items) goto done;
+        if (!b->mem_items) goto done;
         b->d.n_items = (uint32_t)items.n;
         b->d.items = (const og_bin_item *)b->mem_items;
         b->d.qent = (const uint32_t *)b->mem_qent;
@@ -515,16 +503,24 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
         b->d.long_row = (const uint32_t *)b->mem_long_row;
         b->d.long_bin = (const uint32_t *)b->mem_long_bin;
         b->d.ticket = (uint32_t *)b->mem_ticket;
-        if (getenv("OG_BIN_VERIFY") && og_bin_verify(b, pl, rp)) goto done;
+        if (getenv("OG_BIN_VERIFY"))
+        {
+            rp = (uint32_t *)malloc(((size_t)N + 1) * 4);
+            if (!rp) { og_set_error("out of host memory"); goto done; }
+            if (og_hip_check(og_copy(rp, pl->row_ptr, ((size_t)N + 1) * 4, hipMemcpyDeviceToHost), "D2H row_ptr") ||
+                og_bin_verify(b, pl, rp))
+                goto done;
+        }
     }
     rc = 0;
 done:
-    (void)hipStreamSynchronize(s);
-    og_dfree(key_a); og_dfree(val_a); og_dfree(key_b); og_dfree(val_b); og_dfree(scratch);
-    og_dfree(d_tseg); og_dfree(d_tbin); og_dfree(d_tstart); og_dfree(d_tent); og_dfree(d_tcnt); og_dfree(d_tsrc);
-    free(rp); free(bins.p); free(long_rows); free(long_list); free(long_bin_rowordered); free(long_bin);
-    free(tseg); free(tbin); free(tstart); free(tcnt); free(tent); free(order); free(seg_cnt);
-    free(items.p); free(tsrc); free(seg_src); free(qent);
+    if (hipStreamSynchronize(s) != hipSuccess && !rc)
+    {
+        og_set_error("binned pull: the layout's kernels failed");
+        rc = -1;
+    }
+    og_dfree(d_quads); og_dfree(d_bin_quads); og_dfree(d_seg); og_dfree(scratch);
+    free(runs.p); free(bins.p); free(longs.p); free(items.p); free(ids); free(seg_src); free(rp);
     if (rc) og_bin_plan_destroy(b);
     else *out = b;
     return rc;

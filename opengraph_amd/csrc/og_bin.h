@@ -7,7 +7,7 @@
  * segments of OG_BIN_SEG consecutive ids (their contributions fit in LDS).
  * The edges of bin b whose source lies in segment s form tile (b, s).
  * Entries (one per edge) are stored bin by bin, within a bin tile by tile
- * in segment order, within a tile in CSR order:
+ * in segment order, within a tile in any order:
  *   pos[e]  u16  the edge's CSR position minus the bin's first position
  *               (OG_BIN_PAD: a padding entry; each tile is padded to
  *               OG_BIN_TILE_ALIGN entries, so every tile's values fill whole
@@ -108,7 +108,7 @@ typedef struct og_bin_plan
 {
     og_bin_dev d;
     uint64_t n_ent;              /* entries (and sources) including padding and the spares */
-    uint32_t n_tiles, n_zero_bins;
+    uint32_t n_zero_bins;
     uint64_t n_edges, long_terms;  /* in-edges, and those of the long rows */
     /* device allocations */
     void *mem_items, *mem_qent, *mem_src, *mem_pos, *mem_val, *mem_bins;
@@ -131,26 +131,16 @@ uint32_t og_bin_long_grid(const og_bin_plan *b);
 int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, uint32_t it, uint32_t sum_grid,
                        uint32_t long_grid, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1);
 
-/* plan-build kernels */
-int og_launch_bin_keys(const og_bin_desc *bins, uint32_t n_bins, const uint32_t *cols, uint32_t n_seg,
-                       uint32_t *key, uint32_t *val, hipStream_t s);
-/* tile_flag[i] = 1 where sorted entry i starts a tile (a bin's first entry
- * or a change of key) */
-int og_launch_bin_flags(const uint32_t *key, uint32_t n, const og_bin_desc *bins, uint32_t n_seg,
-                        uint32_t *tile_flag, hipStream_t s);
-/* per tile t (from the exclusive scan of the flags): segment, bin, first
- * sorted entry */
-int og_launch_bin_tiles(const uint32_t *key, uint32_t n, uint32_t n_seg, const uint32_t *tile_flag_scan,
-                        uint32_t *tile_seg, uint32_t *tile_bin, uint32_t *tile_start, hipStream_t s);
-/* sorted entry i of tile t: pos at tile_ent[t] + (i - tile_start[t]), src
- * at tile_src[t] + (i - tile_start[t]); then the padding entries of every
- * tile (src 0, pos PAD) */
-int og_launch_bin_fill(const uint32_t *key, const uint32_t *val, uint32_t n, const og_bin_desc *bins,
-                       uint32_t n_seg, const uint32_t *cols, const uint32_t *tile_flag_scan,
-                       const uint32_t *tile_start, const uint32_t *tile_ent, const uint32_t *tile_src,
-                       uint16_t *src, uint16_t *pos, hipStream_t s);
-int og_launch_bin_pads(const uint32_t *tile_ent, const uint32_t *tile_src, const uint32_t *tile_cnt,
-                       uint32_t n_tiles, uint16_t *src, uint16_t *pos, hipStream_t s);
+/* plan-build kernels (og_bin.hip): the rows' runs of equal in-degree
+ * (pairs row, in-degree; *n zeroed by the caller), the tiles' sizes, their
+ * places, the entries */
+int og_launch_bin_runs(const uint32_t *row_ptr, uint32_t Z, uint32_t *runs, uint32_t cap, uint32_t *n, hipStream_t s);
+int og_launch_bin_count(const og_bin_desc *bins, uint32_t n_bins, const uint32_t *cols, uint32_t n_seg,
+                        uint32_t *quads, uint32_t *bin_quads, hipStream_t s);
+int og_launch_bin_place(og_bin_desc *bins, uint32_t n_bins, uint32_t n_all, const uint32_t *bin_quads,
+                        const uint32_t *quads, uint32_t n_seg, uint32_t *seg_src, hipStream_t s);
+int og_launch_bin_fill(const og_bin_desc *bins, uint32_t n_bins, const uint32_t *cols, uint32_t n_seg,
+                       const uint32_t *quads, uint16_t *src, uint16_t *pos, uint32_t *qent, hipStream_t s);
 
 #ifdef __cplusplus
 }
