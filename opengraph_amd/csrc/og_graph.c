@@ -239,7 +239,7 @@ int og_plan_build(const og_graph *g, uint32_t relabel, uint32_t seq_t, uint32_t 
     p->Z = C + cls[2];
     p->L = cls[4];
     /* 4. relabelled in-neighbour lists, reference order kept */
-    if (E && og_launch_plan_copy(H, N, p->new2old, p->old2new, g->i_edges_idx, g->i_dst, p->row_ptr,
+    if (E && og_launch_plan_copy(H, C, p->Z, p->new2old, p->old2new, g->i_edges_idx, g->i_dst, p->row_ptr,
                                  p->cols, s))
         goto done;
     /* 4b. rows [L, H) (several chunks; their sums are a fixed tree, not the
@@ -335,7 +335,7 @@ int og_plan_build(const og_graph *g, uint32_t relabel, uint32_t seq_t, uint32_t 
         if (og_launch_plan_map_pairs(E, g->f_src, g->f_dst, p->old2new, p->push_src, p->push_dst, s))
             goto done;
         if (og_scan_exclusive(p->outdeg, p->f_row_ptr, N, scratch, s)) goto done;
-        if (E && og_launch_plan_copy(0, N, p->new2old, p->old2new, g->f_edges_idx, g->f_dst,
+        if (E && og_launch_plan_copy(0, N, N, p->new2old, p->old2new, g->f_edges_idx, g->f_dst,
                                      p->f_row_ptr, p->f_cols, s))
             goto done;
     }

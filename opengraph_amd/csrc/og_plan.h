@@ -26,8 +26,9 @@ int og_launch_plan_perm(uint32_t N, const uint32_t *new2old, const uint32_t *out
                         const uint32_t *indeg_old, uint32_t seq_t, uint32_t chain_t, uint32_t *old2new,
                         uint32_t *outdeg_new, uint32_t *indeg_new, uint32_t *class_cnt,
                         hipStream_t s);
-/* cols of rows [0, N): a block per row below H, a wavefront per row above. */
-int og_launch_plan_copy(uint32_t H, uint32_t N, const uint32_t *new2old, const uint32_t *old2new,
+/* cols of rows [0, Z): several 64-lane groups per row below H, one below C,
+ * 8 lanes per row above. */
+int og_launch_plan_copy(uint32_t H, uint32_t C, uint32_t Z, const uint32_t *new2old, const uint32_t *old2new,
                         const uint32_t *idx_old, const uint32_t *lists, const uint32_t *row_ptr,
                         uint32_t *cols, hipStream_t s);
 /* rowid[e - base] = r for every edge e of the rows [0, R) of row_ptr. */

@@ -175,41 +175,55 @@ __global__ void og_plan_perm_kernel(uint32_t N, const uint32_t *__restrict__ new
         cnt[og_row_class(d, seq_t)]++;
         if (chain_t && d > chain_t) cnt[4]++;
     }
+    /* one atomic per block and class: the five counters are one cache line
+     * for the whole grid (an atomic per thread took 760 us at 2^22 rows) */
+    __shared__ uint32_t s_cnt[5];
+    if (threadIdx.x < 5) s_cnt[threadIdx.x] = 0;
+    __syncthreads();
     for (int k = 0; k < 5; k++)
-        if (cnt[k]) atomicAdd(&class_cnt[k], cnt[k]);
+    {
+        uint32_t c = cnt[k];
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+        if (c && (threadIdx.x & 63) == 0) atomicAdd(&s_cnt[k], c);
+    }
+    __syncthreads();
+    if (threadIdx.x < 5 && s_cnt[threadIdx.x]) atomicAdd(&class_cnt[threadIdx.x], s_cnt[threadIdx.x]);
 }
 
-/* cols[row_ptr[i] + k] = old2new[src_list[idx_old[o] + k]], o = new2old[i]:
- * one wavefront per row for rows [r0, r1). */
+/* cols[row_ptr[i] + k] = old2new[lists[idx_old[o] + k]], o = new2old[i]: G
+ * lanes per row for rows [r0, r1), in gridDim.y parts each.  Rows come longest
+ * first, so G follows the row class: 64 lanes and several parts for the rows
+ * of several chunks, 64 for those of one chunk, 8 for the short ones (a
+ * wavefront per short row left most of its lanes idle: 710 us at R-MAT-22, and
+ * a single block for the longest row 610 us; now 115 and 290 us). */
+#define OG_COPY_PARTS 16u
+template <uint32_t G>
 __global__ __launch_bounds__(OG_BLOCK) void og_plan_copy_rows_kernel(
     uint32_t r0, uint32_t r1, const uint32_t *__restrict__ new2old,
     const uint32_t *__restrict__ old2new, const uint32_t *__restrict__ idx_old,
     const uint32_t *__restrict__ lists, const uint32_t *__restrict__ row_ptr,
     uint32_t *__restrict__ cols)
 {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
-    for (uint32_t i = r0 + wave; i < r1; i += nwaves)
+    const uint32_t lane = threadIdx.x % G;
+    const uint32_t group = (blockIdx.x * blockDim.x + threadIdx.x) / G;
+    const uint32_t groups = (gridDim.x * blockDim.x) / G;
+    for (uint64_t i = (uint64_t)r0 + group; i < r1; i += groups)
     {
-        uint32_t o = new2old[i];
-        uint32_t src = idx_old[o];
-        uint32_t dst = row_ptr[i], n = row_ptr[i + 1] - dst;
-        for (uint32_t k = lane; k < n; k += 64) cols[dst + k] = old2new[lists[src + k] & OG_ID_MASK];
+        const uint32_t o = new2old[i];
+        const uint32_t src = idx_old[o];
+        const uint32_t dst = row_ptr[i], n = row_ptr[i + 1] - dst;
+        const uint32_t step = G * gridDim.y;
+        uint32_t k = blockIdx.y * G + lane;
+        for (; k < n && n - k > 3 * step; k += 4 * step)
+        {
+            uint32_t v[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) v[u] = lists[src + k + u * step] & OG_ID_MASK;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) cols[dst + k + u * step] = old2new[v[u]];
+        }
+        for (; k < n; k += step) cols[dst + k] = old2new[lists[src + k] & OG_ID_MASK];
     }
-}
-
-/* The same for the rows [0, H) (more than one chunk), one block per row. */
-__global__ __launch_bounds__(OG_BLOCK) void og_plan_copy_hubs_kernel(
-    const uint32_t *__restrict__ new2old, const uint32_t *__restrict__ old2new,
-    const uint32_t *__restrict__ idx_old, const uint32_t *__restrict__ lists,
-    const uint32_t *__restrict__ row_ptr, uint32_t *__restrict__ cols)
-{
-    uint32_t i = blockIdx.x;
-    uint32_t o = new2old[i];
-    uint32_t src = idx_old[o];
-    uint32_t dst = row_ptr[i], n = row_ptr[i + 1] - dst;
-    for (uint32_t k = threadIdx.x; k < n; k += OG_BLOCK) cols[dst + k] = old2new[lists[src + k] & OG_ID_MASK];
 }
 
 /* rowid[e - base] = r for the edges e of rows [0, R) of row_ptr, one
@@ -300,25 +314,25 @@ extern "C" int og_launch_plan_perm(uint32_t N, const uint32_t *new2old, const ui
                                    uint32_t *outdeg_new, uint32_t *indeg_new, uint32_t *class_cnt,
                                    hipStream_t s)
 {
-    OG_LAUNCH(og_plan_perm_kernel, dim3(og_grid(N, 16384)), dim3(OG_BLOCK), 0, s, N, new2old,
+    OG_LAUNCH(og_plan_perm_kernel, dim3(og_grid(N, 2048)), dim3(OG_BLOCK), 0, s, N, new2old,
                        outdeg_old, indeg_old, seq_t, chain_t, old2new, outdeg_new, indeg_new, class_cnt);
     return og_hip_check(og_launch_status(), "og_plan_perm_kernel");
 }
 
-extern "C" int og_launch_plan_copy(uint32_t H, uint32_t N, const uint32_t *new2old,
+extern "C" int og_launch_plan_copy(uint32_t H, uint32_t C, uint32_t Z, const uint32_t *new2old,
                                    const uint32_t *old2new, const uint32_t *idx_old,
                                    const uint32_t *lists, const uint32_t *row_ptr, uint32_t *cols,
                                    hipStream_t s)
 {
-    if (H) OG_LAUNCH(og_plan_copy_hubs_kernel, dim3(H), dim3(OG_BLOCK), 0, s, new2old, old2new,
-                              idx_old, lists, row_ptr, cols);
-    if (N > H)
-    {
-        uint64_t waves = N - H;
-        unsigned grid = (unsigned)((waves + 3) / 4 < 65536 ? (waves + 3) / 4 : 65536);
-        OG_LAUNCH(og_plan_copy_rows_kernel, dim3(grid), dim3(OG_BLOCK), 0, s, H, N, new2old,
-                           old2new, idx_old, lists, row_ptr, cols);
-    }
+    if (H)
+        OG_LAUNCH(og_plan_copy_rows_kernel<64>, dim3(og_grid((uint64_t)H * 64, 65536), OG_COPY_PARTS), dim3(OG_BLOCK), 0,
+                  s, 0u, H, new2old, old2new, idx_old, lists, row_ptr, cols);
+    if (C > H)
+        OG_LAUNCH(og_plan_copy_rows_kernel<64>, dim3(og_grid((uint64_t)(C - H) * 64, 65536)), dim3(OG_BLOCK), 0, s, H, C,
+                  new2old, old2new, idx_old, lists, row_ptr, cols);
+    if (Z > C)
+        OG_LAUNCH(og_plan_copy_rows_kernel<8>, dim3(og_grid((uint64_t)(Z - C) * 8, 65536)), dim3(OG_BLOCK), 0, s, C, Z,
+                  new2old, old2new, idx_old, lists, row_ptr, cols);
     return og_hip_check(og_launch_status(), "og_plan_copy");
 }
 
