@@ -23,40 +23,9 @@ void og_bin_plan_destroy(og_bin_plan *b)
 {
     if (!b) return;
     og_dfree(b->mem_items); og_dfree(b->mem_qent); og_dfree(b->mem_src);
-    og_dfree(b->mem_pos); og_dfree(b->mem_val); og_dfree(b->mem_bins); og_dfree(b->mem_long_row);
-    og_dfree(b->mem_long_bin); og_dfree(b->mem_ticket);
+    og_dfree(b->mem_pos); og_dfree(b->mem_val); og_dfree(b->mem_bins); og_dfree(b->mem_sched);
+    og_dfree(b->mem_blk);
     free(b);
-}
-
-/* Sum and long-row blocks take half a CU's LDS each: two block slots per
- * CU (a long-row block has twice the threads at half the registers).  The
- * long rows get up to one slot in eight, the sum pass the rest, side by
- * side.  Workgroups are dealt to the XCDs in turn, so the sum pass leaves a
- * whole number of slots per XCD free (the long-row blocks rounded up to a
- * multiple of OG_BIN_XCDS); otherwise a long-row block can find its XCD
- * full and wait for a sum block to end. */
-#define OG_BIN_XCDS 8u
-
-uint32_t og_bin_long_grid(const og_bin_plan *b)
-{
-    /* the long rows' share of the slots: their in-edges' share of E, times
-     * 1.6 (an in-edge costs a long-row block about 1.6 times what it costs
-     * the sum pass: R-MAT-24 measurements), in whole XCD rounds, between
-     * OG_BIN_XCDS and a quarter of the CUs */
-    const uint32_t cus = (uint32_t)og_num_cus();
-    const uint32_t cap = cus / 4 ? cus / 4 : 1;
-    uint64_t l = b->n_edges ? (uint64_t)(2.0 * cus * 1.6 * (double)b->long_terms / (double)b->n_edges) : 0;
-    l = (l + OG_BIN_XCDS - 1) / OG_BIN_XCDS * OG_BIN_XCDS;
-    if (l < OG_BIN_XCDS) l = OG_BIN_XCDS;
-    if (l > cap) l = cap;
-    return b->d.n_long < l ? b->d.n_long : (uint32_t)l;
-}
-
-uint32_t og_bin_sum_grid(const og_bin_plan *b)
-{
-    const uint32_t slots = 2u * (uint32_t)og_num_cus();   /* two blocks per CU */
-    const uint32_t l = (og_bin_long_grid(b) + OG_BIN_XCDS - 1) / OG_BIN_XCDS * OG_BIN_XCDS;
-    return slots > l ? slots - l : 1;
 }
 
 /* growable host arrays */
@@ -98,8 +67,8 @@ static void *og_bin_upload(const void *h, size_t bytes)
  * segment, each entry gathered once and its source the edge's (the CSR's
  * column at the entry's slot),
  * slots within their bins, bins and pieces within the entries, rows per bin,
- * CSR positions, the pieces first and each long row's pieces covering its
- * in-edges in order.  Runs before any binned kernel, so a bad layout
+ * CSR positions, the pieces first, and in the sum pass's lists every bin once
+ * and each long row's pieces in order.  Runs before any binned kernel, so a bad layout
  * is an error, not a stray access. */
 static int og_bin_verify(const og_bin_plan *b, const og_plan *pl, const uint32_t *rp)
 {
@@ -109,21 +78,23 @@ static int og_bin_verify(const og_bin_plan *b, const og_plan *pl, const uint32_t
     uint32_t *qent = (uint32_t *)malloc(nq * 4 + 4);
     uint16_t *src = (uint16_t *)malloc(ne * 2), *pos = (uint16_t *)malloc(ne * 2);
     og_bin_desc *bins = (og_bin_desc *)malloc((size_t)d->n_bins * sizeof(og_bin_desc) + 16);
-    uint32_t *lrow = (uint32_t *)malloc((size_t)d->n_long * 4 + 4), *lbin = (uint32_t *)malloc((size_t)d->n_long * 4 + 4);
+    og_bin_desc *sched = (og_bin_desc *)malloc((size_t)d->n_edge_bins * sizeof(og_bin_desc) + 16);
+    uint32_t *blk = (uint32_t *)malloc(((size_t)b->sum_grid + 1) * 4);
+    uint8_t *taken = (uint8_t *)calloc((size_t)d->n_bins + 1, 1);
     uint32_t *gsrc = (uint32_t *)malloc(ne * 4);   /* source id gathered into each entry */
     uint32_t *cols = (uint32_t *)malloc((size_t)pl->E * 4 + 4);
     uint8_t *seen = (uint8_t *)calloc(ne, 1);
     int rc = -1;
 #define OG_BIN_FAIL(...) do { og_set_error("binned layout check: " __VA_ARGS__); goto out; } while (0)
-    if (!items || !qent || !src || !pos || !bins || !lrow || !lbin || !seen || !gsrc || !cols)
+    if (!items || !qent || !src || !pos || !bins || !sched || !blk || !taken || !seen || !gsrc || !cols)
         OG_BIN_FAIL("out of host memory");
     if (og_hip_check(og_copy(items, d->items, (size_t)d->n_items * sizeof(og_bin_item), hipMemcpyDeviceToHost), "D2H") ||
         og_hip_check(og_copy(qent, d->qent, nq * 4, hipMemcpyDeviceToHost), "D2H") ||
         og_hip_check(og_copy(src, d->src, ne * 2, hipMemcpyDeviceToHost), "D2H") ||
         og_hip_check(og_copy(pos, d->pos, ne * 2, hipMemcpyDeviceToHost), "D2H") ||
         og_hip_check(og_copy(bins, d->bins, (size_t)d->n_bins * sizeof(og_bin_desc), hipMemcpyDeviceToHost), "D2H") ||
-        og_hip_check(og_copy(lrow, d->long_row, (size_t)d->n_long * 4, hipMemcpyDeviceToHost), "D2H") ||
-        og_hip_check(og_copy(lbin, d->long_bin, (size_t)d->n_long * 4, hipMemcpyDeviceToHost), "D2H") ||
+        og_hip_check(og_copy(sched, d->sched, (size_t)d->n_edge_bins * sizeof(og_bin_desc), hipMemcpyDeviceToHost), "D2H") ||
+        og_hip_check(og_copy(blk, d->blk, ((size_t)b->sum_grid + 1) * 4, hipMemcpyDeviceToHost), "D2H") ||
         og_hip_check(og_copy(cols, pl->cols, (size_t)pl->E * 4, hipMemcpyDeviceToHost), "D2H"))
         goto out;
     for (uint32_t q = 0; q < d->n_items; q++)
@@ -180,22 +151,43 @@ static int og_bin_verify(const og_bin_plan *b, const og_plan *pl, const uint32_t
         }
         if (real != bd.cnt) OG_BIN_FAIL("bin %u: %u entries for %u in-edges", q, real, bd.cnt);
     }
-    uint64_t pieces = 0;
-    for (uint32_t q = 0; q < d->n_long; q++)
+    /* the sum pass's order: every bin with edges in it once (the bins are
+     * told apart by their first entry), a long row's pieces one after the
+     * other in one block, the first and the last one marked */
+    if (blk[0] != 0 || blk[b->sum_grid] != d->n_edge_bins) OG_BIN_FAIL("block lists");
+    for (uint32_t i = 0; i < b->sum_grid; i++)
     {
-        const uint32_t r = lrow[q];
-        if (r >= pl->Z) OG_BIN_FAIL("long row %u", q);
-        const uint32_t n = rp[r + 1] - rp[r];
-        for (uint32_t c0 = 0, k = lbin[q]; c0 < n; c0 += OG_BIN_CAP, k++, pieces++)
-            if (k >= d->first_bin || bins[k].kind != OG_BIN_PIECE || bins[k].row0 != r || bins[k].pos0 != rp[r] + c0 ||
-                bins[k].cnt != (n - c0 < OG_BIN_CAP ? n - c0 : OG_BIN_CAP))
-                OG_BIN_FAIL("long row %u: piece %u", q, k);
+        if (blk[i + 1] < blk[i] || blk[i + 1] > d->n_edge_bins) OG_BIN_FAIL("block list %u", i);
+        uint32_t next = 0;   /* CSR position the long row under way goes on at, 0 for none */
+        for (uint32_t q = blk[i]; q < blk[i + 1]; q++)
+        {
+            uint32_t lo = 0, hi = d->n_edge_bins;
+            while (hi - lo > 1)
+            {
+                const uint32_t mid = (lo + hi) / 2;
+                if (bins[mid].ent0 <= sched[q].ent0) lo = mid;
+                else hi = mid;
+            }
+            if (memcmp(&bins[lo], &sched[q], sizeof(og_bin_desc)) || taken[lo]) OG_BIN_FAIL("block %u: bin %u", i, q);
+            taken[lo] = 1;
+            const og_bin_desc sd = sched[q];
+            if (sd.kind != OG_BIN_PIECE)
+            {
+                if (next) OG_BIN_FAIL("block %u: a long row breaks off at %u", i, q);
+                continue;
+            }
+            const int first = sd.pos0 == rp[sd.row0], last = sd.pos0 + sd.cnt == rp[sd.row0 + 1];
+            if ((!first && next != sd.pos0) || (first && next) ||
+                sd.row1 != ((first ? OG_BIN_FIRST : 0u) | (last ? OG_BIN_LAST : 0u)))
+                OG_BIN_FAIL("block %u: piece %u", i, q);
+            next = last ? 0 : sd.pos0 + sd.cnt;
+        }
+        if (next) OG_BIN_FAIL("block %u: a long row breaks off", i);
     }
-    if (pieces != d->first_bin) OG_BIN_FAIL("%llu pieces for %u piece bins", (unsigned long long)pieces, d->first_bin);
     rc = 0;
 #undef OG_BIN_FAIL
 out:
-    free(items); free(qent); free(src); free(pos); free(bins); free(lrow); free(lbin); free(seen);
+    free(items); free(qent); free(src); free(pos); free(bins); free(sched); free(blk); free(taken); free(seen);
     free(gsrc); free(cols);
     return rc;
 }
@@ -268,24 +260,12 @@ static int og_bin_runs(const og_plan *pl, og_vec *runs)
     return rc;
 }
 
-/* Long rows (more than OG_BIN_CAP in-edges) and bins: first the pieces of
- * the long rows (OG_BIN_CAP in-edges each, in CSR order), then consecutive
- * rows of one kind (thread rows, wavefront rows of more than OG_BIN_WAVE_ROW
- * in-edges) with at most OG_BIN_CAP in-edges and OG_BIN_RPT * OG_BIN_THREADS
- * rows together. */
-typedef struct
-{
-    uint32_t row, deg, bin;
-} og_bin_long;
-
-static int og_bin_long_cmp(const void *a, const void *b)
-{
-    const og_bin_long *x = (const og_bin_long *)a, *y = (const og_bin_long *)b;
-    if (x->deg != y->deg) return x->deg > y->deg ? -1 : 1;
-    return x->row < y->row ? -1 : x->row > y->row;
-}
-
-static int og_bin_pack(const og_plan *pl, const og_vec *runs, og_vec *bins, og_vec *longs)
+/* Bins: first the pieces of the long rows (more than OG_BIN_CAP in-edges;
+ * OG_BIN_CAP in-edges each, in CSR order), then consecutive rows of one kind
+ * (thread rows, wavefront rows of more than OG_BIN_WAVE_ROW in-edges) with at
+ * most cap <= OG_BIN_CAP in-edges together (or one row of more) and
+ * OG_BIN_RPT * OG_BIN_THREADS rows. */
+static int og_bin_pack(const og_plan *pl, const og_vec *runs, uint32_t cap, og_vec *bins)
 {
     const og_bin_run *run = (const og_bin_run *)runs->p;
     const uint32_t Z = pl->Z;
@@ -299,24 +279,17 @@ static int og_bin_pack(const og_plan *pl, const og_vec *runs, og_vec *bins, og_v
             continue;
         }
         for (uint32_t r = run[i].row; r < r1; r++, pos += deg)
-        {
-            og_bin_long *l = (og_bin_long *)og_vec_push(longs);
-            if (!l) return -1;
-            l->row = r;
-            l->deg = deg;
-            l->bin = (uint32_t)bins->n;
             for (uint32_t p0 = 0; p0 < deg; p0 += OG_BIN_CAP)
             {
                 og_bin_desc *d = (og_bin_desc *)og_vec_push(bins);
                 if (!d) return -1;
                 memset(d, 0, sizeof(*d));
                 d->row0 = r;
-                d->row1 = (uint32_t)longs->n - 1;
+                d->row1 = (p0 == 0 ? OG_BIN_FIRST : 0u) | (deg - p0 <= OG_BIN_CAP ? OG_BIN_LAST : 0u);
                 d->pos0 = pos + p0;
                 d->kind = OG_BIN_PIECE;
                 d->cnt = deg - p0 < OG_BIN_CAP ? deg - p0 : OG_BIN_CAP;
             }
-        }
     }
     og_bin_desc *d = NULL;   /* the open bin (the last one) */
     pos = 0;
@@ -336,7 +309,7 @@ static int og_bin_pack(const og_plan *pl, const og_vec *runs, og_vec *bins, og_v
             uint32_t room = 0;
             if (d && d->kind == kind)
             {
-                room = (OG_BIN_CAP - d->cnt) / deg;
+                room = !d->cnt && deg > cap ? 1 : d->cnt < cap ? (cap - d->cnt) / deg : 0;
                 const uint32_t rows = OG_BIN_RPT * OG_BIN_THREADS - (d->row1 - d->row0);
                 if (room > rows) room = rows;
             }
@@ -360,6 +333,99 @@ static int og_bin_pack(const og_plan *pl, const og_vec *runs, og_vec *bins, og_v
     return 0;
 }
 
+/* In-edges per bin: at least OG_BIN_PER_SLOT bins for each block of the sum
+ * pass (its lists are static: with fewer, some blocks have one bin more than
+ * others and the rest wait), as long as a tile keeps 64 entries (the tiles
+ * are padded to 16) and a bin 4096. */
+#define OG_BIN_PER_SLOT 4u
+static uint32_t og_bin_cap(uint32_t E, uint32_t n_seg, uint32_t slots)
+{
+    uint64_t c = (uint64_t)E / ((uint64_t)OG_BIN_PER_SLOT * slots);
+    if (c < 64ull * n_seg) c = 64ull * n_seg;
+    if (c < 4096) c = 4096;
+    return c > OG_BIN_CAP ? OG_BIN_CAP : (uint32_t)c;
+}
+
+/* The sum pass's order: the bins dealt in their order (the long rows, the
+ * longest ones, come first) to the block with the least so far, a long row's
+ * pieces to one block.  order: the bins block by block; blk: where each
+ * block's begin. */
+typedef struct
+{
+    uint64_t load;
+    uint32_t block;
+} og_bin_slot;
+
+static int og_slot_less(og_bin_slot a, og_bin_slot b)
+{
+    return a.load != b.load ? a.load < b.load : a.block < b.block;
+}
+
+static int og_bin_deal(const og_bin_desc *bins, uint32_t n, uint32_t slots, uint32_t *order, uint32_t *blk)
+{
+    og_bin_slot *heap = (og_bin_slot *)malloc((size_t)slots * sizeof(og_bin_slot));
+    uint32_t *to = (uint32_t *)malloc((size_t)n * 4 + 4);
+    if (!heap || !to)
+    {
+        free(heap); free(to);
+        og_set_error("out of host memory");
+        return -1;
+    }
+    for (uint32_t i = 0; i < slots; i++) { heap[i].load = 0; heap[i].block = i; }
+    memset(blk, 0, ((size_t)slots + 1) * 4);
+    for (uint32_t q = 0; q < n;)
+    {
+        uint32_t e = q;
+        uint64_t cost = 0;
+        do
+            cost += bins[e].cnt + 2048u;   /* a bin's entries and its fixed part (barriers, latencies) */
+        while (bins[e].kind == OG_BIN_PIECE && !(bins[e++].row1 & OG_BIN_LAST) && e < n);
+        if (bins[q].kind != OG_BIN_PIECE) e = q + 1;
+        for (; q < e; q++) to[q] = heap[0].block, blk[heap[0].block + 1]++;
+        heap[0].load += cost;
+        for (uint32_t i = 0;;)   /* sift the root down */
+        {
+            uint32_t c = 2 * i + 1;
+            if (c >= slots) break;
+            if (c + 1 < slots && og_slot_less(heap[c + 1], heap[c])) c++;
+            if (!og_slot_less(heap[c], heap[i])) break;
+            const og_bin_slot t = heap[i];
+            heap[i] = heap[c];
+            heap[c] = t;
+            i = c;
+        }
+    }
+    for (uint32_t i = 0; i < slots; i++) blk[i + 1] += blk[i];
+    for (uint32_t q = n; q-- > 0;) order[--blk[to[q] + 1]] = q;   /* blk[i + 1] falls back to block i's first */
+    for (uint32_t i = 0; i < slots; i++) blk[i] = blk[i + 1];
+    blk[slots] = n;
+    free(heap); free(to);
+    return 0;
+}
+
+/* Sources per gather work item: one round of items over the blocks (one per
+ * CU), or as many equal rounds as OG_BIN_ITEM_SRC allows; a segment's
+ * sources are cut evenly.  (Runs of a fixed 131,072 sources left half of the
+ * CUs idle at 2^24 edges.) */
+static uint32_t og_bin_item_src(const uint32_t *seg_quads, uint32_t n_seg, uint32_t cus)
+{
+    const uint64_t total = (uint64_t)seg_quads[n_seg] * OG_BIN_TILE_ALIGN;
+    const uint64_t rounds = (total + (uint64_t)cus * OG_BIN_ITEM_SRC - 1) / ((uint64_t)cus * OG_BIN_ITEM_SRC);
+    const uint64_t most = rounds * cus;
+    uint64_t size = (total + most - 1) / (most ? most : 1);
+    if (size < 8192) size = 8192;
+    for (int tries = 0; tries < 64; tries++)
+    {
+        uint64_t items = 0;
+        for (uint32_t q = 0; q < n_seg; q++)
+            items += ((uint64_t)(seg_quads[q + 1] - seg_quads[q]) * OG_BIN_TILE_ALIGN + size - 1) / size;
+        if (items <= most) break;
+        size += size / 32;
+        if (size > OG_BIN_ITEM_SRC) return OG_BIN_ITEM_SRC;
+    }
+    return (uint32_t)size;
+}
+
 int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
 {
     *out = NULL;
@@ -376,8 +442,8 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
     }
     og_bin_plan *b = (og_bin_plan *)calloc(1, sizeof(og_bin_plan));
     og_vec runs = {NULL, 0, 0, sizeof(og_bin_run)}, bins = {NULL, 0, 0, sizeof(og_bin_desc)};
-    og_vec longs = {NULL, 0, 0, sizeof(og_bin_long)}, items = {NULL, 0, 0, sizeof(og_bin_item)};
-    uint32_t *ids = NULL, *seg_src = NULL, *rp = NULL;
+    og_vec items = {NULL, 0, 0, sizeof(og_bin_item)};
+    uint32_t *order = NULL, *blk = NULL, *d_order = NULL, *seg_src = NULL, *rp = NULL;
     uint32_t *d_quads = NULL, *d_bin_quads = NULL, *d_seg = NULL;
     void *scratch = NULL;
     hipStream_t s = og_stream();
@@ -388,27 +454,22 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
         goto done;
     }
     if (og_bin_runs(pl, &runs)) goto done;
-    if (og_bin_pack(pl, &runs, &bins, &longs))
     {
-        og_set_error("out of host memory");
-        goto done;
-    }
-    {
-        const uint32_t n_long = (uint32_t)longs.n, n_edge_bins = (uint32_t)bins.n;
-        b->n_edges = E;
-        b->d.first_bin = 0;
-        for (uint32_t q = 0; q < n_edge_bins && ((og_bin_desc *)bins.p)[q].kind == OG_BIN_PIECE; q++) b->d.first_bin++;
-        /* the long rows, longest first, and each one's first piece */
-        if (n_long) qsort(longs.p, n_long, sizeof(og_bin_long), og_bin_long_cmp);
-        ids = (uint32_t *)malloc((size_t)(n_long + 1) * 8);
-        if (!ids) { og_set_error("out of host memory"); goto done; }
-        for (uint32_t i = 0; i < n_long; i++)
+        const uint32_t n_seg = (N + OG_BIN_SEG - 1) / OG_BIN_SEG;
+        const uint32_t cus = og_num_cus() > 0 ? (uint32_t)og_num_cus() : 1;
+        if (og_bin_pack(pl, &runs, og_bin_cap(E, n_seg, 2 * cus), &bins))
         {
-            const og_bin_long *l = (const og_bin_long *)longs.p + i;
-            ids[i] = l->row;
-            ids[n_long + i] = l->bin;
-            b->long_terms += l->deg;
+            og_set_error("out of host memory");
+            goto done;
         }
+        const uint32_t n_edge_bins = (uint32_t)bins.n;
+        for (uint32_t q = 0; q < n_edge_bins && ((og_bin_desc *)bins.p)[q].kind == OG_BIN_PIECE; q++) b->d.first_bin++;
+        /* two sum blocks per CU, no more than there are bins */
+        b->sum_grid = n_edge_bins < 2 * cus ? n_edge_bins : 2 * cus;
+        order = (uint32_t *)malloc((size_t)n_edge_bins * 4 + 4);
+        blk = (uint32_t *)malloc(((size_t)b->sum_grid + 1) * 4);
+        if (!order || !blk) { og_set_error("out of host memory"); goto done; }
+        if (og_bin_deal((const og_bin_desc *)bins.p, n_edge_bins, b->sum_grid, order, blk)) goto done;
         /* rows without in-edges: epilogue-only bins, last */
         for (uint32_t r0 = Z; r0 < N; r0 += OG_BIN_ZERO_ROWS)
         {
@@ -421,7 +482,6 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
             d->kind = OG_BIN_THREAD_ROWS;
         }
         b->n_zero_bins = (uint32_t)bins.n - n_edge_bins;
-        const uint32_t n_seg = (N + OG_BIN_SEG - 1) / OG_BIN_SEG;
         if ((uint64_t)n_edge_bins * n_seg > 0xFFFF0000ull)
         {
             og_set_error("binned pull: graph too large for 32-bit tile keys");
@@ -431,7 +491,7 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
         b->d.n_seg = n_seg;
         b->d.n_bins = (uint32_t)bins.n;
         b->d.n_bins_live = (uint32_t)bins.n;
-        b->d.n_long = n_long;
+        b->d.n_edge_bins = n_edge_bins;
 
         /* ---- device: the tiles' sizes in quads (16 entries), segment by
          * segment; prefix sums give each tile's place among the sources and
@@ -465,29 +525,30 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
         b->mem_pos = og_dalloc(b->n_ent * 2);
         b->mem_val = og_dalloc(b->n_ent * 4);
         b->mem_qent = og_dalloc(ent / OG_BIN_TILE_ALIGN * 4);
-        b->mem_long_row = og_bin_upload(ids, (size_t)n_long * 4);
-        b->mem_long_bin = og_bin_upload(ids + n_long, (size_t)n_long * 4);
-        b->mem_ticket = og_dalloc(256);
-        if (!b->mem_src || !b->mem_pos || !b->mem_val || !b->mem_qent || !b->mem_long_row || !b->mem_long_bin ||
-            !b->mem_ticket)
+        b->mem_sched = og_dalloc((size_t)n_edge_bins * sizeof(og_bin_desc));
+        b->mem_blk = og_bin_upload(blk, ((size_t)b->sum_grid + 1) * 4);
+        d_order = (uint32_t *)og_bin_upload(order, (size_t)n_edge_bins * 4);
+        if (!b->mem_src || !b->mem_pos || !b->mem_val || !b->mem_qent || !b->mem_sched || !b->mem_blk || !d_order)
             goto done;
-        if (og_launch_bin_fill(d_bins, n_edge_bins, pl->cols, n_seg, d_quads, (uint16_t *)b->mem_src,
+        if (og_launch_bin_sched(d_bins, d_order, n_edge_bins, (og_bin_desc *)b->mem_sched, s) ||
+            og_launch_bin_fill(d_bins, n_edge_bins, pl->cols, n_seg, d_quads, (uint16_t *)b->mem_src,
                                (uint16_t *)b->mem_pos, (uint32_t *)b->mem_qent, s) ||
             og_launch_fill_u32((uint32_t *)((uint16_t *)b->mem_src + ent), 0, OG_BIN_SPARE / 2, s))
             goto done;
 
-        /* ---- host: the work items: each segment's sources in runs of at
-         * most OG_BIN_ITEM_SRC ---- */
+        /* ---- host: the work items ---- */
+        const uint32_t item_src = og_bin_item_src(seg_src, n_seg, cus);
         for (uint32_t q = 0; q < n_seg; q++)
         {
-            const uint64_t end = (uint64_t)seg_src[q + 1] * OG_BIN_TILE_ALIGN;
-            for (uint64_t f0 = (uint64_t)seg_src[q] * OG_BIN_TILE_ALIGN; f0 < end; f0 += OG_BIN_ITEM_SRC)
+            const uint64_t quads = seg_src[q + 1] - seg_src[q];
+            const uint64_t parts = (quads * OG_BIN_TILE_ALIGN + item_src - 1) / item_src;
+            for (uint64_t k = 0; k < parts; k++)
             {
                 og_bin_item *it = (og_bin_item *)og_vec_push(&items);
                 if (!it) { og_set_error("out of host memory"); goto done; }
                 it->seg = q;
-                it->f0 = (uint32_t)f0;
-                it->f1 = (uint32_t)(end - f0 < OG_BIN_ITEM_SRC ? end : f0 + OG_BIN_ITEM_SRC);
+                it->f0 = (uint32_t)((seg_src[q] + quads * k / parts) * OG_BIN_TILE_ALIGN);
+                it->f1 = (uint32_t)((seg_src[q] + quads * (k + 1) / parts) * OG_BIN_TILE_ALIGN);
                 it->pad = 0;
             }
         }
@@ -500,9 +561,8 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
         b->d.pos = (const uint16_t *)b->mem_pos;
         b->d.val = (float *)b->mem_val;
         b->d.bins = d_bins;
-        b->d.long_row = (const uint32_t *)b->mem_long_row;
-        b->d.long_bin = (const uint32_t *)b->mem_long_bin;
-        b->d.ticket = (uint32_t *)b->mem_ticket;
+        b->d.sched = (const og_bin_desc *)b->mem_sched;
+        b->d.blk = (const uint32_t *)b->mem_blk;
         if (getenv("OG_BIN_VERIFY"))
         {
             rp = (uint32_t *)malloc(((size_t)N + 1) * 4);
@@ -520,7 +580,8 @@ done:
         rc = -1;
     }
     og_dfree(d_quads); og_dfree(d_bin_quads); og_dfree(d_seg); og_dfree(scratch);
-    free(runs.p); free(bins.p); free(longs.p); free(items.p); free(ids); free(seg_src); free(rp);
+    og_dfree(d_order);
+    free(runs.p); free(bins.p); free(items.p); free(order); free(blk); free(seg_src); free(rp);
     if (rc) og_bin_plan_destroy(b);
     else *out = b;
     return rc;

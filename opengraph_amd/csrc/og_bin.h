@@ -26,20 +26,17 @@
  *                lds[src[f]] for the item's sources, 4 consecutive ones
  *                per lane (one 8-byte source load, one quad entry, one
  *                16-byte value store), 256 per wavefront and step.
- *   sum pass     one 1024-thread block per CU: per bin, val[e] is written
+ *   sum pass     two 512-thread blocks per CU: per bin, val[e] is written
  *                to LDS slot pos[e] (the bin's in-edge values in CSR order),
  *                then every row is added from its slots in order -- the
  *                reference's running sum -- by a thread (rows of at most
- *                OG_BIN_WAVE_ROW in-edges) or a wavefront (longer rows, an
- *                exact fast-forward over binades), and the update runs.
+ *                OG_BIN_WAVE_ROW in-edges) or a wavefront (longer rows,
+ *                dozens of terms per lane and step), and the update runs.
  *                The next bin's entries and row metadata are loaded into
- *                registers while a bin's rows are added.
- *   long rows    rows with more than OG_BIN_CAP in-edges are cut into
- *                pieces of OG_BIN_CAP (bins of their own, first in the bin
- *                list); one block per long row, on CUs of its own beside
- *                the sum pass, puts each piece in LDS as the sum pass puts
- *                a bin and adds them in order (exact fast-forward,
- *                block-wide).
+ *                registers while a bin's rows are added.  Rows with more
+ *                than OG_BIN_CAP in-edges are cut into pieces of OG_BIN_CAP
+ *                (bins of their own, first in the bin list), which one block
+ *                takes one after the other.
  * Every row is therefore summed in the reference's order: the fp32 pull is
  * bit-exact, and every global access is a streaming one.
  */
@@ -61,25 +58,27 @@ extern "C" {
 #define OG_BIN_SEG 39936u      /* sources per segment: 156 KB of fp32 in LDS */
 #define OG_BIN_CAP 19968u      /* in-edge values per bin: 78 KB of LDS, two bins per CU */
 #define OG_BIN_PAD 0xFFFFu     /* pos of a padding entry */
-#define OG_BIN_WAVE_ROW 4096u  /* rows with more in-edges are added by a wavefront */
+#define OG_BIN_WAVE_ROW 1024u  /* rows with more in-edges are added by a wavefront */
 #define OG_BIN_RPT 1u          /* rows per thread and bin: a bin holds at most RPT * THREADS rows */
 #define OG_BIN_TILE_ALIGN 16u  /* tiles padded to 16 entries: 64-byte value runs */
 #define OG_BIN_ITEM_SRC (2048u * 64u) /* sources per gather work item at most */
 #define OG_BIN_SPARE 256u      /* spare entries past the last tile (the gather's idle stores) */
-#define OG_BIN_THREADS 512u    /* sum and long-row blocks (two per CU) */
+#define OG_BIN_THREADS 512u    /* sum blocks (two per CU) */
 #define OG_BIN_GTHREADS 1024u  /* gather blocks (one per CU: a segment fills LDS) */
-#define OG_BIN_LTHREADS 1024u  /* long-row blocks (a whole CU each: two sum-block slots) */
 
 enum { OG_BIN_THREAD_ROWS = 0, OG_BIN_WAVE_ROWS = 1, OG_BIN_PIECE = 2 };
 
-/* One bin: rows [row0, row1) (a piece: the long row row0 and row1 = the
- * index of that long row in row order), entries [ent0, ent1) (ent1 - ent0
+/* One bin: rows [row0, row1) (a piece: the long row row0, and in row1
+ * whether it is the row's first and last piece), entries [ent0, ent1) (ent1 - ent0
  * a multiple of 16), first CSR position pos0, cnt in-edges. */
 typedef struct
 {
     uint32_t row0, row1, ent0, ent1;
     uint32_t pos0, kind, pad, cnt;
 } og_bin_desc;
+
+#define OG_BIN_FIRST 1u
+#define OG_BIN_LAST 2u
 
 /* Gather work item: segment seg, sources [f0, f1) (f0 and f1 multiples
  * of 16, within the segment's sources). */
@@ -91,17 +90,17 @@ typedef struct
 /* Everything the binned kernels read, by value. */
 typedef struct og_bin_dev
 {
-    uint32_t N, n_seg, n_items, n_bins, n_bins_live, n_long;
+    uint32_t N, n_seg, n_items, n_bins, n_bins_live;
     uint32_t first_bin;          /* bins [0, first_bin) are the long rows' pieces */
+    uint32_t n_edge_bins;        /* the bins past them hold the rows without in-edges */
     uint32_t n_ent;              /* entries in tiles; OG_BIN_SPARE spare ones follow */
     const og_bin_item *items;
     const uint32_t *qent;        /* n_ent / 16 */
     const uint16_t *src, *pos;
     float *val;
     const og_bin_desc *bins;
-    const uint32_t *long_row;    /* n_long: the long rows (new ids), longest first */
-    const uint32_t *long_bin;    /* n_long: each one's first piece */
-    uint32_t *ticket;            /* the long-row pass's row counter (zeroed by the gather) */
+    const og_bin_desc *sched;    /* the bins with edges in the sum pass's order */
+    const uint32_t *blk;         /* block i of the sum pass takes sched[blk[i], blk[i + 1]) */
 } og_bin_dev;
 
 typedef struct og_bin_plan
@@ -109,27 +108,22 @@ typedef struct og_bin_plan
     og_bin_dev d;
     uint64_t n_ent;              /* entries (and sources) including padding and the spares */
     uint32_t n_zero_bins;
-    uint64_t n_edges, long_terms;  /* in-edges, and those of the long rows */
+    uint32_t sum_grid;           /* blocks of the sum pass (its statistics partials) */
     /* device allocations */
     void *mem_items, *mem_qent, *mem_src, *mem_pos, *mem_val, *mem_bins;
-    void *mem_long_row, *mem_long_bin, *mem_ticket;
+    void *mem_sched, *mem_blk;
 } og_bin_plan;
 
 /* Builds the binned layout of a plan whose rows keep the reference's
  * in-neighbour order (relabel 2 or 0). */
 int og_bin_plan_build(const og_plan *pl, og_bin_plan **out);
 void og_bin_plan_destroy(og_bin_plan *b);
-/* Blocks of the sum pass and of the long-row pass (statistics partials;
- * together one per CU: the passes run side by side). */
-uint32_t og_bin_sum_grid(const og_bin_plan *b);
-uint32_t og_bin_long_grid(const og_bin_plan *b);
 
-/* One binned pull iteration: gather, then the sum pass and (on the side
- * stream) the long rows; ev0 / ev1 (may be NULL) bracket them.  Statistics
- * partials: the sum pass's blocks, then the long-row blocks; then the final
- * reduction. */
-int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, uint32_t it, uint32_t sum_grid,
-                       uint32_t long_grid, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1);
+/* One binned pull iteration: gather, then the sum pass; ev0 / ev1 (may be
+ * NULL) bracket them.  Statistics partials: the sum pass's blocks; then the
+ * final reduction. */
+int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, uint32_t sum_grid, hipStream_t s, hipEvent_t ev0,
+                       hipEvent_t ev1);
 
 /* plan-build kernels (og_bin.hip): the rows' runs of equal in-degree
  * (pairs row, in-degree; *n zeroed by the caller), the tiles' sizes, their
@@ -139,6 +133,8 @@ int og_launch_bin_count(const og_bin_desc *bins, uint32_t n_bins, const uint32_t
                         uint32_t *quads, uint32_t *bin_quads, hipStream_t s);
 int og_launch_bin_place(og_bin_desc *bins, uint32_t n_bins, uint32_t n_all, const uint32_t *bin_quads,
                         const uint32_t *quads, uint32_t n_seg, uint32_t *seg_src, hipStream_t s);
+int og_launch_bin_sched(const og_bin_desc *bins, const uint32_t *order, uint32_t n, og_bin_desc *sched,
+                        hipStream_t s);
 int og_launch_bin_fill(const og_bin_desc *bins, uint32_t n_bins, const uint32_t *cols, uint32_t n_seg,
                        const uint32_t *quads, uint16_t *src, uint16_t *pos, uint32_t *qent, hipStream_t s);
 

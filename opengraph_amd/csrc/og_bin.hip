@@ -5,17 +5,18 @@
  * Exactness.  The reference adds a row's in-edges one after the other into
  * an fp32 running sum (pageRank.c:998-1011).  Here every row is added in
  * that order from LDS: one thread per short row, one wavefront per longer
- * row and one block per row longer than a bin.  Wavefronts and blocks use an
- * exact fast-forward: while the running sum y stays in one binade
- * [2^(e-1), 2^e), every representable value is a multiple of u = 2^(e-24),
- * so for a term a >= 0 the rounded sum is fl(y + a) = y + u * m with m the
- * integer nearest a / u, unless a / u ends in exactly one half (then the
- * tie goes to the even neighbour, which depends on y).  A run of terms is
- * therefore y + u * (prefix sum of their m), an integer scan, up to the
- * first term that is a tie, negative or not finite, or whose sum reaches
- * 2^e; that term is added as an ordinary fp32 add, and the scan restarts
- * after it in the new binade.  The result equals the sequential fp32 sum
- * bit for bit.
+ * row, a row longer than a bin piece by piece by one wavefront.  A wavefront
+ * adds a few dozen terms per lane at a time (og_bin_wave_sum).  While the
+ * running sum y stays in one binade [2^(e-1), 2^e), every representable
+ * value is a multiple of u = 2^(e-24) and a term a >= 0 moves y by a whole
+ * number of u that depends only on a and, where a / u ends in exactly one
+ * half, on whether y / u is even.  So what a run of terms does to any y of
+ * the binade is two numbers, the move of an even and of an odd y, and the
+ * hardware's own adds give them: the run added to the binade's first two
+ * values.  The pairs compose (an associative scan over the lanes); the first
+ * lane whose terms leave the binade, or are negative or not finite, adds its
+ * terms one by one from its exact y, and the scan goes on after it in the
+ * new binade.  The result equals the sequential fp32 sum bit for bit.
  */
 #include <hip/hip_runtime.h>
 
@@ -26,11 +27,9 @@
 #define BT OG_BIN_THREADS
 #define BW (OG_BIN_THREADS / 64)
 #define GT OG_BIN_GTHREADS       /* the gather pass's blocks */
-#define LT OG_BIN_LTHREADS       /* the long-row pass's blocks */
-#define LW (OG_BIN_LTHREADS / 64)
 #define GW (OG_BIN_GTHREADS / 64)
 #define GATHER_Q 8u   /* runs of 4 consecutive sources per lane in flight in the gather */
-#define OG_BIN_HEAD 128u  /* leading terms of a long sum added one by one */
+#define OG_BIN_HEAD 64u  /* leading terms of a wavefront row added one by one */
 
 /* ------------------------------------------------------------------ */
 /* shared pieces                                                       */
@@ -62,19 +61,41 @@ __device__ __forceinline__ uint32_t og_bin_wave_scan(uint32_t v)
     return v;
 }
 
-/* The fast-forward quantities of term a for a running sum in the binade
- * whose unit is 2^-sc: m (valid when !bad) and bad (tie, negative, not
- * finite, or a term of at least the binade's top).  Branch-free: every
- * lane computes, the result is selected. */
-__device__ __forceinline__ void og_bin_term(float a, int sc, bool valid, uint32_t &m, bool &bad)
+/* (d0, d1): the moves of an even and of an odd running sum over a run of
+ * terms; the run A, then the run B. */
+struct og_bin_move
 {
-    const float t = ldexpf(a, sc);   /* a / u, exact for the ranks' range */
-    const float fl = floorf(t);
-    const float fr = t - fl;         /* exact */
-    const bool in = (t >= 0.0f) & (t < 0x1p24f);   /* false for NaN */
-    bad = valid & (!in | (fr == 0.5f));
-    const uint32_t mm = (uint32_t)fl + (fr > 0.5f ? 1u : 0u);
-    m = (valid & !bad) ? mm : 0u;
+    uint32_t d0, d1;
+};
+
+__device__ __forceinline__ og_bin_move og_bin_then(og_bin_move a, og_bin_move b)
+{
+    og_bin_move c;
+    c.d0 = a.d0 + ((a.d0 & 1u) ? b.d1 : b.d0);
+    c.d1 = a.d1 + ((a.d1 & 1u) ? b.d0 : b.d1);
+    return c;
+}
+
+/* the run of the lanes that the DPP control reads, then this lane's (lanes
+ * with none there read the empty run) */
+template <int CTRL, int ROWS, bool BOUND>
+__device__ __forceinline__ void og_bin_scan_step(og_bin_move &m)
+{
+    og_bin_move p;
+    p.d0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m.d0, CTRL, ROWS, 0xF, BOUND);
+    p.d1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m.d1, CTRL, ROWS, 0xF, BOUND);
+    m = og_bin_then(p, m);
+}
+
+/* Inclusive scan of the lanes' runs, by the steps of og_bin_wave_scan. */
+__device__ __forceinline__ void og_bin_move_scan(og_bin_move &m)
+{
+    og_bin_scan_step<0x111, 0xF, true>(m);
+    og_bin_scan_step<0x112, 0xF, true>(m);
+    og_bin_scan_step<0x114, 0xF, true>(m);
+    og_bin_scan_step<0x118, 0xF, true>(m);
+    og_bin_scan_step<0x142, 0xA, false>(m);
+    og_bin_scan_step<0x143, 0xC, false>(m);
 }
 
 /* One thread's sequential fp32 sum of slot[j, j1): the 16-byte groups
@@ -136,102 +157,121 @@ __device__ __forceinline__ float og_bin_row_sum(const float *slot, uint32_t j, u
     return s;
 }
 
-/* x[i + 4 * lane + k] for k < 4 where inside [0, n), else 0 (n > 0;
- * branch-free: the index is clamped, the value selected) */
-__device__ __forceinline__ void og_bin_wave_load4(const float *x, uint32_t i, uint32_t n, uint32_t lane,
-                                                  float (&a)[4])
+/* One step of og_bin_wave_sum: T consecutive terms per lane (in x) added in
+ * lane order onto the running sum with bits yb (uniform). */
+template <uint32_t T>
+__device__ __forceinline__ uint32_t og_bin_wave_step(const float4 (&x)[T / 4], uint32_t yb)
 {
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t sign = 0;
 #pragma unroll
-    for (uint32_t k = 0; k < 4; k++)
+    for (uint32_t k = 0; k < T / 4; k++)
+        sign |= __float_as_uint(x[k].x) | __float_as_uint(x[k].y) | __float_as_uint(x[k].z) | __float_as_uint(x[k].w);
+    uint32_t p = 0;   /* lanes below p are added */
+    for (;;)
     {
-        const uint32_t p = i + 4 * lane + k;
-        const float v = x[min(p, n - 1)];
-        a[k] = p < n ? v : 0.0f;
+        uint32_t f = p;
+        if (yb - 0x0D800000u < 0x64000000u)   /* 2^-100 <= y < 2^100 */
+        {
+            const uint32_t bb = yb & 0xFF800000u;
+            float s0 = __uint_as_float(bb), s1 = __uint_as_float(bb | 1u);
+#pragma unroll
+            for (uint32_t k = 0; k < T / 4; k++)
+            {
+                s0 = s0 + x[k].x;
+                s1 = s1 + x[k].x;
+                s0 = s0 + x[k].y;
+                s1 = s1 + x[k].y;
+                s0 = s0 + x[k].z;
+                s1 = s1 + x[k].z;
+                s0 = s0 + x[k].w;
+                s1 = s1 + x[k].w;
+            }
+            og_bin_move m;
+            m.d0 = __float_as_uint(s0) - bb;
+            m.d1 = __float_as_uint(s1) - (bb | 1u);
+            const bool bad = ((sign >> 31) != 0) | (m.d0 >= (1u << 23)) | (m.d1 >= (1u << 23));
+            m.d0 = bad ? 1u << 24 : m.d0;   /* 64 of them stay below 2^31 */
+            m.d1 = bad ? 1u << 24 : m.d1;
+            m.d0 = lane < p ? 0u : m.d0;
+            m.d1 = lane < p ? 0u : m.d1;
+            og_bin_move_scan(m);
+            const uint32_t d = (yb & 1u) ? m.d1 : m.d0;
+            const uint64_t fail = __ballot((yb & 0x7FFFFFu) + d >= (1u << 23));
+            if (!fail) return yb + (uint32_t)__builtin_amdgcn_readlane(d, 63);
+            f = (uint32_t)__builtin_ctzll(fail);
+            if (f) yb += (uint32_t)__builtin_amdgcn_readlane(d, f - 1);
+        }
+        /* lane f's terms one by one */
+        float s = __uint_as_float(yb);
+#pragma unroll
+        for (uint32_t k = 0; k < T / 4; k++)
+        {
+            s = s + x[k].x;
+            s = s + x[k].y;
+            s = s + x[k].z;
+            s = s + x[k].w;
+        }
+        yb = (uint32_t)__builtin_amdgcn_readlane(__float_as_uint(s), f);
+        p = f + 1;
+        if (p == 64) return yb;
     }
 }
 
-/* The sequential fp32 sum of slot[j0, j0 + n) (LDS, n > 0), one
- * wavefront, result uniform: the first OG_BIN_HEAD terms one after the
- * other (where the running sum crosses binades every few terms), then 256
- * terms per step, 4 consecutive ones per lane (a lane's prefix of its own
- * terms, then a wavefront scan of the lanes' totals); the next 256 are
- * read while a step is scanned. */
-__device__ float og_bin_wave_sum(const float *slot, uint32_t j0, uint32_t n, float y0)
+/* Lane's T terms slot[j + T * lane ..] (j a multiple of 4), those at or past
+ * j1 as +0 when TAIL.  T is a multiple of 4 and not of 8: the lanes' 16-byte
+ * reads then fall on all the banks. */
+template <uint32_t T, bool TAIL>
+__device__ __forceinline__ void og_bin_wave_read(const float *slot, uint32_t j, uint32_t j1, float4 (&x)[T / 4])
 {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t h = n < OG_BIN_HEAD ? n : OG_BIN_HEAD;
-    float y = og_bin_uniform(og_bin_row_sum(slot, j0, j0 + h, y0));
-    const float *x = slot + j0;
-    uint32_t i = h;
-    float a[4];
-    og_bin_wave_load4(x, i, n, lane, a);
-    while (i < n)
+    constexpr uint32_t QMAX = OG_BIN_CAP / 4 - 1;
+    const float4 *s4 = reinterpret_cast<const float4 *>(slot);
+    const uint32_t i = j + T * (threadIdx.x & 63);
+#pragma unroll
+    for (uint32_t k = 0; k < T / 4; k++)
     {
-        const uint32_t left = n - i;
-        if (!(y >= 0x1p-100f && y < 0x1p100f))
+        x[k] = s4[TAIL ? min(i / 4 + k, QMAX) : i / 4 + k];
+        if (TAIL)
         {
-            /* zero, tiny or not finite: one ordinary add */
-            y = og_bin_uniform(y + x[i]);
-            i += 1;
-            og_bin_wave_load4(x, i, n, lane, a);
-            continue;
-        }
-        float an[4];
-        og_bin_wave_load4(x, i + 256, n, lane, an);   /* used when the whole step is taken */
-        int ey;
-        frexpf(y, &ey);
-        const int sc = 24 - ey;
-        const uint32_t Y = (uint32_t)ldexpf(y, sc);   /* in [2^23, 2^24) */
-        uint32_t L[4];
-        bool bad[4], valid[4];
-        uint32_t tot = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < 4; k++)
-        {
-            uint32_t m;
-            valid[k] = 4 * lane + k < left;
-            og_bin_term(a[k], sc, valid[k], m, bad[k]);
-            tot = min(tot + m, 1u << 25);
-            L[k] = tot;
-        }
-        const uint32_t incl = og_bin_wave_scan(tot);   /* <= 2^31 */
-        const uint32_t X = incl - tot;                 /* the earlier lanes' terms */
-        uint32_t kfail = 4;
-#pragma unroll
-        for (int k = 3; k >= 0; k--)
-            kfail = (valid[k] & (bad[k] | (Y + X + L[k] >= (1u << 24)))) ? (uint32_t)k : kfail;
-        const uint64_t fb = __ballot(kfail < 4);
-        if (fb == 0)
-        {
-            const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(incl, 63);
-            y = og_bin_uniform(ldexpf((float)(Y + total), -sc));
-            i += left < 256 ? left : 256;
-#pragma unroll
-            for (uint32_t k = 0; k < 4; k++) a[k] = an[k];
-        }
-        else
-        {
-            /* the first failing term: the prefix before it, then an
-             * ordinary add of it */
-            const uint32_t lf = (uint32_t)__builtin_ctzll(fb);
-            uint32_t pre = X;
-            float af = a[0];
-#pragma unroll
-            for (uint32_t k = 1; k < 4; k++)
-                if (kfail == k)
-                {
-                    pre = X + L[k - 1];
-                    af = a[k];
-                }
-            const uint32_t kf = (uint32_t)__builtin_amdgcn_readlane(kfail, lf);
-            const uint32_t p = (uint32_t)__builtin_amdgcn_readlane(pre, lf);
-            y = ldexpf((float)(Y + p), -sc);
-            y = og_bin_uniform(y + og_bin_lane(af, lf));
-            i += 4 * lf + kf + 1;
-            og_bin_wave_load4(x, i, n, lane, a);
+            x[k].x = i + 4 * k < j1 ? x[k].x : 0.0f;
+            x[k].y = i + 4 * k + 1 < j1 ? x[k].y : 0.0f;
+            x[k].z = i + 4 * k + 2 < j1 ? x[k].z : 0.0f;
+            x[k].w = i + 4 * k + 3 < j1 ? x[k].w : 0.0f;
         }
     }
-    return y;
+}
+
+/* The sequential fp32 sum of slot[j, j1) (LDS) onto y0, one wavefront, result
+ * uniform: `head` leading terms (and those up to a multiple of 4) one after
+ * the other -- near 0 the running sum crosses a binade every few terms --
+ * then 64 * T terms a step. */
+#define OG_BIN_WT 28u   /* terms per lane and step */
+#define OG_BIN_WS 12u   /* of a last step of at most 64 * 12 terms */
+__device__ __forceinline__ float og_bin_wave_sum(const float *slot, uint32_t j, uint32_t j1, float y0, uint32_t head)
+{
+    const uint32_t jh = min((j + head + 3u) & ~3u, j1);
+    uint32_t yb = (uint32_t)__builtin_amdgcn_readfirstlane(
+        __float_as_int(jh > j ? og_bin_row_sum(slot, j, jh, y0) : y0));
+    j = jh;
+    for (; j1 - j >= 64u * OG_BIN_WT; j += 64u * OG_BIN_WT)
+    {
+        float4 x[OG_BIN_WT / 4];
+        og_bin_wave_read<OG_BIN_WT, false>(slot, j, j1, x);
+        yb = og_bin_wave_step<OG_BIN_WT>(x, yb);
+    }
+    if (j1 - j > 64u * OG_BIN_WS)
+    {
+        float4 x[OG_BIN_WT / 4];
+        og_bin_wave_read<OG_BIN_WT, true>(slot, j, j1, x);
+        yb = og_bin_wave_step<OG_BIN_WT>(x, yb);
+    }
+    else if (j < j1)
+    {
+        float4 x[OG_BIN_WS / 4];
+        og_bin_wave_read<OG_BIN_WS, true>(slot, j, j1, x);
+        yb = og_bin_wave_step<OG_BIN_WS>(x, yb);
+    }
+    return __uint_as_float(yb);
 }
 
 /* ------------------------------------------------------------------ */
@@ -262,7 +302,6 @@ __global__ __launch_bounds__(GT) void og_bin_gather_kernel(og_bin_dev b, const f
 {
     __shared__ __align__(16) float seg[OG_BIN_SEG];
     if (*done) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *b.ticket = 0u;   /* the long-row pass's row counter */
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (uint32_t q = blockIdx.x; q < b.n_items; q += gridDim.x)
@@ -389,7 +428,12 @@ __device__ __forceinline__ uint32_t og_bin_meta_row(const og_bin_desc &d, uint32
 
 __device__ __forceinline__ void og_bin_meta_load(const og_pr_dev &a, const og_bin_desc &d, og_bin_meta &m)
 {
-    if (d.kind == OG_BIN_PIECE) return;
+    if (d.kind == OG_BIN_PIECE)
+    {
+        m.prev[0] = __builtin_nontemporal_load(&a.r[d.row0]);
+        m.deg[0] = __builtin_nontemporal_load(&a.outdeg[d.row0]);
+        return;
+    }
 #pragma unroll
     for (uint32_t k = 0; k < OG_BIN_RPT; k++)
     {
@@ -506,6 +550,13 @@ __device__ __forceinline__ void og_bin_put(const og_bin_dev &b, float *slot, con
                         __builtin_nontemporal_load((const og_f32x4 *)(b.val + e + 4)));
 }
 
+/* Block i takes the bins sched[blk[i], blk[i + 1]) in that order (a long
+ * row's pieces one after the other), then, while rows without in-edges still
+ * change, every gridDim.x-th of their bins.  Bound by the streamed entries (6
+ * bytes each); two blocks a CU, so that one's rows overlap the other's
+ * entries.  R-MAT-24: 490 us = 3.6 TB/s (567 us beside a long-row kernel on
+ * CUs of its own before); R-MAT-22: 117 us, where that kernel's longest row
+ * took 158; R-MAT-16, whose wavefront rows bound it: 17 us against 33. */
 __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_dev a)
 {
     __shared__ __align__(16) float slot[OG_BIN_CAP];
@@ -514,18 +565,20 @@ __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_d
     og_bin_stat_init(st);
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    /* the long rows' pieces (bins [0, first_bin)) are the long-row pass's */
-    uint32_t q = b.first_bin + blockIdx.x;
+    uint32_t q = b.blk[blockIdx.x];
+    const uint32_t qe = b.blk[blockIdx.x + 1];
     og_bin_desc d;
     og_bin_regs regs;
     og_bin_meta meta;
-    if (q < b.n_bins_live)
+    float carry = 0.0f;   /* the running sum of a long row between its pieces (wavefront 0) */
+    static_assert(OG_BIN_RPT == 1, "a lane holds one wavefront row");
+    if (q < qe)
     {
-        d = b.bins[q];
+        d = b.sched[q];
         og_bin_load(b, d, regs);
         og_bin_meta_load(a, d, meta);
     }
-    for (; q < b.n_bins_live; q += gridDim.x)
+    for (; q < qe; q++)
     {
         __syncthreads();   /* the previous bin's reads of slot are done */
         /* this bin's values to their CSR slots */
@@ -534,9 +587,9 @@ __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_d
         const og_bin_meta cm = meta;
         /* the next bin's entries and row metadata load while this one's
          * rows are added */
-        if (q + gridDim.x < b.n_bins_live)
+        if (q + 1 < qe)
         {
-            d = b.bins[q + gridDim.x];
+            d = b.sched[q + 1];
             og_bin_load(b, d, regs);
             og_bin_meta_load(a, d, meta);
         }
@@ -556,22 +609,32 @@ __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_d
         }
         else
         {
-#pragma unroll
-            for (uint32_t k = 0; k < OG_BIN_RPT; k++)
+            /* wavefront w's rows row0 + w, + BW, ... (a piece: wavefront 0,
+             * the whole bin, going on from the row's earlier pieces) */
+            const bool piece = cd.kind == OG_BIN_PIECE;
+            const bool first = !piece || (cd.row1 & OG_BIN_FIRST), last = !piece || (cd.row1 & OG_BIN_LAST);
+            const uint32_t row1 = piece ? cd.row0 + 1 : cd.row1;
+            uint32_t l = 0;
+            for (uint32_t v = cd.row0 + wave; v < row1; v += BW, l++)
             {
-                if (cd.row0 + wave + BT * k >= cd.row1) break;
-                for (uint32_t l = 0; l < 64; l++)
-                {
-                    const uint32_t v = cd.row0 + wave + BW * l + BT * k;
-                    if (v >= cd.row1) break;
-                    const uint32_t j0 = (uint32_t)__builtin_amdgcn_readlane(cm.p0[k], l) - cd.pos0;
-                    const uint32_t j1 = (uint32_t)__builtin_amdgcn_readlane(cm.p1[k], l) - cd.pos0;
-                    const float prev = og_bin_lane(cm.prev[k], l);
-                    const float y = og_bin_wave_sum(slot, j0, j1 - j0, a.spmv ? prev : 0.0f);
-                    const uint32_t deg = (uint32_t)__builtin_amdgcn_readlane(cm.deg[k], l);
-                    if (lane == 0) og_bin_epilogue_pf(a, v, y, prev, deg, st);
-                }
+                const uint32_t j0 = piece ? 0 : (uint32_t)__builtin_amdgcn_readlane(cm.p0[0], l) - cd.pos0;
+                const uint32_t j1 = piece ? cd.cnt : (uint32_t)__builtin_amdgcn_readlane(cm.p1[0], l) - cd.pos0;
+                const float prev = og_bin_lane(cm.prev[0], l);
+                const uint32_t deg = (uint32_t)__builtin_amdgcn_readlane(cm.deg[0], l);
+                carry = og_bin_wave_sum(slot, j0, j1, !first ? carry : a.spmv ? prev : 0.0f,
+                                        first ? OG_BIN_HEAD : 0);
+                if (last && lane == 0) og_bin_epilogue_pf(a, v, carry, prev, deg, st);
             }
+        }
+    }
+    for (q = b.n_edge_bins + blockIdx.x; q < b.n_bins_live; q += gridDim.x)
+    {
+        const og_bin_desc z = b.bins[q];
+#pragma unroll
+        for (uint32_t k = 0; k < OG_BIN_RPT; k++)
+        {
+            const uint32_t v = z.row0 + threadIdx.x + BT * k;
+            if (v < z.row1) og_bin_epilogue(a, v, 0.0f, st);
         }
     }
     og_bin_stat r = og_bin_block_stat<BT>(st);
@@ -579,232 +642,18 @@ __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_d
 }
 
 /* ------------------------------------------------------------------ */
-/* long rows                                                           */
-/* ------------------------------------------------------------------ */
-
-/* One block per long row (longest first, taken in turn from a counter),
- * running beside the sum pass: the row's pieces in order, each scattered
- * from its entries into LDS in CSR order (as the sum pass does for a bin)
- * and added with the block-wide exact fast-forward, 4 consecutive terms
- * per thread (4096 terms) per step. */
-#define OG_BIN_LTT 4u                  /* terms per thread and step */
-
-/* sum (saturated at 2^25) or minimum over the 16 wavefronts' values, read
- * by every lane */
-__device__ __forceinline__ void og_bin_waves_read(const uint32_t *v, uint32_t (&w)[LW])
-{
-    const uint4 *v4 = reinterpret_cast<const uint4 *>(v);   /* 16-byte aligned */
-#pragma unroll
-    for (uint32_t i = 0; i < LW / 4; i++)
-    {
-        const uint4 t = v4[i];
-        w[4 * i] = t.x;
-        w[4 * i + 1] = t.y;
-        w[4 * i + 2] = t.z;
-        w[4 * i + 3] = t.w;
-    }
-}
-
-__device__ __forceinline__ uint32_t og_bin_waves_sum(const uint32_t *v)
-{
-    uint32_t w[LW];
-    og_bin_waves_read(v, w);
-    uint32_t x = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < LW; i++) x = min(x + w[i], 1u << 25);
-    return x;
-}
-
-__device__ __forceinline__ uint32_t og_bin_waves_min(const uint32_t *v)
-{
-    uint32_t w[LW];
-    og_bin_waves_read(v, w);
-    uint32_t x = w[0];
-#pragma unroll
-    for (uint32_t i = 1; i < LW; i++) x = min(x, w[i]);
-    return x;
-}
-
-/* The block-wide fast-forward of the running sum y (identical in every
- * thread) over xs[p, clen) (LDS); par alternates the partial arrays from
- * step to step. */
-__device__ __forceinline__ float og_bin_block_sum(const float *xs, uint32_t p, uint32_t clen, float y,
-                                                  uint32_t (&s_wsum)[2][LW], uint32_t (&s_wfail)[2][LW],
-                                                  uint32_t &s_pre, uint32_t &par)
-{
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wave = threadIdx.x >> 6;
-    while (p < clen)
-    {
-        const uint32_t left = clen - p;
-        if (!(y >= 0x1p-100f && y < 0x1p100f))
-        {
-            y = y + xs[p];
-            p += 1;
-            continue;
-        }
-        int ey;
-        frexpf(y, &ey);
-        const int sc = 24 - ey;
-        const uint32_t Y = (uint32_t)ldexpf(y, sc);   /* in [2^23, 2^24) */
-        /* this thread's terms p + 4t .. p + 4t + 3 */
-        uint32_t m[OG_BIN_LTT], l[OG_BIN_LTT];
-        bool bad[OG_BIN_LTT], valid[OG_BIN_LTT];
-        uint32_t tot = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < OG_BIN_LTT; k++)
-        {
-            const uint32_t i = OG_BIN_LTT * threadIdx.x + k;
-            valid[k] = i < left;
-            const float v = xs[min(p + i, clen - 1)];
-            og_bin_term(valid[k] ? v : 0.0f, sc, valid[k], m[k], bad[k]);
-            tot = min(tot + m[k], 1u << 25);
-            l[k] = tot;
-        }
-        const uint32_t incl_w = og_bin_wave_scan(tot);          /* <= 2^31 */
-        if (lane == 63) s_wsum[par][wave] = min(incl_w, 1u << 25);
-        __syncthreads();
-        uint32_t base = 0;
-        {
-            /* prefix of the earlier wavefronts' sums */
-            uint32_t w[LW];
-            og_bin_waves_read(s_wsum[par], w);
-#pragma unroll
-            for (uint32_t k = 0; k < LW; k++)
-                if (k < wave) base = min(base + w[k], 1u << 25);
-        }
-        const uint32_t X = min(base + incl_w - tot, 1u << 25);   /* before this thread's terms */
-        uint32_t kfail = OG_BIN_LTT;
-#pragma unroll
-        for (int k = (int)OG_BIN_LTT - 1; k >= 0; k--)
-            kfail = (valid[k] & (bad[k] | (Y + X + l[k] >= (1u << 24)))) ? (uint32_t)k : kfail;
-        const uint64_t fb = __ballot(kfail < OG_BIN_LTT);
-        if (lane == 0)
-        {
-            uint32_t idx = 0xFFFFFFFFu;
-            if (fb)
-            {
-                const uint32_t fl = (uint32_t)__builtin_ctzll(fb);
-                idx = OG_BIN_LTT * (64u * wave + fl) + (uint32_t)__builtin_amdgcn_readlane(kfail, fl);
-            }
-            s_wfail[par][wave] = idx;
-        }
-        __syncthreads();
-        const uint32_t kf = og_bin_waves_min(s_wfail[par]);
-        if (kf == 0xFFFFFFFFu)
-        {
-            const uint32_t total = og_bin_waves_sum(s_wsum[par]);
-            y = ldexpf((float)(Y + total), -sc);
-            p += left < OG_BIN_LTT * LT ? left : OG_BIN_LTT * LT;
-        }
-        else
-        {
-            const uint32_t t = kf / OG_BIN_LTT, kk = kf % OG_BIN_LTT;
-            if (threadIdx.x == t)
-            {
-                uint32_t pre = X;
-#pragma unroll
-                for (uint32_t k = 0; k < OG_BIN_LTT; k++)
-                    if (k + 1 == kk) pre = X + l[k];
-                s_pre = pre;
-            }
-            __syncthreads();
-            y = ldexpf((float)(Y + s_pre), -sc);
-            y = y + xs[p + kf];
-            p += kf + 1;
-            __syncthreads();   /* s_pre read by all before its next write */
-        }
-        par ^= 1;
-    }
-    return y;
-}
-
-__global__ __launch_bounds__(LT) void og_bin_long_kernel(og_bin_dev b, og_pr_dev a, uint32_t part_base)
-{
-    __shared__ __align__(16) float buf[OG_BIN_CAP];
-    __shared__ __align__(16) uint32_t s_wsum[2][LW];
-    __shared__ __align__(16) uint32_t s_wfail[2][LW];
-    __shared__ uint32_t s_pre, s_row;
-    if (*a.done) return;
-    og_bin_stat st;
-    og_bin_stat_init(st);
-    uint32_t par = 0;    /* which s_wsum / s_wfail set a step uses */
-    /* rows taken in turn from a counter the gather pass zeroed (longest
-     * first: each block takes the next when it is done) */
-    for (;;)
-    {
-        __syncthreads();   /* the previous row's reads of buf and s_row are done */
-        if (threadIdx.x == 0) s_row = atomicAdd(b.ticket, 1u);
-        __syncthreads();
-        const uint32_t q = s_row;
-        if (q >= b.n_long) break;
-        const uint32_t v = b.long_row[q];
-        const uint32_t n = a.row_ptr[v + 1] - a.row_ptr[v];
-        float y = a.spmv ? a.r[v] : 0.0f;     /* identical in every thread */
-        uint32_t bin = b.long_bin[q];
-        for (uint32_t c0 = 0; c0 < n; c0 += OG_BIN_CAP, bin++)
-        {
-            const og_bin_desc d = b.bins[bin];
-            __syncthreads();   /* the previous piece's reads of buf are done */
-            /* the piece's entries to their slots, two sweeps of 8 per thread at a time */
-            for (uint32_t e = d.ent0 + 8 * threadIdx.x; e < d.ent1; e += 16 * LT)
-            {
-                const uint32_t e2 = e + 8 * LT;
-                const bool two = e2 < d.ent1;
-                const uint32_t f = two ? e2 : e;
-                const og_u32x4 p0 = __builtin_nontemporal_load((const og_u32x4 *)(b.pos + e));
-                const og_f32x4 x0 = __builtin_nontemporal_load((const og_f32x4 *)(b.val + e));
-                const og_f32x4 x1 = __builtin_nontemporal_load((const og_f32x4 *)(b.val + e + 4));
-                const og_u32x4 p1 = __builtin_nontemporal_load((const og_u32x4 *)(b.pos + f));
-                const og_f32x4 y0 = __builtin_nontemporal_load((const og_f32x4 *)(b.val + f));
-                const og_f32x4 y1 = __builtin_nontemporal_load((const og_f32x4 *)(b.val + f + 4));
-                og_bin_scatter8(buf, p0, x0, x1);
-                if (two) og_bin_scatter8(buf, p1, y0, y1);
-            }
-            __syncthreads();
-            uint32_t p = 0;
-            if (c0 == 0)
-            {
-                /* the leading terms one after the other (the running sum
-                 * crosses binades every few terms there) */
-                p = d.cnt < OG_BIN_HEAD ? d.cnt : OG_BIN_HEAD;
-                y = og_bin_uniform(og_bin_row_sum(buf, 0, p, y));
-            }
-            y = og_bin_block_sum(buf, p, d.cnt, y, s_wsum, s_wfail, s_pre, par);
-        }
-        if (threadIdx.x == 0) og_bin_epilogue(a, v, y, st);
-    }
-    og_bin_stat r = og_bin_block_stat<LT>(st);
-    og_bin_write_part(a, part_base + blockIdx.x, r);
-}
-
-/* ------------------------------------------------------------------ */
 /* launch                                                              */
 /* ------------------------------------------------------------------ */
 
-extern "C" int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, uint32_t it, uint32_t sum_grid,
-                                  uint32_t long_grid, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
+extern "C" int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, uint32_t sum_grid, hipStream_t s,
+                                  hipEvent_t ev0, hipEvent_t ev1)
 {
-    (void)it;
     if (ev0 && og_hip_check(hipEventRecord(ev0, s), "hipEventRecord")) return -1;
-    if (!b->n_items && og_launch_fill_u32(b->ticket, 0u, 1, s)) return -1;
     if (b->n_items)
         OG_LAUNCH(og_bin_gather_kernel, dim3(og_num_cus() > 0 ? og_num_cus() : 1), dim3(GT), 0, s, *b,
                   (const float *)a->g_in,
                   (const uint32_t *)a->done);
-    if (long_grid)
-    {
-        /* the long rows on the side stream, on CUs of their own, while the
-         * sum pass runs on the others */
-        hipStream_t side = og_side_stream();
-        if (og_hip_check(hipEventRecord(og_side_fork(), s), "hipEventRecord") ||
-            og_hip_check(hipStreamWaitEvent(side, og_side_fork(), 0), "hipStreamWaitEvent"))
-            return -1;
-        OG_LAUNCH(og_bin_long_kernel, dim3(long_grid), dim3(LT), 0, side, *b, *a, sum_grid);
-        if (og_hip_check(hipEventRecord(og_side_join(), side), "hipEventRecord")) return -1;
-    }
     OG_LAUNCH(og_bin_sum_kernel, dim3(sum_grid), dim3(BT), 0, s, *b, *a);
-    if (long_grid && og_hip_check(hipStreamWaitEvent(s, og_side_join(), 0), "hipStreamWaitEvent")) return -1;
     if (ev1 && og_hip_check(hipEventRecord(ev1, s), "hipEventRecord")) return -1;
     return og_hip_check(og_launch_status(), "og_bin_pull");
 }
@@ -905,6 +754,13 @@ __global__ void og_bin_place_kernel(og_bin_desc *__restrict__ bins, uint32_t n_b
     }
 }
 
+__global__ void og_bin_sched_kernel(const og_bin_desc *__restrict__ bins, const uint32_t *__restrict__ order, uint32_t n,
+                                    og_bin_desc *__restrict__ sched)
+{
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        sched[i] = bins[order[i]];
+}
+
 __global__ __launch_bounds__(BUILD_T) void og_bin_fill_kernel(const og_bin_desc *__restrict__ bins, uint32_t n_bins,
                                                               const uint32_t *__restrict__ cols, uint32_t n_seg,
                                                               const uint32_t *__restrict__ quads,
@@ -1000,6 +856,14 @@ extern "C" int og_launch_bin_place(og_bin_desc *bins, uint32_t n_bins, uint32_t 
     OG_LAUNCH(og_bin_place_kernel, dim3(og_bin_grid(n_all > n_seg ? n_all : n_seg + 1)), dim3(256), 0, s, bins, n_bins,
               n_all, bin_quads, quads, n_seg, seg_src);
     return og_hip_check(og_launch_status(), "og_bin_place_kernel");
+}
+
+extern "C" int og_launch_bin_sched(const og_bin_desc *bins, const uint32_t *order, uint32_t n, og_bin_desc *sched,
+                                   hipStream_t s)
+{
+    if (!n) return 0;
+    OG_LAUNCH(og_bin_sched_kernel, dim3(og_bin_grid(n)), dim3(256), 0, s, bins, order, n, sched);
+    return og_hip_check(og_launch_status(), "og_bin_sched_kernel");
 }
 
 extern "C" int og_launch_bin_fill(const og_bin_desc *bins, uint32_t n_bins, const uint32_t *cols, uint32_t n_seg,

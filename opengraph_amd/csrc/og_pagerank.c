@@ -377,12 +377,7 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
         }
         p->bins = NULL;   /* default: the gather pull instead */
     }
-    if (p->bins)
-    {
-        p->bin_sum_grid = og_bin_sum_grid(p->bins);
-        p->bin_long_grid = og_bin_long_grid(p->bins);
-        p->n_final_bin = og_final_blocks(p->bin_sum_grid + p->bin_long_grid, 0);
-    }
+    if (p->bins) p->n_final_bin = og_final_blocks(p->bins->sum_grid, 0);
     p->seconds_plan = og_now() - t0;
     og_plan *pl = p->plan;
     if ((p->push || p->dd) && !pl->push_src)
@@ -475,7 +470,7 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     uint32_t parts = pull_blocks > p->gv ? pull_blocks : p->gv;
     if (parts < pp_blocks) parts = pp_blocks;
     if (push_chains && parts < p->gv + chain_blocks) parts = p->gv + chain_blocks;
-    if (p->bins && parts < p->bin_sum_grid + p->bin_long_grid) parts = p->bin_sum_grid + p->bin_long_grid;
+    if (p->bins && parts < p->bins->sum_grid) parts = p->bins->sum_grid;
     p->parts_cap = parts;
     uint32_t fins = p->n_final_pull > p->n_final_vert ? p->n_final_pull : p->n_final_vert;
     if (fins < p->n_final_bin) fins = p->n_final_bin;
@@ -696,21 +691,21 @@ static int og_pr_launch_iter(ogpu_pr *p, uint32_t it, int allow_stop, hipEvent_t
     if (p->bins)
     {
         /* binned pull: gather, sum (rows without in-edges only in the first
-         * two iterations, as below), long rows, final reduction */
+         * two iterations, as below), final reduction */
         og_bin_dev b = p->bins->d;
         if (it >= 2)
         {
             b.n_bins_live = b.n_bins - p->bins->n_zero_bins;
             a.z_active = 0.0 >= a.epsilon ? a.N - a.Z : 0;
         }
-        a.n_parts = p->bin_sum_grid + p->bin_long_grid;
+        a.n_parts = p->bins->sum_grid;
         a.n_final_blocks = p->n_final_bin;
         if (a.n_parts > p->parts_cap)
         {
             og_set_error("binned pull with %u partials, %u allocated", a.n_parts, p->parts_cap);
             return -1;
         }
-        if (og_launch_bin_pull(&b, &a, row, p->bin_sum_grid, p->bin_long_grid, s, e0, e1) ||
+        if (og_launch_bin_pull(&b, &a, p->bins->sum_grid, s, e0, e1) ||
             og_launch_final(&a, row, s))
             return -1;
         return 0;

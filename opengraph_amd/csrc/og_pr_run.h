@@ -59,10 +59,9 @@ struct ogpu_pr
     double *lscratch;
     /* every-row-exact fp32 pull: rows [0, C) longest first (device) */
     uint32_t *chain_rows;
-    /* binned fp32 pull (og_bin.h): layout, grids of its passes, blocks of
-     * its final reduction */
+    /* binned fp32 pull (og_bin.h): layout, blocks of its final reduction */
     struct og_bin_plan *bins;
-    uint32_t bin_sum_grid, bin_long_grid, n_final_bin;
+    uint32_t n_final_bin;
     /* partitioned push (og_push_part_kernel): destination ranges (device
      * n_pp + 1 row bounds), each inverse-CSR edge's offset in its range,
      * the first range pushed, blocks of its final reduction */

@@ -141,17 +141,17 @@ static int og_spmv_launch_iter(ogpu_spmv *s, hipEvent_t e0, hipEvent_t e1)
     a.next = s->acc;
     if (p->bins)
     {
-        /* binned: gather of the terms, then the sum and long-row passes
-         * adding onto each row's y; rows without in-edges keep theirs */
+        /* binned: gather of the terms, then the sum pass adding onto each
+         * row's y; rows without in-edges keep theirs */
         og_bin_dev b = p->bins->d;
         b.n_bins_live = b.n_bins - p->bins->n_zero_bins;
-        a.n_parts = p->bin_sum_grid + p->bin_long_grid;
+        a.n_parts = p->bins->sum_grid;
         if (a.n_parts > p->parts_cap)
         {
             og_set_error("SpMV binned pass with %u partials, %u allocated", a.n_parts, p->parts_cap);
             return -1;
         }
-        return og_launch_bin_pull(&b, &a, 0, p->bin_sum_grid, p->bin_long_grid, st, e0, e1);
+        return og_launch_bin_pull(&b, &a, p->bins->sum_grid, st, e0, e1);
     }
     /* rows [Z, N) have no in-edges: their y stays 0 */
     a.row_end = a.Z;
