@@ -197,18 +197,13 @@ out:
  * offsets.  A relabelled plan orders its rows by in-degree, so there are at
  * most about sqrt(2 E) runs and the device lists them; a plan in original
  * order (relabel 0) has its row offsets read back instead. */
-typedef struct
-{
-    uint32_t row, deg;
-} og_bin_run;
-
 static int og_bin_run_cmp(const void *a, const void *b)
 {
     const uint32_t x = ((const og_bin_run *)a)->row, y = ((const og_bin_run *)b)->row;
     return x < y ? -1 : x > y;
 }
 
-static int og_bin_runs(const og_plan *pl, og_vec *runs)
+static int og_bin_list_runs(const og_plan *pl, og_vec *runs)
 {
     const uint32_t Z = pl->Z;
     hipStream_t s = og_stream();
@@ -257,6 +252,16 @@ static int og_bin_runs(const og_plan *pl, og_vec *runs)
         o->deg = d;
     }
     free(rp);
+    return rc;
+}
+
+int og_bin_runs(const og_plan *pl, og_bin_run **runs, size_t *n)
+{
+    og_vec v = {NULL, 0, 0, sizeof(og_bin_run)};
+    const int rc = og_bin_list_runs(pl, &v);
+    if (rc) free(v.p);
+    *runs = rc ? NULL : (og_bin_run *)v.p;
+    *n = rc ? 0 : v.n;
     return rc;
 }
 
@@ -453,7 +458,7 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
         og_set_error("out of host memory");
         goto done;
     }
-    if (og_bin_runs(pl, &runs)) goto done;
+    if (og_bin_list_runs(pl, &runs)) goto done;
     {
         const uint32_t n_seg = (N + OG_BIN_SEG - 1) / OG_BIN_SEG;
         const uint32_t cus = og_num_cus() > 0 ? (uint32_t)og_num_cus() : 1;

@@ -58,7 +58,9 @@ extern "C" {
 #define OG_BIN_SEG 39936u      /* sources per segment: 156 KB of fp32 in LDS */
 #define OG_BIN_CAP 19968u      /* in-edge values per bin: 78 KB of LDS, two bins per CU */
 #define OG_BIN_PAD 0xFFFFu     /* pos of a padding entry */
-#define OG_BIN_WAVE_ROW 1024u  /* rows with more in-edges are added by a wavefront */
+/* rows with more in-edges are added by a wavefront (1024: 3 % slower at
+ * R-MAT-24, the same at 20-22) */
+#define OG_BIN_WAVE_ROW 2048u
 #define OG_BIN_RPT 1u          /* rows per thread and bin: a bin holds at most RPT * THREADS rows */
 #define OG_BIN_TILE_ALIGN 16u  /* tiles padded to 16 entries: 64-byte value runs */
 #define OG_BIN_ITEM_SRC (2048u * 64u) /* sources per gather work item at most */
@@ -113,6 +115,14 @@ typedef struct og_bin_plan
     void *mem_items, *mem_qent, *mem_src, *mem_pos, *mem_val, *mem_bins;
     void *mem_sched, *mem_blk;
 } og_bin_plan;
+
+/* Runs of rows of one in-degree: the first row and the in-degree. */
+typedef struct
+{
+    uint32_t row, deg;
+} og_bin_run;
+/* The runs of a plan's rows [0, Z), ascending (malloc'ed). */
+int og_bin_runs(const og_plan *pl, og_bin_run **runs, size_t *n);
 
 /* Builds the binned layout of a plan whose rows keep the reference's
  * in-neighbour order (relabel 2 or 0). */

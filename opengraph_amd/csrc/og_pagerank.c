@@ -16,6 +16,7 @@
 #include <time.h>
 
 #include "og_bin.h"
+#include "og_dir.h"
 #include "og_internal.h"
 #include "og_learn.h"
 #include "og_pr.h"
@@ -23,6 +24,12 @@
 #include "opengraph_amd_ext.h"
 
 #define OG_CHECK_EVERY 8u
+/* iterations of one launch of the direct pull, which stops by itself */
+#define OG_DIR_CHECK_EVERY 256u
+/* past this many in-edges the binned pull's streaming passes are as fast
+ * (R-MAT-18, 4.2 M edges: 34 us an iteration direct, 42 binned; R-MAT-17 25 and
+ * 33; uniform, 2 M: 18 and 23) */
+#define OG_DIR_MAX_EDGES (1u << 23)
 /* Rows with more in-edges than this go to the chunk waves: 12..16 is the
  * fastest on R-MAT 24 (1.38-1.40 ms against 1.47 at 32 and 1.50 at 4) and
  * on Erdos-Renyi 24 (4.80-4.87 ms against 5.08 at 32). */
@@ -116,6 +123,7 @@ void ogpu_pr_free(ogpu_pr *p)
     og_dfree(p->part_min); og_dfree(p->part_max); og_dfree(p->fin_min); og_dfree(p->fin_max);
     og_dfree(p->ticket); og_dfree(p->done); og_dfree(p->stats); og_dfree(p->qp);
     if (p->done_host) (void)hipHostFree(p->done_host);
+    if (p->report) (void)hipHostFree(p->report);
     for (uint32_t i = 0; i < p->n_iter_ev; i++) (void)hipEventDestroy(p->iter_ev[i]);
     for (uint32_t i = 0; i < p->n_kev; i++) (void)hipEventDestroy(p->kev[i]);
     free(p->iter_ev);
@@ -125,6 +133,7 @@ void ogpu_pr_free(ogpu_pr *p)
     og_dfree(p->feat); og_dfree(p->lscratch);
     og_dfree(p->chain_rows);
     og_bin_plan_destroy(p->bins);
+    og_dir_plan_destroy(p->dir);
     og_dfree(p->pp_v0); og_dfree(p->pp_dloc);
     free(p);
 }
@@ -368,7 +377,13 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
         ogpu_pr_free(p);
         return -1;
     }
-    if (binned && og_bin_plan_build(p->plan, &p->bins))
+    /* a small graph's pull runs direct unless the binned one is asked for */
+    if (binned && opt->binned != 1 && og_dir_plan_build(p->plan, OG_DIR_MAX_EDGES, &p->dir))
+    {
+        ogpu_pr_free(p);
+        return -1;
+    }
+    if (binned && !p->dir && og_bin_plan_build(p->plan, &p->bins))
     {
         if (opt->binned == 1)
         {
@@ -470,6 +485,7 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     uint32_t parts = pull_blocks > p->gv ? pull_blocks : p->gv;
     if (parts < pp_blocks) parts = pp_blocks;
     if (push_chains && parts < p->gv + chain_blocks) parts = p->gv + chain_blocks;
+    if (p->dir && parts < 2 * p->dir->d.n_bins) parts = 2 * p->dir->d.n_bins;
     if (p->bins && parts < p->bins->sum_grid) parts = p->bins->sum_grid;
     p->parts_cap = parts;
     uint32_t fins = p->n_final_pull > p->n_final_vert ? p->n_final_pull : p->n_final_vert;
@@ -599,6 +615,19 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
         ogpu_pr_free(p);
         return -1;
     }
+    if (p->dir)
+    {
+        p->dir->d.stats_cap = p->stats_cap;
+        a->bar = p->dir->d.bar;
+        a->bar_words = OG_DIR_BAR_WORDS;
+        if (opt->max_iter > 1 && opt->max_iter <= OG_DIR_CHECK_EVERY &&
+            og_hip_check(hipHostMalloc((void **)&p->report, sizeof(og_pr_report) + opt->max_iter * sizeof(og_iter_stat),
+                                       hipHostMallocDefault), "hipHostMalloc"))
+        {
+            ogpu_pr_free(p);
+            return -1;
+        }
+    }
     if (og_launch_fill_u32(p->ticket, 0, 1, og_stream())) { ogpu_pr_free(p); return -1; }
     *out = p;
     return 0;
@@ -649,7 +678,6 @@ static int og_pr_init_state(ogpu_pr *p)
     hipStream_t s = og_stream();
     p->it = 0;
     p->kev_used = 0;
-    if (og_launch_fill_u32(p->done, 0, 1, s) || og_launch_fill_u32(p->ticket, 0, 1, s)) return -1;
     if (p->next && og_launch_fill_u32((uint32_t *)p->next, 0, (uint64_t)p->g->N * 2, s)) return -1;
     og_pr_dev a = p->dev;
     a.c_out = p->c[0];
@@ -688,6 +716,16 @@ static int og_pr_launch_iter(ogpu_pr *p, uint32_t it, int allow_stop, hipEvent_t
     a.c_out = p->quant ? p->c[0] : p->c[(it + 1) & 1];
     uint32_t row = it % p->stats_cap;
     int rc;
+    if (p->dir)
+    {
+        if (e0 && og_hip_check(hipEventRecord(e0, s), "hipEventRecord")) return -1;
+        if (og_launch_dir(&p->dir->d, &a, (float *)p->c[0], (float *)p->c[1], it, 1, s)) return -1;
+        if (e1 && og_hip_check(hipEventRecord(e1, s), "hipEventRecord")) return -1;
+        a.n_parts = p->dir->d.n_bins;
+        a.n_final_blocks = 1;
+        if (it >= 2) a.z_active = 0.0 >= a.epsilon ? a.N - a.Z : 0;
+        return og_launch_final(&a, row, s);
+    }
     if (p->bins)
     {
         /* binned pull: gather, sum (rows without in-edges only in the first
@@ -830,18 +868,40 @@ static int64_t og_pr_solve(ogpu_pr *p)
 {
     hipStream_t s = og_stream();
     const uint32_t max_iter = p->opt.max_iter;
-    if (og_pr_events(&p->iter_ev, &p->n_iter_ev, max_iter + 1)) return -1;
-    if (og_hip_check(hipEventRecord(p->iter_ev[0], s), "hipEventRecord")) return -1;
+    /* (the iterations' end times are for the printed table only) */
+    if (p->print_rows && (og_pr_events(&p->iter_ev, &p->n_iter_ev, max_iter + 1) ||
+                          og_hip_check(hipEventRecord(p->iter_ev[0], s), "hipEventRecord")))
+        return -1;
     if (og_pr_init_state(p)) return -1;
     uint32_t launched = 0;
     while (launched < max_iter)
     {
-        uint32_t n = max_iter - launched < OG_CHECK_EVERY ? max_iter - launched : OG_CHECK_EVERY;
-        for (uint32_t i = 0; i < n; i++)
+        const int many = p->dir && !p->print_rows && !p->dir_single;
+        const uint32_t every = many ? OG_DIR_CHECK_EVERY : OG_CHECK_EVERY;
+        uint32_t n = max_iter - launched < every ? max_iter - launched : every;
+        if (many && n > 1)
         {
-            if (og_pr_launch_iter(p, launched + i, 1, NULL, NULL)) return -1;
-            if (og_hip_check(hipEventRecord(p->iter_ev[launched + i + 1], s), "hipEventRecord")) return -1;
+            uint32_t fail = 0;
+            if (og_launch_dir(&p->dir->d, &p->dev, (float *)p->c[0], (float *)p->c[1], launched, n, s) ||
+                og_hip_check(og_copy(&fail, p->dir->d.bar + OG_DIR_FAIL, 4, hipMemcpyDeviceToHost), "D2H barrier"))
+                return -1;
+            if (fail)
+            {
+                /* its blocks could not all be resident: from the start, one
+                 * iteration a launch */
+                p->dir_single = 1;
+                if (og_pr_init_state(p)) return -1;
+                launched = 0;
+                continue;
+            }
         }
+        else
+            for (uint32_t i = 0; i < n; i++)
+            {
+                if (og_pr_launch_iter(p, launched + i, 1, NULL, NULL)) return -1;
+                if (p->print_rows && og_hip_check(hipEventRecord(p->iter_ev[launched + i + 1], s), "hipEventRecord"))
+                    return -1;
+            }
         launched += n;
         if (og_hip_check(hipMemcpyAsync(p->done_host, p->done, 4, hipMemcpyDeviceToHost, s), "D2H done") ||
             og_hip_check(hipStreamSynchronize(s), "sync iterations") || og_pr_print_rows(p, launched))
@@ -851,31 +911,59 @@ static int64_t og_pr_solve(ogpu_pr *p)
     return launched;
 }
 
-static int og_pr_collect(ogpu_pr *p, uint32_t launched, double pr_sum, ogpu_pr_result *res);
+static int og_pr_collect(ogpu_pr *p, uint32_t launched, const og_iter_stat *rows, double pr_sum, ogpu_pr_result *res);
+
+/* A whole run of the direct pull behind one wait: the init, every iteration
+ * (the kernel stops by itself), the normalized ranks, and what the host needs
+ * written to its memory.  1: the kernel's blocks could not all be resident,
+ * nothing is done. */
+static int og_pr_run_direct(ogpu_pr *p, ogpu_pr_result *res)
+{
+    hipStream_t s = og_stream();
+    const uint32_t n = p->opt.max_iter;
+    const double t0 = og_now();
+    og_pr_dev a = p->dev;
+    a.n_parts = p->gv;
+    if (og_pr_init_state(p) || og_launch_dir(&p->dir->d, &p->dev, (float *)p->c[0], (float *)p->c[1], 0, n, s) ||
+        og_launch_normalize_report(&a, p->out_old, p->dir->d.bar + OG_DIR_FAIL, n, p->report, s) ||
+        og_hip_check(hipStreamSynchronize(s), "sync run"))
+        return -1;
+    if (p->report->fail) return 1;
+    res->seconds_total = og_now() - t0;
+    return og_pr_collect(p, n, p->report->rows, p->report->sum, res);
+}
 
 int ogpu_pr_run(ogpu_pr *p, ogpu_pr_result *res)
 {
     memset(res, 0, sizeof(*res));
     res->seconds_plan = p->seconds_plan;
     if (p->dd) return og_dd_run(p, res);
+    if (p->report && !p->print_rows && !p->dir_single)
+    {
+        const int rc = og_pr_run_direct(p, res);
+        if (rc <= 0) return rc;
+        p->dir_single = 1;
+    }
     double t0 = og_now();
     int64_t launched = og_pr_solve(p);
     if (launched < 0) return -1;
     double pr_sum = 0.0;
     if (og_pr_finish(p, &pr_sum)) return -1;
     res->seconds_total = og_now() - t0;
-    return og_pr_collect(p, (uint32_t)launched, pr_sum, res);
+    return og_pr_collect(p, (uint32_t)launched, NULL, pr_sum, res);
 }
 
-/* Statistics rows of the last solve: iterations by the stop rule, the
- * reference's iteration count, last error / active. */
-static int og_pr_collect(ogpu_pr *p, uint32_t launched, double pr_sum, ogpu_pr_result *res)
+/* Statistics rows of the last solve (already on the host, or NULL): iterations
+ * by the stop rule, the reference's iteration count, last error / active. */
+static int og_pr_collect(ogpu_pr *p, uint32_t launched, const og_iter_stat *stats, double pr_sum, ogpu_pr_result *res)
 {
     hipStream_t s = og_stream();
     const uint32_t max_iter = p->opt.max_iter;
     free(p->rows_host);
     p->rows_host = (og_iter_stat *)calloc(launched ? launched : 1, sizeof(og_iter_stat));
-    if (launched &&
+    if (!p->rows_host) { og_set_error("out of host memory"); return -1; }
+    if (stats) memcpy(p->rows_host, stats, (size_t)launched * sizeof(og_iter_stat));
+    else if (launched &&
         (og_hip_check(hipMemcpyAsync(p->rows_host, p->stats, (size_t)launched * sizeof(og_iter_stat),
                                      hipMemcpyDeviceToHost, s), "D2H stats") ||
          og_hip_check(hipStreamSynchronize(s), "sync stats")))
@@ -1846,7 +1934,7 @@ int ogpu_multi_result(ogpu_multi *m, uint32_t g, ogpu_pr_result *res, float *ran
     double pr_sum = 0.0;
     if (og_pr_finish(p, &pr_sum)) return -1;
     uint32_t launched = m->launched[g] > 0 ? (uint32_t)m->launched[g] : 0;
-    if (og_pr_collect(p, launched, pr_sum, res)) return -1;
+    if (og_pr_collect(p, launched, NULL, pr_sum, res)) return -1;
     res->seconds_plan = p->seconds_plan;
     return ranks ? ogpu_pr_ranks(p, ranks) : 0;
 }

@@ -101,6 +101,8 @@ typedef struct og_pr_dev
     float *fin_min, *fin_max;
     uint32_t *ticket;
     uint32_t *done;
+    uint32_t *bar;           /* direct pull: its barrier's words, zeroed by the init kernel */
+    uint32_t bar_words;
     og_iter_stat *stats;
     og_qparams *qp, *qp_next;
     /* data-driven variants (pageRank.c:2405-2896) */
@@ -202,6 +204,17 @@ int og_launch_init(const og_pr_dev *a, int mode, const float *init_old, float in
                    hipStream_t s);
 int og_launch_final(const og_pr_dev *a, uint32_t it, hipStream_t s);
 int og_launch_normalize(const og_pr_dev *a, float *d_out_old, double *d_sum, hipStream_t s);
+/* The same, and what the host reads of a finished run in one place it can
+ * read without a copy (host memory): the sum, the word *fail, the statistics
+ * rows [0, n_rows). */
+typedef struct og_pr_report
+{
+    double sum;
+    uint32_t fail, pad;
+    og_iter_stat rows[];
+} og_pr_report;
+int og_launch_normalize_report(const og_pr_dev *a, float *d_out_old, const uint32_t *fail, uint32_t n_rows,
+                               og_pr_report *host, hipStream_t s);
 int og_launch_fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t s);
 /* data-driven variants */
 int og_launch_dd_contrib(const og_pr_dev *a, hipStream_t s);

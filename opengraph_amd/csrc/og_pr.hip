@@ -1220,13 +1220,23 @@ __global__ __launch_bounds__(OG_BLOCK) void og_final_kernel(og_pr_dev a, uint32_
 /* ------------------------------------------------------------------ */
 
 /* r = initial ranks (pageRank.c:65-70 or the caller's start vector, given
- * in old ids), c = contributions of r, min/max partials for quantization. */
+ * in old ids), c = contributions of r, min/max partials for quantization; the
+ * run's flags and counters cleared. */
 template <int MODE>
 __global__ __launch_bounds__(OG_BLOCK) void og_init_kernel(og_pr_dev a, const float *init_old,
                                                           float init_value)
 {
     og_stat st;
     og_stat_init(st);
+    if (blockIdx.x == 0)
+    {
+        if (threadIdx.x == 0)
+        {
+            *a.done = 0;
+            *a.ticket = 0;
+        }
+        for (uint32_t i = threadIdx.x; i < a.bar_words; i += OG_BLOCK) a.bar[i] = 0;
+    }
     for (uint32_t v = blockIdx.x * OG_BLOCK + threadIdx.x; v < a.N; v += gridDim.x * OG_BLOCK)
     {
         float r = init_old ? init_old[a.new2old[v]] : a.ppr ? (v == a.ppr_src ? 1.0f : 0.0f) : init_value;
@@ -1271,6 +1281,20 @@ __global__ void og_sum_parts_kernel(const double *p, uint32_t n, double *out)
     for (uint32_t i = threadIdx.x; i < n; i += OG_BLOCK) s += p[i];
     s = og_block_sum<double>(s);
     if (threadIdx.x == 0) *out = s;
+}
+
+__global__ void og_report_kernel(const double *p, uint32_t n, const uint32_t *fail, const og_iter_stat *rows,
+                                 uint32_t n_rows, og_pr_report *out)
+{
+    double s = 0.0;
+    for (uint32_t i = threadIdx.x; i < n; i += OG_BLOCK) s += p[i];
+    s = og_block_sum<double>(s);
+    for (uint32_t i = threadIdx.x; i < n_rows; i += OG_BLOCK) out->rows[i] = rows[i];
+    if (threadIdx.x == 0)
+    {
+        out->sum = s;
+        out->fail = *fail;
+    }
 }
 
 /* ------------------------------------------------------------------ */
@@ -1498,6 +1522,14 @@ extern "C" int og_launch_final(const og_pr_dev *a, uint32_t it, hipStream_t s)
 {
     OG_LAUNCH(og_final_kernel, dim3(a->n_final_blocks), dim3(OG_BLOCK), 0, s, *a, it);
     return og_hip_check(og_launch_status(), "og_final_kernel");
+}
+
+extern "C" int og_launch_normalize_report(const og_pr_dev *a, float *d_out_old, const uint32_t *fail, uint32_t n_rows,
+                                          og_pr_report *host, hipStream_t s)
+{
+    OG_LAUNCH(og_normalize_kernel, dim3(a->n_parts), dim3(OG_BLOCK), 0, s, *a, d_out_old);
+    OG_LAUNCH(og_report_kernel, dim3(1), dim3(OG_BLOCK), 0, s, a->part_err, a->n_parts, fail, a->stats, n_rows, host);
+    return og_hip_check(og_launch_status(), "og_normalize_kernel");
 }
 
 extern "C" int og_launch_normalize(const og_pr_dev *a, float *d_out_old, double *d_sum,

@@ -62,6 +62,11 @@ struct ogpu_pr
     /* binned fp32 pull (og_bin.h): layout, blocks of its final reduction */
     struct og_bin_plan *bins;
     uint32_t n_final_bin;
+    /* direct fp32 pull (og_dir.h): the iterations of a small graph in one
+     * launch */
+    struct og_dir_plan *dir;
+    int dir_single;           /* one iteration a launch */
+    og_pr_report *report;     /* host memory a whole run's results land in */
     /* partitioned push (og_push_part_kernel): destination ranges (device
      * n_pp + 1 row bounds), each inverse-CSR edge's offset in its range,
      * the first range pushed, blocks of its final reduction */

@@ -19,6 +19,7 @@
 #include <time.h>
 
 #include "og_bin.h"
+#include "og_dir.h"
 #include "og_internal.h"
 #include "og_pr.h"
 #include "og_pr_run.h"
@@ -139,6 +140,12 @@ static int og_spmv_launch_iter(ogpu_spmv *s, hipEvent_t e0, hipEvent_t e1)
     }
     a.spmv = 1;
     a.next = s->acc;
+    if (p->dir)
+    {
+        if (e0 && og_hip_check(hipEventRecord(e0, st), "hipEventRecord")) return -1;
+        if (og_launch_dir(&p->dir->d, &a, (float *)s->terms, (float *)s->terms, 0, 1, st)) return -1;
+        return e1 ? og_hip_check(hipEventRecord(e1, st), "hipEventRecord") : 0;
+    }
     if (p->bins)
     {
         /* binned: gather of the terms, then the sum pass adding onto each
