@@ -267,10 +267,10 @@ int og_bin_runs(const og_plan *pl, og_bin_run **runs, size_t *n)
 
 /* Bins: first the pieces of the long rows (more than OG_BIN_CAP in-edges;
  * OG_BIN_CAP in-edges each, in CSR order), then consecutive rows of one kind
- * (thread rows, wavefront rows of more than OG_BIN_WAVE_ROW in-edges) with at
+ * (thread rows, wavefront rows of more than wave_row in-edges) with at
  * most cap <= OG_BIN_CAP in-edges together (or one row of more) and
  * OG_BIN_RPT * OG_BIN_THREADS rows. */
-static int og_bin_pack(const og_plan *pl, const og_vec *runs, uint32_t cap, og_vec *bins)
+static int og_bin_pack(const og_plan *pl, const og_vec *runs, uint32_t cap, uint32_t wave_row, og_vec *bins)
 {
     const og_bin_run *run = (const og_bin_run *)runs->p;
     const uint32_t Z = pl->Z;
@@ -301,7 +301,7 @@ static int og_bin_pack(const og_plan *pl, const og_vec *runs, uint32_t cap, og_v
     for (size_t i = 0; i < runs->n; i++)
     {
         const uint32_t r1 = i + 1 < runs->n ? run[i + 1].row : Z, deg = run[i].deg;
-        const uint32_t kind = deg > OG_BIN_WAVE_ROW ? OG_BIN_WAVE_ROWS : OG_BIN_THREAD_ROWS;
+        const uint32_t kind = deg > wave_row ? OG_BIN_WAVE_ROWS : OG_BIN_THREAD_ROWS;
         uint32_t r = run[i].row;
         if (deg > OG_BIN_CAP)
         {
@@ -431,7 +431,7 @@ static uint32_t og_bin_item_src(const uint32_t *seg_quads, uint32_t n_seg, uint3
     return (uint32_t)size;
 }
 
-int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
+int og_bin_plan_build(const og_plan *pl, int mode, og_bin_plan **out)
 {
     *out = NULL;
     const uint32_t N = pl->N, E = pl->E, Z = pl->Z, H = pl->H;
@@ -462,7 +462,8 @@ int og_bin_plan_build(const og_plan *pl, og_bin_plan **out)
     {
         const uint32_t n_seg = (N + OG_BIN_SEG - 1) / OG_BIN_SEG;
         const uint32_t cus = og_num_cus() > 0 ? (uint32_t)og_num_cus() : 1;
-        if (og_bin_pack(pl, &runs, og_bin_cap(E, n_seg, 2 * cus), &bins))
+        if (og_bin_pack(pl, &runs, og_bin_cap(E, n_seg, 2 * cus),
+                        mode == OG_MODE_F32 ? OG_BIN_WAVE_ROW : OG_BIN_CAP, &bins))
         {
             og_set_error("out of host memory");
             goto done;

@@ -59,7 +59,8 @@ extern "C" {
 #define OG_BIN_CAP 19968u      /* in-edge values per bin: 78 KB of LDS, two bins per CU */
 #define OG_BIN_PAD 0xFFFFu     /* pos of a padding entry */
 /* rows with more in-edges are added by a wavefront (1024: 3 % slower at
- * R-MAT-24, the same at 20-22) */
+ * R-MAT-24, the same at 20-22); the integer modes' bins take any number of
+ * lanes per row instead */
 #define OG_BIN_WAVE_ROW 2048u
 #define OG_BIN_RPT 1u          /* rows per thread and bin: a bin holds at most RPT * THREADS rows */
 #define OG_BIN_TILE_ALIGN 16u  /* tiles padded to 16 entries: 64-byte value runs */
@@ -126,14 +127,22 @@ int og_bin_runs(const og_plan *pl, og_bin_run **runs, size_t *n);
 
 /* Builds the binned layout of a plan whose rows keep the reference's
  * in-neighbour order (relabel 2 or 0). */
-int og_bin_plan_build(const og_plan *pl, og_bin_plan **out);
+int og_bin_plan_build(const og_plan *pl, int mode, og_bin_plan **out);
 void og_bin_plan_destroy(og_bin_plan *b);
 
-/* One binned pull iteration: gather, then the sum pass; ev0 / ev1 (may be
+/* Arithmetic the binned and direct pulls run in: 32-bit gathered elements,
+ * fp32 sums in the reference's order or u64 sums (OG_MODE_FX64 gathers the fp32
+ * quotients and converts them where they are added). */
+static inline int og_bin_mode(int mode)
+{
+    return mode == OG_MODE_F32 || mode == OG_MODE_FX64 || mode == OG_MODE_FX32 || mode == OG_MODE_Q32;
+}
+
+/* One binned pull iteration in `mode`: gather, then the sum pass; ev0 / ev1 (may be
  * NULL) bracket them.  Statistics partials: the sum pass's blocks; then the
  * final reduction. */
-int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, uint32_t sum_grid, hipStream_t s, hipEvent_t ev0,
-                       hipEvent_t ev1);
+int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, int mode, uint32_t sum_grid, hipStream_t s,
+                       hipEvent_t ev0, hipEvent_t ev1);
 
 /* plan-build kernels (og_bin.hip): the rows' runs of equal in-degree
  * (pairs row, in-degree; *n zeroed by the caller), the tiles' sizes, their

@@ -111,44 +111,45 @@ __global__ __launch_bounds__(GT) void og_bin_gather_kernel(og_bin_dev b, const f
 /* ------------------------------------------------------------------ */
 
 /* What a bin's rows need besides their values -- slot range (row
- * offsets), old rank, out-degree -- for the OG_BIN_RPT rows a thread holds:
- * row og_bin_meta_row(d, k) for slot k.  Thread rows: thread t holds rows
- * t, t + BT, ...; wavefront rows: lane l of wavefront w holds the
- * wavefront's rows l, l + 64, ... (rows w + BW * l + BT * k).  Loaded with
- * the bin's entries, one bin ahead, so adding a bin's rows issues no
- * global load (a load there would wait for the next bin's entries too:
+ * offsets), old rank, out-degree -- of the row a thread holds.  fp32 thread
+ * rows: thread t row t; wavefront rows: lane l of wavefront w the wavefront's
+ * l-th (row w + BW * l); integer modes: thread t row t / G, G lanes per row.
+ * Loaded with the bin's entries, one bin ahead, so adding a bin's rows issues
+ * no global load (a load there would wait for the next bin's entries too:
  * loads complete in order). */
 struct og_bin_meta
 {
-    uint32_t p0[OG_BIN_RPT], p1[OG_BIN_RPT], deg[OG_BIN_RPT];
-    float prev[OG_BIN_RPT];
+    uint32_t p0, p1, deg;
+    float prev;
 };
 
-__device__ __forceinline__ uint32_t og_bin_meta_row(const og_bin_desc &d, uint32_t k)
+/* integer modes: log2 of the lanes per row, all the block's threads on the
+ * bin's rows, at most a wavefront each */
+__device__ __forceinline__ uint32_t og_bin_group(const og_bin_desc &d)
 {
-    const uint32_t t = d.kind == OG_BIN_WAVE_ROWS ? (threadIdx.x >> 6) + BW * (threadIdx.x & 63) : threadIdx.x;
-    return d.row0 + t + BT * k;
+    const uint32_t n = d.row1 - d.row0;   /* <= BT */
+    return min(6u, n <= 1 ? 6u : (uint32_t)__builtin_clz(n - 1) - (uint32_t)__builtin_clz(BT - 1));
 }
 
+template <int MODE>
 __device__ __forceinline__ void og_bin_meta_load(const og_pr_dev &a, const og_bin_desc &d, og_bin_meta &m)
 {
     if (d.kind == OG_BIN_PIECE)
     {
-        m.prev[0] = __builtin_nontemporal_load(&a.r[d.row0]);
-        m.deg[0] = __builtin_nontemporal_load(&a.outdeg[d.row0]);
+        m.prev = __builtin_nontemporal_load(&a.r[d.row0]);
+        m.deg = __builtin_nontemporal_load(&a.outdeg[d.row0]);
         return;
     }
-#pragma unroll
-    for (uint32_t k = 0; k < OG_BIN_RPT; k++)
+    const uint32_t t = MODE != OG_MODE_F32             ? threadIdx.x >> og_bin_group(d)
+                       : d.kind == OG_BIN_WAVE_ROWS ? (threadIdx.x >> 6) + BW * (threadIdx.x & 63)
+                                                     : threadIdx.x;
+    const uint32_t v = d.row0 + t;
+    if (v < d.row1)
     {
-        const uint32_t v = og_bin_meta_row(d, k);
-        if (v < d.row1)
-        {
-            m.p0[k] = a.row_ptr[v];
-            m.p1[k] = a.row_ptr[v + 1];
-            m.prev[k] = __builtin_nontemporal_load(&a.r[v]);
-            m.deg[k] = __builtin_nontemporal_load(&a.outdeg[v]);
-        }
+        m.p0 = a.row_ptr[v];
+        m.p1 = a.row_ptr[v + 1];
+        m.prev = __builtin_nontemporal_load(&a.r[v]);
+        m.deg = __builtin_nontemporal_load(&a.outdeg[v]);
     }
 }
 
@@ -211,14 +212,18 @@ __device__ __forceinline__ void og_bin_put(const og_bin_dev &b, float *slot, con
 }
 
 /* Block i takes the bins sched[blk[i], blk[i + 1]) in that order (a long
- * row's pieces one after the other), then, while rows without in-edges still
+ * row's pieces one after the other); integer modes put all the block's
+ * threads on a bin's rows, a power of two each (a thread per row, the fp32
+ * split, left most of them idle: 400 us at R-MAT-22, now 128); then, while rows without in-edges still
  * change, every gridDim.x-th of their bins.  Bound by the streamed entries (6
  * bytes each); two blocks a CU, so that one's rows overlap the other's
  * entries.  R-MAT-24: 490 us = 3.6 TB/s (567 us beside a long-row kernel on
  * CUs of its own before); R-MAT-22: 117 us, where that kernel's longest row
  * took 158; R-MAT-16, whose wavefront rows bound it: 17 us against 33. */
+template <int MODE>
 __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_dev a)
 {
+    typedef typename og_mode<MODE>::acc A;
     __shared__ __align__(16) float slot[OG_BIN_CAP];
     if (*a.done) return;
     og_bin_stat st;
@@ -230,13 +235,13 @@ __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_d
     og_bin_desc d;
     og_bin_regs regs;
     og_bin_meta meta;
-    float carry = 0.0f;   /* the running sum of a long row between its pieces (wavefront 0) */
-    static_assert(OG_BIN_RPT == 1, "a lane holds one wavefront row");
+    A carry = 0;          /* a long row's sum between its pieces: wavefront 0's running one, or a thread's share */
+    static_assert(OG_BIN_RPT == 1 && OG_BIN_THREADS == 512, "a thread holds one row; og_bin_group");
     if (q < qe)
     {
         d = b.sched[q];
         og_bin_load(b, d, regs);
-        og_bin_meta_load(a, d, meta);
+        og_bin_meta_load<MODE>(a, d, meta);
     }
     for (; q < qe; q++)
     {
@@ -251,20 +256,53 @@ __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_d
         {
             d = b.sched[q + 1];
             og_bin_load(b, d, regs);
-            og_bin_meta_load(a, d, meta);
+            og_bin_meta_load<MODE>(a, d, meta);
         }
         __syncthreads();
-        if (cd.kind == OG_BIN_THREAD_ROWS)
+        if constexpr (MODE != OG_MODE_F32)
         {
-#pragma unroll
-            for (uint32_t k = 0; k < OG_BIN_RPT; k++)
+            if (cd.kind != OG_BIN_PIECE)
             {
-                const uint32_t v = cd.row0 + threadIdx.x + BT * k;
-                if (v >= cd.row1) break;
-                /* (an SpMV pass continues the row's running y) */
-                const float s = og_bin_row_sum(slot, cm.p0[k] - cd.pos0, cm.p1[k] - cd.pos0,
-                                               a.spmv ? cm.prev[k] : 0.0f);
-                og_bin_epilogue_pf(a, v, s, cm.prev[k], cm.deg[k], st);
+                const uint32_t lg = og_bin_group(cd), G = 1u << lg;
+                const uint32_t v = cd.row0 + (threadIdx.x >> lg);
+                if (v < cd.row1)
+                {
+                    const uint32_t j0 = cm.p0 - cd.pos0, j1 = cm.p1 - cd.pos0, g = threadIdx.x & (G - 1);
+                    A s = G == 1 ? og_bin_int_row_sum<MODE>(slot, j0, j1)
+                                 : og_bin_int_strided<MODE>(slot, j0 + g, j1, G);
+                    for (uint32_t o = 1; o < G; o <<= 1) s += __shfl_xor(s, o, 64);
+                    if (g == 0) og_bin_epilogue_pf<MODE>(a, v, s, cm.prev, cm.deg, st);
+                }
+            }
+            else
+            {
+                /* every thread its share of the row's pieces, added up at the last */
+                if (cd.row1 & OG_BIN_FIRST) carry = 0;
+                carry += og_bin_int_strided<MODE>(slot, threadIdx.x, cd.cnt, BT);
+                if (cd.row1 & OG_BIN_LAST)
+                {
+                    A s = carry;
+                    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+                    __syncthreads();   /* slot is read */
+                    if (lane == 0) ((uint64_t *)slot)[wave] = s;
+                    __syncthreads();
+                    if (threadIdx.x == 0)
+                    {
+                        s = 0;
+                        for (uint32_t w = 0; w < BW; w++) s += ((const uint64_t *)slot)[w];
+                        og_bin_epilogue_pf<MODE>(a, cd.row0, s, cm.prev, cm.deg, st);
+                    }
+                }
+            }
+        }
+        else if (cd.kind == OG_BIN_THREAD_ROWS)
+        {
+            const uint32_t v = cd.row0 + threadIdx.x;
+            if (v < cd.row1)
+            {
+                /* (a SpMV pass continues the row's running y) */
+                const float s = og_bin_row_sum(slot, cm.p0 - cd.pos0, cm.p1 - cd.pos0, a.spmv ? cm.prev : 0.0f);
+                og_bin_epilogue_pf<MODE>(a, v, s, cm.prev, cm.deg, st);
             }
         }
         else
@@ -277,13 +315,13 @@ __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_d
             uint32_t l = 0;
             for (uint32_t v = cd.row0 + wave; v < row1; v += BW, l++)
             {
-                const uint32_t j0 = piece ? 0 : (uint32_t)__builtin_amdgcn_readlane(cm.p0[0], l) - cd.pos0;
-                const uint32_t j1 = piece ? cd.cnt : (uint32_t)__builtin_amdgcn_readlane(cm.p1[0], l) - cd.pos0;
-                const float prev = og_bin_lane(cm.prev[0], l);
-                const uint32_t deg = (uint32_t)__builtin_amdgcn_readlane(cm.deg[0], l);
+                const uint32_t j0 = piece ? 0 : (uint32_t)__builtin_amdgcn_readlane(cm.p0, l) - cd.pos0;
+                const uint32_t j1 = piece ? cd.cnt : (uint32_t)__builtin_amdgcn_readlane(cm.p1, l) - cd.pos0;
+                const float prev = og_bin_lane(cm.prev, l);
+                const uint32_t deg = (uint32_t)__builtin_amdgcn_readlane(cm.deg, l);
                 carry = og_bin_wave_sum(slot, j0, j1, !first ? carry : a.spmv ? prev : 0.0f,
                                         first ? OG_BIN_HEAD : 0);
-                if (last && lane == 0) og_bin_epilogue_pf(a, v, carry, prev, deg, st);
+                if (last && lane == 0) og_bin_epilogue_pf<MODE>(a, v, carry, prev, deg, st);
             }
         }
     }
@@ -294,18 +332,17 @@ __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_d
         for (uint32_t k = 0; k < OG_BIN_RPT; k++)
         {
             const uint32_t v = z.row0 + threadIdx.x + BT * k;
-            if (v < z.row1) og_bin_epilogue(a, v, 0.0f, st);
+            if (v < z.row1) og_bin_epilogue<MODE>(a, v, 0, st);
         }
     }
-    og_bin_stat r = og_bin_block_stat<BT>(st);
-    og_bin_write_part(a, blockIdx.x, r);
+    og_bin_write_part(a, blockIdx.x, og_bin_block_stat<BT, MODE == OG_MODE_Q32>(st));
 }
 
 /* ------------------------------------------------------------------ */
 /* launch                                                              */
 /* ------------------------------------------------------------------ */
 
-extern "C" int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, uint32_t sum_grid, hipStream_t s,
+extern "C" int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, int mode, uint32_t sum_grid, hipStream_t s,
                                   hipEvent_t ev0, hipEvent_t ev1)
 {
     if (ev0 && og_hip_check(hipEventRecord(ev0, s), "hipEventRecord")) return -1;
@@ -313,7 +350,14 @@ extern "C" int og_launch_bin_pull(const og_bin_dev *b, const og_pr_dev *a, uint3
         OG_LAUNCH(og_bin_gather_kernel, dim3(og_num_cus() > 0 ? og_num_cus() : 1), dim3(GT), 0, s, *b,
                   (const float *)a->g_in,
                   (const uint32_t *)a->done);
-    OG_LAUNCH(og_bin_sum_kernel, dim3(sum_grid), dim3(BT), 0, s, *b, *a);
+    switch (mode)
+    {
+    case OG_MODE_F32: OG_LAUNCH(og_bin_sum_kernel<OG_MODE_F32>, dim3(sum_grid), dim3(BT), 0, s, *b, *a); break;
+    case OG_MODE_FX64: OG_LAUNCH(og_bin_sum_kernel<OG_MODE_FX64>, dim3(sum_grid), dim3(BT), 0, s, *b, *a); break;
+    case OG_MODE_FX32: OG_LAUNCH(og_bin_sum_kernel<OG_MODE_FX32>, dim3(sum_grid), dim3(BT), 0, s, *b, *a); break;
+    case OG_MODE_Q32: OG_LAUNCH(og_bin_sum_kernel<OG_MODE_Q32>, dim3(sum_grid), dim3(BT), 0, s, *b, *a); break;
+    default: og_set_error("og_launch_bin_pull: bad mode %d", mode); return -1;
+    }
     if (ev1 && og_hip_check(hipEventRecord(ev1, s), "hipEventRecord")) return -1;
     return og_hip_check(og_launch_status(), "og_bin_pull");
 }

@@ -15,6 +15,7 @@
 /* Rows of more in-edges are added by a wavefront: a thread takes about 13
  * cycles a term, which the whole grid waits for. */
 #define OG_DIR_WAVE_ROW 512u
+#define OG_DIR_WAVE_ROW_INT 128u
 
 void og_dir_plan_destroy(og_dir_plan *b)
 {
@@ -26,8 +27,8 @@ void og_dir_plan_destroy(og_dir_plan *b)
 
 /* Bins of at most cap in-edges (or one row) into out (room for most);
  * returns their number, most + 1 when there are more. */
-static uint32_t og_dir_pack(const og_bin_run *run, size_t n_runs, uint32_t Z, uint32_t cap, og_dir_bin *out,
-                            uint32_t most)
+static uint32_t og_dir_pack(const og_bin_run *run, size_t n_runs, uint32_t Z, uint32_t cap, uint32_t wave_row,
+                            og_dir_bin *out, uint32_t most)
 {
     uint32_t n = 0, pos = 0;
     og_dir_bin *d = NULL;   /* the open bin */
@@ -35,7 +36,7 @@ static uint32_t og_dir_pack(const og_bin_run *run, size_t n_runs, uint32_t Z, ui
     {
         const uint32_t r1 = i + 1 < n_runs ? run[i + 1].row : Z, deg = run[i].deg;
         const uint32_t kind = deg > OG_DIR_CAP ? OG_BIN_PIECE
-                            : deg > OG_DIR_WAVE_ROW ? OG_BIN_WAVE_ROWS : OG_BIN_THREAD_ROWS;
+                            : deg > wave_row ? OG_BIN_WAVE_ROWS : OG_BIN_THREAD_ROWS;
         uint32_t r = run[i].row;
         while (r < r1)
         {
@@ -66,7 +67,7 @@ static uint32_t og_dir_pack(const og_bin_run *run, size_t n_runs, uint32_t Z, ui
     return n;
 }
 
-int og_dir_plan_build(const og_plan *pl, uint32_t max_edges, og_dir_plan **out)
+int og_dir_plan_build(const og_plan *pl, int mode, uint32_t max_edges, og_dir_plan **out)
 {
     *out = NULL;
     const uint32_t E = pl->E, N = pl->N, Z = pl->Z;
@@ -87,7 +88,8 @@ int og_dir_plan_build(const og_plan *pl, uint32_t max_edges, og_dir_plan **out)
     if (og_bin_runs(pl, &run, &n_runs)) goto done;
     uint32_t n = most + 1;
     for (uint64_t cap = OG_DIR_EDGES; n > most && cap <= OG_DIR_CAP; cap += cap / 4)
-        if ((uint64_t)E <= cap * most) n = og_dir_pack(run, n_runs, Z, (uint32_t)cap, bins, most);
+        if ((uint64_t)E <= cap * most) n = og_dir_pack(run, n_runs, Z, (uint32_t)cap, mode == OG_MODE_F32 ? OG_DIR_WAVE_ROW : OG_DIR_WAVE_ROW_INT,
+                            bins, most);
     if (n > most)
     {
         rc = 0;

@@ -70,7 +70,7 @@ typedef struct og_dir_plan
 
 /* The bins of a plan in CSR order for at most max_edges in-edges; *out stays
  * NULL (and 0 is returned) where the graph does not fit. */
-int og_dir_plan_build(const og_plan *pl, uint32_t max_edges, og_dir_plan **out);
+int og_dir_plan_build(const og_plan *pl, int mode, uint32_t max_edges, og_dir_plan **out);
 void og_dir_plan_destroy(og_dir_plan *b);
 /* Blocks of the kernel the device holds at once. */
 uint32_t og_dir_resident(void);
@@ -81,7 +81,7 @@ uint32_t og_dir_resident(void);
  * word and leave, and the run is to be started again one iteration a launch
  * (n = 1: nothing waits; the statistics are partials for the final
  * reduction, as the other pulls'). */
-int og_launch_dir(const og_dir_dev *b, const og_pr_dev *a, float *c0, float *c1, uint32_t it0, uint32_t n,
+int og_launch_dir(const og_dir_dev *b, const og_pr_dev *a, int mode, void *c0, void *c1, uint32_t it0, uint32_t n,
                   hipStream_t s);
 
 #ifdef __cplusplus

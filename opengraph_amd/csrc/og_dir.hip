@@ -188,10 +188,11 @@ __device__ __forceinline__ void og_dir_put(uint32_t i0, uint32_t n, const float 
         }
 }
 
-template <bool WAIT>
+template <int MODE, bool WAIT>
 __global__ __launch_bounds__(DT, 4) void og_dir_kernel(og_dir_dev b, og_pr_dev a, float *c0, float *c1, uint32_t it0,
                                                        uint32_t n_it)
 {
+    typedef typename og_mode<MODE>::acc A;
     __shared__ __align__(16) float slot[OG_DIR_CAP];
     if (*a.done) return;
     const uint32_t lane = threadIdx.x & 63;
@@ -225,16 +226,21 @@ __global__ __launch_bounds__(DT, 4) void og_dir_kernel(og_dir_dev b, og_pr_dev a
         og_bin_stat_init(st);
         /* the rank of a row from its sum, its statistics and next
          * contribution (pageRank.c:1016-1028, :989-996) */
-        auto update = [&](uint32_t row, float sum, float prev, uint32_t dg) {
-            if (a.spmv) return sum;   /* SpMV: the running y, started from the old one */
-            const float nr = OG_BASE_PR + (OG_DAMP * sum);
+        auto update = [&](uint32_t row, A sum, float prev, uint32_t dg) {
+            if (a.spmv)   /* fp32: the running y, started from the old one; u64: added onto y */
+            {
+                if constexpr (MODE == OG_MODE_F32) return sum;
+                ((uint64_t *)a.next)[row] += (uint64_t)sum;
+                return prev;
+            }
+            const float nr = og_next_rank<MODE>(sum, a.qp);
             const double err = fabs((double)(nr - prev));
             st.err += err;
             st.active += err >= a.epsilon;
-            og_dir_post(&cn[row], dg ? nr / (float)dg : 0.0f);
+            og_dir_post(&cn[row], og_bin_contrib<MODE>(nr, dg));
             return nr;
         };
-        float y = 0.0f;
+        A y = 0;
         for (uint32_t q0 = 0; q0 < d.cnt; q0 += OG_DIR_CAP)
         {
             const uint32_t n = min(d.cnt - q0, OG_DIR_CAP);
@@ -273,7 +279,9 @@ __global__ __launch_bounds__(DT, 4) void og_dir_kernel(og_dir_dev b, og_pr_dev a
             if (d.kind == OG_BIN_THREAD_ROWS)
             {
                 rp = r;
-                if (mine) r = update(v, og_bin_row_sum(slot, p0, p1, a.spmv ? r : 0.0f), r, deg);
+                if (mine)
+                    r = update(v, og_row_by_thread<MODE>(slot, p0, p1, (A)(MODE == OG_MODE_F32 && a.spmv ? r : 0.0f)), r,
+                               deg);
             }
             else
             {
@@ -285,7 +293,8 @@ __global__ __launch_bounds__(DT, 4) void og_dir_kernel(og_dir_dev b, og_pr_dev a
                     const uint32_t j1 = piece ? n : (uint32_t)__builtin_amdgcn_readlane(p1, l);
                     const float prev = og_bin_lane(r, l);
                     const uint32_t dg = (uint32_t)__builtin_amdgcn_readlane(deg, l);
-                    y = og_bin_wave_sum<28>(slot, j0, j1, q0 ? y : a.spmv ? prev : 0.0f, q0 ? 0 : OG_BIN_HEAD);
+                    const A y0 = q0 ? y : (A)(MODE == OG_MODE_F32 && a.spmv ? prev : 0.0f);
+                    y = og_row_by_wave<MODE, 28>(slot, j0, j1, y0, q0 ? 0 : OG_BIN_HEAD);
                     if (lane == l && q0 + n >= d.cnt)
                     {
                         rp = r;
@@ -302,7 +311,7 @@ __global__ __launch_bounds__(DT, 4) void og_dir_kernel(og_dir_dev b, og_pr_dev a
             /* rows without in-edges reach their fixed rank in iteration 0 and
              * have both contribution buffers filled after iteration 1 */
             for (uint32_t z = a.Z + blockIdx.x * DT + threadIdx.x; z < a.N; z += gridDim.x * DT)
-                a.r[z] = update(z, 0.0f, a.r[z], a.outdeg[z]);
+                a.r[z] = update(z, 0, a.r[z], a.outdeg[z]);
         }
         if (WAIT) og_dir_done(b, a, it, st);
         else
@@ -323,20 +332,36 @@ __global__ __launch_bounds__(DT, 4) void og_dir_kernel(og_dir_dev b, og_pr_dev a
     if (mine) a.r[v] = stop ? rp : r;
 }
 
+/* (the fp32 kernel needs the most registers) */
 extern "C" uint32_t og_dir_resident(void)
 {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void *)og_dir_kernel<true>, DT, 0) != hipSuccess) return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void *)og_dir_kernel<OG_MODE_F32, true>, DT, 0) !=
+        hipSuccess)
+        return 0;
     const uint32_t n = nb > 0 ? (uint32_t)nb * (uint32_t)og_num_cus() : 0;
     return n < OG_DIR_MAX_BLOCKS ? n : OG_DIR_MAX_BLOCKS;
 }
 
-extern "C" int og_launch_dir(const og_dir_dev *b, const og_pr_dev *a, float *c0, float *c1, uint32_t it0, uint32_t n,
-                             hipStream_t s)
+template <int MODE>
+static void og_launch_dir_t(const og_dir_dev *b, const og_pr_dev *a, float *c0, float *c1, uint32_t it0, uint32_t n,
+                            hipStream_t s)
 {
     if (n > 1 || a->spmv)
-        OG_LAUNCH(og_dir_kernel<true>, dim3(b->n_bins), dim3(DT), 0, s, *b, *a, c0, c1, it0, n);
+        OG_LAUNCH((og_dir_kernel<MODE, true>), dim3(b->n_bins), dim3(DT), 0, s, *b, *a, c0, c1, it0, n);
     else if (n)
-        OG_LAUNCH(og_dir_kernel<false>, dim3(b->n_bins), dim3(DT), 0, s, *b, *a, c0, c1, it0, n);
+        OG_LAUNCH((og_dir_kernel<MODE, false>), dim3(b->n_bins), dim3(DT), 0, s, *b, *a, c0, c1, it0, n);
+}
+
+extern "C" int og_launch_dir(const og_dir_dev *b, const og_pr_dev *a, int mode, void *c0, void *c1, uint32_t it0,
+                             uint32_t n, hipStream_t s)
+{
+    switch (mode)
+    {
+    case OG_MODE_F32: og_launch_dir_t<OG_MODE_F32>(b, a, (float *)c0, (float *)c1, it0, n, s); break;
+    case OG_MODE_FX64: og_launch_dir_t<OG_MODE_FX64>(b, a, (float *)c0, (float *)c1, it0, n, s); break;
+    case OG_MODE_FX32: og_launch_dir_t<OG_MODE_FX32>(b, a, (float *)c0, (float *)c1, it0, n, s); break;
+    default: og_set_error("og_launch_dir: bad mode %d", mode); return -1;
+    }
     return og_hip_check(og_launch_status(), "og_dir_kernel");
 }

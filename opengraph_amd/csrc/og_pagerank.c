@@ -330,6 +330,20 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
      * source rules it out */
     int binned = opt->variant == 0 && !opt->ppr && opt->binned != 2 && g->E > 0 &&
                  !(plan && plan->relabel == 1 && plan->H);
+    /* The same passes serve the other variants whose gathered elements are 32
+     * bits (the u64 fixed-point ones gather the fp32 quotients they convert)
+     * where no option asks for a row split, a hot copy or a scatter: the
+     * integer sums are exact in any order, and a push's destination adds its
+     * terms one at a time, here in the reference's source order.  (The fp32
+     * push with exact_above 0 keeps its atomics.)  Per iteration: u64 pull,
+     * R-MAT-22, 377 us by the hot-cache gather, 235 streamed (the partitioned
+     * u64 push likewise); fp32 push, R-MAT-20, 243 us by ranges with their
+     * chains beside them, 80 streamed. */
+    if (!binned && (opt->variant == 1 || opt->variant == 2 || opt->variant == 3 || opt->variant == 4 ||
+                    opt->variant == 9) &&
+        opt->binned == 0 && !opt->hub_threshold && !opt->hot_cache && g->E > 0 &&
+        !(opt->variant == 1 && !opt->exact_above) && !(plan && plan->relabel == 1 && plan->H))
+        binned = 1;
     if (opt->binned == 1 && !binned)
     {
         og_set_error("binned pull: fp32 pull (variant 0, not personalized) on a graph with edges and a "
@@ -364,7 +378,8 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     else
     {
         const uint32_t rel = (chain || binned) && p->opt.relabel == 1 ? 2u : p->opt.relabel;
-        if (og_plan_build(g, rel, chain ? OG_EXACT_SEQ_T : p->opt.hub_threshold, chain_t, p->push || p->dd,
+        if (og_plan_build(g, rel, chain ? OG_EXACT_SEQ_T : p->opt.hub_threshold, chain_t,
+                          (p->push && !binned) || p->dd,
                           &p->plan))
         {
             free(p);
@@ -378,12 +393,12 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
         return -1;
     }
     /* a small graph's pull runs direct unless the binned one is asked for */
-    if (binned && opt->binned != 1 && og_dir_plan_build(p->plan, OG_DIR_MAX_EDGES, &p->dir))
+    if (binned && opt->binned != 1 && !p->quant && og_dir_plan_build(p->plan, p->mode, OG_DIR_MAX_EDGES, &p->dir))
     {
         ogpu_pr_free(p);
         return -1;
     }
-    if (binned && !p->dir && og_bin_plan_build(p->plan, &p->bins))
+    if (binned && !p->dir && og_bin_plan_build(p->plan, p->mode, &p->bins))
     {
         if (opt->binned == 1)
         {
@@ -393,9 +408,22 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
         p->bins = NULL;   /* default: the gather pull instead */
     }
     if (p->bins) p->n_final_bin = og_final_blocks(p->bins->sum_grid, 0);
+    const int streamed = p->bins || p->dir;
+    if (binned && !streamed && opt->variant != 0 && p->own_plan)
+    {
+        /* no layout for this graph: the variant's own kernels and their plan */
+        og_plan_destroy(p->plan);
+        p->plan = NULL;
+        if (og_plan_build(g, p->opt.relabel, p->opt.hub_threshold,
+                          opt->variant == 1 && opt->exact_above ? OG_PUSH_EXACT_ABOVE : 0, p->push, &p->plan))
+        {
+            ogpu_pr_free(p);
+            return -1;
+        }
+    }
     p->seconds_plan = og_now() - t0;
     og_plan *pl = p->plan;
-    if ((p->push || p->dd) && !pl->push_src)
+    if ((p->push || p->dd) && !streamed && !pl->push_src)
     {
         og_set_error("plan has no forward edges for variant %u", opt->variant);
         ogpu_pr_free(p);
@@ -410,7 +438,7 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     uint32_t hot_grid = 0;
     /* (the every-row-exact pull stages its chains in LDS instead; the
      * chains of exact_above run beside it, in a launch of their own) */
-    if (!p->push && !p->dd && opt->hot_cache != 2 && !p->chain_rows)
+    if (!p->push && !p->dd && opt->hot_cache != 2 && !p->chain_rows && !(streamed && opt->variant != 0))
     {
         int on = opt->hot_cache == 1;
         const uint32_t nh = (uint32_t)(OG_HOT_BYTES / og_elem_bytes(p->mode));
@@ -447,7 +475,7 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
      * their chunks skipped; otherwise every chunk */
     uint32_t n_chains = 0, ch_first = 0, chunk_blocks = pl->n_chunk_blocks;
     /* (a borrowed plan may carry chains the options did not ask for) */
-    const int push_chains = opt->variant == 1 && opt->exact_above && pl->L;
+    const int push_chains = opt->variant == 1 && opt->exact_above && pl->L && !streamed;
     if (p->chain_rows)
     {
         n_chains = pl->C;
@@ -475,7 +503,7 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     p->n_final_pull = og_final_blocks(pull_blocks, pl->H);
     p->n_final_vert = og_final_blocks(p->gv + (push_chains ? chain_blocks : 0), 0);
     /* the default push (hot_cache 0): partitioned by destination range */
-    if (p->push && !p->dd && opt->hot_cache == 0 && og_push_parts(p, push_chains ? n_chains : 0))
+    if (p->push && !p->dd && opt->hot_cache == 0 && !streamed && og_push_parts(p, push_chains ? n_chains : 0))
     {
         ogpu_pr_free(p);
         return -1;
@@ -499,7 +527,8 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     p->c[0] = og_dalloc((size_t)N * cbytes);
     p->c[1] = og_dalloc((size_t)N * cbytes);
     if (p->quant) p->cq = og_dalloc((size_t)N * eb);
-    if (p->push || p->dd) p->next = og_dalloc((size_t)N * 8);
+    const int need_next = (p->push && !streamed) || p->dd;
+    if (need_next) p->next = og_dalloc((size_t)N * 8);
     p->chunk_sum = og_dalloc((size_t)(pl->n_chunks + 1) * 8);
     p->out_old = og_dalloc((size_t)N * 4);
     p->d_sum = og_dalloc(8);
@@ -515,7 +544,7 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     p->done = og_dalloc(4);
     p->stats = og_dalloc((size_t)p->stats_cap * sizeof(og_iter_stat));
     p->qp = og_dalloc(2 * sizeof(og_qparams));
-    if (!p->r || !p->c[0] || !p->c[1] || (p->quant && !p->cq) || ((p->push || p->dd) && !p->next) ||
+    if (!p->r || !p->c[0] || !p->c[1] || (p->quant && !p->cq) || (need_next && !p->next) ||
         !p->chunk_sum || !p->out_old || !p->d_sum || !p->part_err || !p->part_act || !p->part_min ||
         !p->part_max || !p->fin_err || !p->fin_act || !p->fin_min || !p->fin_max || !p->ticket ||
         !p->done || !p->stats || !p->qp)
@@ -690,7 +719,10 @@ static int og_pr_init_state(ogpu_pr *p)
         if (!p->init_d) { og_set_error("init_mode 2 needs ogpu_pr_set_init"); return -1; }
         init_old = p->init_d;
     }
-    if (og_launch_init(&a, p->mode, init_old, init_value, s)) return -1;
+    /* (the streamed u64 modes gather the fp32 quotients) */
+    if (og_launch_init(&a, (p->bins || p->dir) && p->mode == OG_MODE_FX64 ? OG_MODE_F32 : p->mode, init_old,
+                       init_value, s))
+        return -1;
     if (p->quant)
     {
         a.n_final_blocks = p->n_final_vert;
@@ -703,6 +735,16 @@ static int og_pr_init_state(ogpu_pr *p)
         if (og_launch_quantize(&a, p->mode, s)) return -1;
     }
     return 0;
+}
+
+/* The next iteration's quantized contributions, with the parameters of the
+ * final reduction of iteration `it`. */
+static int og_pr_quantize_next(ogpu_pr *p, og_pr_dev a, uint32_t it)
+{
+    a.cq_src = p->c[0];
+    a.cq_dst = p->cq;
+    a.qp = p->qp + ((it + 1) & 1);
+    return og_launch_quantize(&a, p->mode, og_stream());
 }
 
 static int og_pr_launch_iter(ogpu_pr *p, uint32_t it, int allow_stop, hipEvent_t e0, hipEvent_t e1)
@@ -719,7 +761,7 @@ static int og_pr_launch_iter(ogpu_pr *p, uint32_t it, int allow_stop, hipEvent_t
     if (p->dir)
     {
         if (e0 && og_hip_check(hipEventRecord(e0, s), "hipEventRecord")) return -1;
-        if (og_launch_dir(&p->dir->d, &a, (float *)p->c[0], (float *)p->c[1], it, 1, s)) return -1;
+        if (og_launch_dir(&p->dir->d, &a, p->mode, p->c[0], p->c[1], it, 1, s)) return -1;
         if (e1 && og_hip_check(hipEventRecord(e1, s), "hipEventRecord")) return -1;
         a.n_parts = p->dir->d.n_bins;
         a.n_final_blocks = 1;
@@ -731,7 +773,7 @@ static int og_pr_launch_iter(ogpu_pr *p, uint32_t it, int allow_stop, hipEvent_t
         /* binned pull: gather, sum (rows without in-edges only in the first
          * two iterations, as below), final reduction */
         og_bin_dev b = p->bins->d;
-        if (it >= 2)
+        if (it >= 2 && !p->quant)   /* (a quantized run's range is over every contribution) */
         {
             b.n_bins_live = b.n_bins - p->bins->n_zero_bins;
             a.z_active = 0.0 >= a.epsilon ? a.N - a.Z : 0;
@@ -743,10 +785,8 @@ static int og_pr_launch_iter(ogpu_pr *p, uint32_t it, int allow_stop, hipEvent_t
             og_set_error("binned pull with %u partials, %u allocated", a.n_parts, p->parts_cap);
             return -1;
         }
-        if (og_launch_bin_pull(&b, &a, p->bins->sum_grid, s, e0, e1) ||
-            og_launch_final(&a, row, s))
-            return -1;
-        return 0;
+        if (og_launch_bin_pull(&b, &a, p->mode, p->bins->sum_grid, s, e0, e1) || og_launch_final(&a, row, s)) return -1;
+        return p->quant ? og_pr_quantize_next(p, a, it) : 0;
     }
     if (!p->push && !p->quant && !p->dd && it >= 2)
     {
@@ -782,14 +822,7 @@ static int og_pr_launch_iter(ogpu_pr *p, uint32_t it, int allow_stop, hipEvent_t
         rc = og_launch_push(&a, p->mode, row, s, e0, e1);
     }
     if (rc) return -1;
-    if (p->quant)
-    {
-        a.cq_src = p->c[0];
-        a.cq_dst = p->cq;
-        a.qp = p->qp + ((it + 1) & 1);
-        if (og_launch_quantize(&a, p->mode, s)) return -1;
-    }
-    return 0;
+    return p->quant ? og_pr_quantize_next(p, a, it) : 0;
 }
 
 int og_pr_events(hipEvent_t **arr, uint32_t *have, uint32_t need)
@@ -882,7 +915,7 @@ static int64_t og_pr_solve(ogpu_pr *p)
         if (many && n > 1)
         {
             uint32_t fail = 0;
-            if (og_launch_dir(&p->dir->d, &p->dev, (float *)p->c[0], (float *)p->c[1], launched, n, s) ||
+            if (og_launch_dir(&p->dir->d, &p->dev, p->mode, p->c[0], p->c[1], launched, n, s) ||
                 og_hip_check(og_copy(&fail, p->dir->d.bar + OG_DIR_FAIL, 4, hipMemcpyDeviceToHost), "D2H barrier"))
                 return -1;
             if (fail)
@@ -924,7 +957,7 @@ static int og_pr_run_direct(ogpu_pr *p, ogpu_pr_result *res)
     const double t0 = og_now();
     og_pr_dev a = p->dev;
     a.n_parts = p->gv;
-    if (og_pr_init_state(p) || og_launch_dir(&p->dir->d, &p->dev, (float *)p->c[0], (float *)p->c[1], 0, n, s) ||
+    if (og_pr_init_state(p) || og_launch_dir(&p->dir->d, &p->dev, p->mode, p->c[0], p->c[1], 0, n, s) ||
         og_launch_normalize_report(&a, p->out_old, p->dir->d.bar + OG_DIR_FAIL, n, p->report, s) ||
         og_hip_check(hipStreamSynchronize(s), "sync run"))
         return -1;
@@ -1059,6 +1092,7 @@ int ogpu_pr_ranks(ogpu_pr *p, float *host_out)
 double ogpu_pr_bytes_per_iteration(const ogpu_pr *p)
 {
     double N = p->g->N, E = p->g->E;
+    if (p->bins || p->dir) return 8.0 * E + 20.0 * N;   /* index + 32-bit element per edge */
     switch (p->opt.variant)
     {
     /* the partitioned pushes: source id, u16 destination offset and the

@@ -195,9 +195,9 @@ int og_launch_push_dloc(const uint32_t *row_ptr, const uint32_t *pp_v0, uint32_t
 int og_launch_push_scatter(const og_pr_dev *a, int pmode, hipStream_t s, hipEvent_t ev0,
                            hipEvent_t ev1);
 /* SpMV (og_spmv.hip): the per-vertex terms w * x of -p code 0..3 in new ids
- * into `terms` (fp32, u32 or u64), and vector_output in old ids from r
+ * into `terms` (fp32, u32 or, code 3 unless narrow, u64), and vector_output in old ids from r
  * (codes 0, 1) or the u64 accumulators in next (codes 2, 3). */
-int og_launch_spmv_terms(const og_pr_dev *a, uint32_t code, void *terms, hipStream_t s);
+int og_launch_spmv_terms(const og_pr_dev *a, uint32_t code, int narrow, void *terms, hipStream_t s);
 int og_launch_spmv_out(const og_pr_dev *a, uint32_t code, float *out_old, hipStream_t s);
 int og_launch_quantize(const og_pr_dev *a, int mode, hipStream_t s);
 int og_launch_init(const og_pr_dev *a, int mode, const float *init_old, float init_value,

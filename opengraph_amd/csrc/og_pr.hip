@@ -42,71 +42,13 @@
 #include <hip/hip_runtime.h>
 
 #include "og_internal.h"
+#include "og_modes.h"
 #include "og_pr.h"
 
 #define OG_BLOCK 256
 #define OG_WAVES (OG_BLOCK / 64)
 #define OG_CH_SLOTS (OG_CH / 64) /* edges per lane of a chunk */
 #define OG_ROW_BATCH 8           /* edges of a short row loaded together */
-
-/* ------------------------------------------------------------------ */
-/* per-mode arithmetic                                                 */
-/* ------------------------------------------------------------------ */
-
-template <int MODE> struct og_mode;
-template <> struct og_mode<OG_MODE_F32>  { typedef float    elem; typedef float    acc; };
-template <> struct og_mode<OG_MODE_FX64> { typedef uint64_t elem; typedef uint64_t acc; };
-template <> struct og_mode<OG_MODE_FX32> { typedef uint32_t elem; typedef uint64_t acc; };
-template <> struct og_mode<OG_MODE_FX16> { typedef uint16_t elem; typedef uint64_t acc; };
-template <> struct og_mode<OG_MODE_FX8>  { typedef uint8_t  elem; typedef uint64_t acc; };
-template <> struct og_mode<OG_MODE_Q32>  { typedef uint32_t elem; typedef uint64_t acc; };
-template <> struct og_mode<OG_MODE_Q16>  { typedef uint16_t elem; typedef uint64_t acc; };
-template <> struct og_mode<OG_MODE_Q8>   { typedef uint8_t  elem; typedef uint64_t acc; };
-
-/* The reference's next-rank expression for each variant, from the gathered
- * sum (pageRank.c:1016, :1278, :1412, :1544, :1676, :1944, :2083, :2222). */
-template <int MODE>
-__device__ __forceinline__ float og_next_rank(typename og_mode<MODE>::acc s, const og_qparams *qp)
-{
-    const float base = OG_BASE_PR, damp = OG_DAMP;
-    if constexpr (MODE == OG_MODE_F32) return base + (damp * s);
-    else if constexpr (MODE == OG_MODE_FX64)
-        return (float)((double)base + ((double)damp * ((double)s / 4294967296.0)));
-    else if constexpr (MODE == OG_MODE_FX32) return base + (damp * ((float)s / 65536.0f));
-    else if constexpr (MODE == OG_MODE_FX16) return base + (damp * ((float)s / 16384.0f));
-    else if constexpr (MODE == OG_MODE_FX8) return base + (damp * ((float)s / 64.0f));
-    else if constexpr (MODE == OG_MODE_Q32) return base + damp * (float)(qp->scale_d * (double)s);
-    else return base + damp * (qp->scale_f * (float)s);
-}
-
-/* The contribution the next iteration gathers (pageRank.c:989-996 and the
- * fixed-point conversions of fixedPoint.h:29-36).  Quantized modes store
- * the fp32 quotient; og_quantize_kernel converts it once the scale is known. */
-template <int MODE>
-__device__ __forceinline__ void og_store_contrib(void *c_out, uint32_t v, float r, uint32_t deg)
-{
-    /* Stores are non-temporal: the next iteration reads them back through
-     * L2, this one must not let them evict the lines being gathered. */
-    if constexpr (MODE == OG_MODE_F32 || MODE >= OG_MODE_Q32)
-        __builtin_nontemporal_store(deg ? r / (float)deg : 0.0f, &((float *)c_out)[v]);
-    else
-    {
-        typedef typename og_mode<MODE>::elem E;
-        E x = 0;
-        if (deg)
-        {
-            float q = r / (float)deg;
-            if constexpr (MODE == OG_MODE_FX64) x = og_fixed64_of(q);
-            else if constexpr (MODE == OG_MODE_FX32)
-                x = (uint32_t)og_x86_f2i64(q * 65536.0f + (q >= 0 ? 0.5f : -0.5f));
-            else if constexpr (MODE == OG_MODE_FX16)
-                x = (uint16_t)og_x86_f2i32(q * 16384.0f + (q >= 0 ? 0.5f : -0.5f));
-            else
-                x = (uint8_t)og_x86_f2i32(q * 64.0f + (q >= 0 ? 0.5f : -0.5f));
-        }
-        __builtin_nontemporal_store(x, &((E *)c_out)[v]);
-    }
-}
 
 /* Running per-thread statistics of the epilogue. */
 struct og_stat

@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include "og_bin.h"
+#include "og_modes.h"
 #include "og_pr.h"
 
 #define OG_BIN_HEAD 64u  /* leading terms of a wavefront row added one by one */
@@ -269,62 +270,166 @@ __device__ __forceinline__ float og_bin_wave_sum(const float *slot, uint32_t j, 
     return __uint_as_float(yb);
 }
 
+/* ---- integer modes: u64 sums, exact in any order ----
+ * A value in LDS is the gathered 32-bit element: the fixed-point or quantized
+ * number itself, or (OG_MODE_FX64) the fp32 quotient its Q32.32 number is the
+ * conversion of. */
+template <int MODE> __device__ __forceinline__ uint64_t og_bin_int(float x)
+{
+    if constexpr (MODE == OG_MODE_FX64) return og_fixed64_split(x);
+    else return __float_as_uint(x);
+}
+
+template <int MODE> __device__ __forceinline__ uint64_t og_bin_int4(float4 x)
+{
+    return (og_bin_int<MODE>(x.x) + og_bin_int<MODE>(x.y)) + (og_bin_int<MODE>(x.z) + og_bin_int<MODE>(x.w));
+}
+
+/* one thread's sum of slot[j, j1) */
+template <int MODE> __device__ __forceinline__ uint64_t og_bin_int_row_sum(const float *slot, uint32_t j, uint32_t j1)
+{
+    uint64_t s = 0;
+    for (; (j & 3u) && j < j1; j++) s += og_bin_int<MODE>(slot[j]);
+    const float4 *s4 = reinterpret_cast<const float4 *>(slot);
+    for (; j + 8 <= j1; j += 8)
+    {
+        const float4 x = s4[j / 4], y = s4[j / 4 + 1];
+        s += og_bin_int4<MODE>(x) + og_bin_int4<MODE>(y);
+    }
+    for (; j < j1; j++) s += og_bin_int<MODE>(slot[j]);
+    return s;
+}
+
+/* every G-th value from slot[j] on (j: this lane's first), below j1 */
+template <int MODE>
+__device__ __forceinline__ uint64_t og_bin_int_strided(const float *slot, uint32_t j, uint32_t j1, uint32_t G)
+{
+    uint64_t s = 0;
+    for (; j + 3 * G < j1; j += 4 * G)
+    {
+        const float4 x = make_float4(slot[j], slot[j + G], slot[j + 2 * G], slot[j + 3 * G]);
+        s += og_bin_int4<MODE>(x);
+    }
+    for (; j < j1; j += G) s += og_bin_int<MODE>(slot[j]);
+    return s;
+}
+
+/* one wavefront's, the same in every lane */
+template <int MODE> __device__ __forceinline__ uint64_t og_bin_int_wave_sum(const float *slot, uint32_t j, uint32_t j1)
+{
+    uint64_t s = og_bin_int_strided<MODE>(slot, j + (threadIdx.x & 63), j1, 64);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    return s;
+}
+
+/* Row sums in the mode's own way: fp32 in order onto y0, integers onto 0. */
+template <int MODE>
+__device__ __forceinline__ typename og_mode<MODE>::acc og_row_by_thread(const float *slot, uint32_t j, uint32_t j1,
+                                                                        typename og_mode<MODE>::acc y0)
+{
+    if constexpr (MODE == OG_MODE_F32) return og_bin_row_sum(slot, j, j1, y0);
+    else return y0 + og_bin_int_row_sum<MODE>(slot, j, j1);
+}
+
+template <int MODE, uint32_t WT>
+__device__ __forceinline__ typename og_mode<MODE>::acc og_row_by_wave(const float *slot, uint32_t j, uint32_t j1,
+                                                                      typename og_mode<MODE>::acc y0, uint32_t head)
+{
+    if constexpr (MODE == OG_MODE_F32) return og_bin_wave_sum<WT>(slot, j, j1, y0, head);
+    else return y0 + og_bin_int_wave_sum<MODE>(slot, j, j1);
+}
+
 /* running statistics of the updates a thread made */
 struct og_bin_stat
 {
     double err;
     uint32_t active;
+    float cmin, cmax;   /* quantized modes: of the contributions */
 };
 
 __device__ __forceinline__ void og_bin_stat_init(og_bin_stat &s)
 {
     s.err = 0.0;
     s.active = 0;
+    s.cmin = 3.402823466e38f;
+    s.cmax = -3.402823466e38f;
+}
+
+/* the contribution of a rank as the gather wants it: fp32 quotients but for
+ * FX32's numbers (pageRank.c:989-996, fixedPoint.h:31) */
+template <int MODE> __device__ __forceinline__ float og_bin_contrib(float r, uint32_t deg)
+{
+    const float q = deg ? r / (float)deg : 0.0f;
+    if constexpr (MODE == OG_MODE_FX32)
+        return __uint_as_float(deg ? (uint32_t)og_x86_f2i64(q * 65536.0f + (q >= 0 ? 0.5f : -0.5f)) : 0u);
+    else return q;
 }
 
 /* pageRank.c:1016-1028 and the next contribution (pageRank.c:989-996),
  * with the old rank and out-degree already loaded. */
-__device__ __forceinline__ void og_bin_epilogue_pf(const og_pr_dev &a, uint32_t v, float sum, float prev,
-                                                   uint32_t deg, og_bin_stat &st)
+template <int MODE>
+__device__ __forceinline__ void og_bin_epilogue_pf(const og_pr_dev &a, uint32_t v, typename og_mode<MODE>::acc sum,
+                                                   float prev, uint32_t deg, og_bin_stat &st)
 {
     if (a.spmv)
     {
-        /* SpMV pass: the running y, started from the old one, is the sum */
-        __builtin_nontemporal_store(sum, &a.r[v]);
+        /* SpMV pass: fp32, the running y, started from the old one, is the sum */
+        if constexpr (MODE == OG_MODE_F32) __builtin_nontemporal_store(sum, &a.r[v]);
+        else ((uint64_t *)a.next)[v] += sum;
         return;
     }
-    const float nr = OG_BASE_PR + (OG_DAMP * sum);
+    const float nr = og_next_rank<MODE>(sum, a.qp);
     __builtin_nontemporal_store(nr, &a.r[v]);
     const double err = fabs((double)(nr - prev));
     st.err += err / (double)a.N;
     st.active += err >= a.epsilon;
-    __builtin_nontemporal_store(deg ? nr / (float)deg : 0.0f, &((float *)a.c_out)[v]);
+    const float c = og_bin_contrib<MODE>(nr, deg);
+    __builtin_nontemporal_store(c, &((float *)a.c_out)[v]);
+    if constexpr (MODE == OG_MODE_Q32)
+    {
+        st.cmin = fminf(st.cmin, c);
+        st.cmax = fmaxf(st.cmax, c);
+    }
 }
 
-__device__ __forceinline__ void og_bin_epilogue(const og_pr_dev &a, uint32_t v, float sum, og_bin_stat &st)
+template <int MODE>
+__device__ __forceinline__ void og_bin_epilogue(const og_pr_dev &a, uint32_t v, typename og_mode<MODE>::acc sum,
+                                                og_bin_stat &st)
 {
     const float prev = __builtin_nontemporal_load(&a.r[v]);
     const uint32_t deg = __builtin_nontemporal_load(&a.outdeg[v]);
-    og_bin_epilogue_pf(a, v, sum, prev, deg, st);
+    og_bin_epilogue_pf<MODE>(a, v, sum, prev, deg, st);
 }
 
-/* og_stat over the block of NT threads (fixed order); result in thread 0 */
-template <uint32_t NT>
+/* the statistics over the block of NT threads (fixed order; MM: with the
+ * contributions' range); result in thread 0 */
+template <uint32_t NT, bool MM = false>
 __device__ og_bin_stat og_bin_block_stat(og_bin_stat s)
 {
     constexpr uint32_t W = NT / 64;
     __shared__ double sh_err[W];
     __shared__ uint32_t sh_act[W];
+    __shared__ float sh_min[MM ? W : 1], sh_max[MM ? W : 1];
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int o = 32; o > 0; o >>= 1)
     {
         s.err += __shfl_down(s.err, o, 64);
         s.active += __shfl_down(s.active, o, 64);
+        if constexpr (MM)
+        {
+            s.cmin = fminf(s.cmin, __shfl_down(s.cmin, o, 64));
+            s.cmax = fmaxf(s.cmax, __shfl_down(s.cmax, o, 64));
+        }
     }
     if (lane == 0)
     {
         sh_err[w] = s.err;
         sh_act[w] = s.active;
+        if constexpr (MM)
+        {
+            sh_min[w] = s.cmin;
+            sh_max[w] = s.cmax;
+        }
     }
     __syncthreads();
     og_bin_stat r;
@@ -334,21 +439,25 @@ __device__ og_bin_stat og_bin_block_stat(og_bin_stat s)
         {
             r.err += sh_err[i];
             r.active += sh_act[i];
+            if constexpr (MM)
+            {
+                r.cmin = fminf(r.cmin, sh_min[i]);
+                r.cmax = fmaxf(r.cmax, sh_max[i]);
+            }
         }
     __syncthreads();
     return r;
 }
 
-/* first-level partial idx of the final reduction (min / max unused: the
- * neutral values) */
+/* first-level partial idx of the final reduction */
 __device__ __forceinline__ void og_bin_write_part(const og_pr_dev &a, uint32_t idx, const og_bin_stat &r)
 {
     if (threadIdx.x == 0)
     {
         a.part_err[idx] = r.err;
         a.part_act[idx] = r.active;
-        a.part_min[idx] = 3.402823466e38f;
-        a.part_max[idx] = -3.402823466e38f;
+        a.part_min[idx] = r.cmin;
+        a.part_max[idx] = r.cmax;
     }
 }
 

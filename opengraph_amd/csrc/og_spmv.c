@@ -4,14 +4,11 @@
  *
  * y = 0; `iterations` times y += A^T (w x) with the fixed x and w of the
  * reference (og_spmv.hip).  The passes are PageRank's kernels with the SpMV
- * store.  -p 0 runs on the binned pull by default: every row continues y
- * in the reference's order (bit-exact); with a hub_threshold it runs on the
- * degree-binned gather pull, where rows of at most hub_threshold in-edges
- * continue y in order and longer rows add their fixed-tree sum.  -p 2 (and
- * 3 by default) gather over the in-edges, -p 1 (and 3 on request) push over
- * the forward edges, partitioned by destination range.  The integer sums of
- * -p 2 and 3 are exact in any order, so -p 3 (a push in the reference)
- * gathers by default: the same bits without atomics.
+ * store, by default the streaming ones (direct or binned): -p 0 and 1 continue
+ * y in the reference's order (bit-exact with -p 0; -p 1, its unordered atomics,
+ * has no order of its own), -p 2 and 3 add u64 sums, exact in any order.  A
+ * hub_threshold selects the degree-binned gather pull, hot_cache and scatter
+ * the pushes over the forward edges.
  */
 #include <stdio.h>
 #include <stdlib.h>
@@ -32,6 +29,7 @@ struct ogpu_spmv
     ogpu_spmv_options opt;
     int mode;                 /* arithmetic of the gathered / scattered terms */
     int scatter;              /* 1: push scatter over the forward edges */
+    int narrow;               /* code 3: 32-bit terms */
     void *terms;              /* w * x per vertex, new ids */
     uint64_t *acc;            /* u64 accumulators of -p 2, 3 */
     uint32_t it;              /* iterations enqueued since the reset */
@@ -73,12 +71,20 @@ int og_spmv_create_with(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt
     ogpu_spmv *s = (ogpu_spmv *)calloc(1, sizeof(ogpu_spmv));
     if (!s) { og_set_error("out of host memory"); return -1; }
     s->opt = o;
-    s->scatter = o.code == 1 || (o.code == 3 && o.scatter);
-    s->mode = o.code < 2 ? OG_MODE_F32 : o.code == 2 ? OG_MODE_FX32 : OG_MODE_FX64;
+    /* The default: the streaming passes (direct or binned, og_dir.h, og_bin.h)
+     * for every code -- fp32 y in the reference's order, which is one of the
+     * orders its atomics may land in, and u64 sums of the integer terms, all of
+     * which fit 32 bits.  An option that asks for a row split, a hot copy or a
+     * scatter selects the kernels it is about. */
+    const int streamed = !o.hub_threshold && !o.hot_cache && !(o.code == 3 && o.scatter) &&
+                         !(plan && plan->relabel == 1 && plan->H);
+    s->scatter = (o.code == 1 && !streamed) || (o.code == 3 && o.scatter);
+    s->mode = o.code < 2 ? OG_MODE_F32 : o.code == 2 || streamed ? OG_MODE_FX32 : OG_MODE_FX64;
     ogpu_pr_options po;
     ogpu_pr_default_options(&po);
     /* the PageRank variant whose plan, buffers and kernels the passes use */
-    po.variant = o.code == 0 ? 0 : o.code == 1 ? 1 : o.code == 2 ? 9 : (s->scatter ? 3 : 2);
+    po.variant = o.code == 0 || (o.code == 1 && streamed) ? 0 : o.code == 1 ? 1
+               : o.code == 2 || streamed ? 9 : (s->scatter ? 3 : 2);
     po.max_iter = 1;
     po.hub_threshold = o.hub_threshold;
     /* the pushes (-p 1, -p 3 scattered) are partitioned by destination
@@ -87,16 +93,14 @@ int og_spmv_create_with(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt
     po.hot_cache = o.hot_cache;
     /* every destination of the -p 1 scatter takes its adds as atomics (the
      * PageRank push would gather its longest rows instead) */
-    if (o.code == 1) po.exact_above = 0;
-    /* -p 0 with the default row split runs on the binned pull (every row's
-     * running y in the reference's order); a given hub_threshold, and the
-     * other codes, on the gather pull's kernels */
-    po.binned = o.code == 0 && o.hub_threshold == 0 ? 0 : 2;
+    if (o.code == 1 && !streamed) po.exact_above = 0;
+    po.binned = streamed || (o.code == 0 && !o.hub_threshold) ? 0 : 2;
     if (og_pr_create_with(g, plan, &po, &s->p))
     {
         free(s);
         return -1;
     }
+    s->narrow = o.code == 3 && streamed;
     s->terms = s->p->c[0];
     if (o.code >= 2)
     {
@@ -119,7 +123,7 @@ int ogpu_spmv_reset(ogpu_spmv *s)
     if (og_launch_fill_u32(p->done, 0, 1, st) || og_launch_fill_u32(p->ticket, 0, 1, st) ||
         og_launch_fill_u32((uint32_t *)p->r, 0, N, st) ||
         (s->acc && og_launch_fill_u32((uint32_t *)s->acc, 0, (uint64_t)N * 2, st)) ||
-        og_launch_spmv_terms(&a, s->opt.code, s->terms, st))
+        og_launch_spmv_terms(&a, s->opt.code, s->narrow, s->terms, st))
         return -1;
     return 0;
 }
@@ -143,7 +147,7 @@ static int og_spmv_launch_iter(ogpu_spmv *s, hipEvent_t e0, hipEvent_t e1)
     if (p->dir)
     {
         if (e0 && og_hip_check(hipEventRecord(e0, st), "hipEventRecord")) return -1;
-        if (og_launch_dir(&p->dir->d, &a, (float *)s->terms, (float *)s->terms, 0, 1, st)) return -1;
+        if (og_launch_dir(&p->dir->d, &a, s->mode, s->terms, s->terms, 0, 1, st)) return -1;
         return e1 ? og_hip_check(hipEventRecord(e1, st), "hipEventRecord") : 0;
     }
     if (p->bins)
@@ -158,7 +162,7 @@ static int og_spmv_launch_iter(ogpu_spmv *s, hipEvent_t e0, hipEvent_t e1)
             og_set_error("SpMV binned pass with %u partials, %u allocated", a.n_parts, p->parts_cap);
             return -1;
         }
-        return og_launch_bin_pull(&b, &a, p->bins->sum_grid, st, e0, e1);
+        return og_launch_bin_pull(&b, &a, s->mode, p->bins->sum_grid, st, e0, e1);
     }
     /* rows [Z, N) have no in-edges: their y stays 0 */
     a.row_end = a.Z;
@@ -242,6 +246,7 @@ int ogpu_spmv_output(ogpu_spmv *s, float *host_out)
 double ogpu_spmv_bytes_per_iteration(const ogpu_spmv *s)
 {
     const double N = s->p->g->N, E = s->p->g->E;
+    if (!s->scatter && (s->p->bins || s->p->dir)) return 8.0 * E + (s->opt.code < 2 ? 12.0 : 20.0) * N;
     switch (s->opt.code)
     {
     /* partitioned pushes: source id, u16 destination offset, gathered term
@@ -307,15 +312,16 @@ static struct SPMVStats *og_spmv_dropin(struct Arguments *arguments, struct Grap
 {
     og_graph *g = NULL;
     og_plan *plan = NULL;
-    if (og_cache_graph(graph, code == 1, &g, &plan)) og_spmv_fatal("graph upload");
+    if (og_cache_graph(graph, 0, &g, &plan)) og_spmv_fatal("graph upload");
     og_trace_entry("SPMVGraphCSR", g->N, g->E);
     ogpu_spmv_options o;
     ogpu_spmv_default_options(&o);
     o.code = code;
     ogpu_spmv *s = NULL;
-    /* -p 0 runs binned, on a plan of its own that keeps every row in CSR
-     * order (the cached plan sorts long rows for the gather pulls) */
-    if (og_spmv_create_with(g, code == 0 ? NULL : plan, &o, &s)) og_spmv_fatal("spmv setup");
+    /* on a plan of its own that keeps every row in CSR order (the cached plan
+     * sorts long rows for the gather pulls) */
+    (void)plan;
+    if (og_spmv_create_with(g, NULL, &o, &s)) og_spmv_fatal("spmv setup");
     struct SPMVStats *stats = newSPMVStatsGraphCSR(graph);
     stats->arguments = arguments;
     /* SPMV.c:663-669: the input vector the passes use */

@@ -55,14 +55,16 @@ __global__ __launch_bounds__(SB) void og_spmv_terms_fx32_kernel(og_pr_dev a, uin
 
 /* code 3 (SPMV.c:995-1030, fixedPoint.h:36 and :71-72): Q32.32 input and
  * weight DoubleToFixed64, MULFixed64V1 = the 128-bit product >> 32. */
-__global__ __launch_bounds__(SB) void og_spmv_terms_fx64_kernel(og_pr_dev a, uint64_t *__restrict__ t)
+/* (below 2^32: the weight is 429496, the input at most 1; T u32 or u64) */
+template <typename T>
+__global__ __launch_bounds__(SB) void og_spmv_terms_fx64_kernel(og_pr_dev a, T *__restrict__ t)
 {
     const uint64_t wu = og_x86_d2u64((double)0.0001f * 4294967296.0 + 0.5);
     for (uint32_t v = blockIdx.x * SB + threadIdx.x; v < a.N; v += gridDim.x * SB)
     {
         const uint64_t xq = og_x86_d2u64((double)og_spmv_x(a, v) * 4294967296.0 + 0.5);
         const uint64_t lo = wu * xq, hi = __umul64hi(wu, xq);
-        t[v] = (hi << 32) | (lo >> 32);
+        t[v] = (T)((hi << 32) | (lo >> 32));
     }
 }
 
@@ -81,13 +83,14 @@ __global__ __launch_bounds__(SB) void og_spmv_out_kernel(og_pr_dev a, uint32_t c
     }
 }
 
-extern "C" int og_launch_spmv_terms(const og_pr_dev *a, uint32_t code, void *terms, hipStream_t s)
+extern "C" int og_launch_spmv_terms(const og_pr_dev *a, uint32_t code, int narrow, void *terms, hipStream_t s)
 {
     const unsigned g = og_sgrid(a->N);
     if (code < 2) OG_LAUNCH(og_spmv_terms_f32_kernel, dim3(g), dim3(SB), 0, s, *a, (float *)terms);
     else if (code == 2)
         OG_LAUNCH(og_spmv_terms_fx32_kernel, dim3(g), dim3(SB), 0, s, *a, (uint32_t *)terms);
-    else OG_LAUNCH(og_spmv_terms_fx64_kernel, dim3(g), dim3(SB), 0, s, *a, (uint64_t *)terms);
+    else if (narrow) OG_LAUNCH(og_spmv_terms_fx64_kernel<uint32_t>, dim3(g), dim3(SB), 0, s, *a, (uint32_t *)terms);
+    else OG_LAUNCH(og_spmv_terms_fx64_kernel<uint64_t>, dim3(g), dim3(SB), 0, s, *a, (uint64_t *)terms);
     return og_hip_check(og_launch_status(), "og_spmv_terms");
 }
 
