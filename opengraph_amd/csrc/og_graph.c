@@ -387,9 +387,7 @@ int ogpu_graph_array(const ogpu_graph *gg, uint32_t which, uint32_t *host_out)
     default: og_set_error("unknown graph array %u", which); return -1;
     }
     if (n == 0) return 0;
-    if (og_hip_check(hipMemcpyAsync(host_out, src, n * 4, hipMemcpyDeviceToHost, og_stream()), "D2H"))
-        return -1;
-    return og_hip_check(hipStreamSynchronize(og_stream()), "sync");
+    return og_hip_check(og_download(host_out, src, n * 4), "D2H");
 }
 
 /* A CSR pair is well formed when, for both the forward and the inverse list

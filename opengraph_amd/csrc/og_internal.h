@@ -35,7 +35,8 @@ hipEvent_t og_side_fork(void);
 hipEvent_t og_side_join(void);
 int og_num_cus(void);
 void og_trace_entry(const char *fn, uint32_t n_vertices, uint32_t n_edges);
-/* hipMalloc / hipFree with error text; og_dalloc returns NULL on failure. */
+/* Device memory from the library's pool (og_runtime.c), of any content;
+ * og_dalloc returns NULL with the error set on failure. */
 void *og_dalloc(size_t bytes);
 void og_dfree(void *p);
 /* Checks a HIP status; on failure records "<what>: <hip error>" and returns -1. */
@@ -58,6 +59,9 @@ hipError_t og_launch_status(void);
  * complete on return (hipMemcpy itself runs on the null stream, which the
  * library's non-blocking stream does not wait for). */
 hipError_t og_copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind);
+/* The same from the device to the caller's memory, the large ones by several
+ * threads (og_runtime.c). */
+hipError_t og_download(void *dst, const void *src, size_t bytes);
 #define OG_HIP(call) do { if (og_hip_check((call), #call)) return -1; } while (0)
 /* 128-byte aligned host allocation, as the reference's my_malloc
  * (myMalloc.c:24-67); exits on failure like the reference. */

@@ -657,7 +657,12 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
             return -1;
         }
     }
-    if (og_launch_fill_u32(p->ticket, 0, 1, og_stream())) { ogpu_pr_free(p); return -1; }
+    if (og_launch_fill_u32(p->ticket, 0, 1, og_stream()) ||
+        og_hip_check(hipStreamSynchronize(og_stream()), "sync state"))
+    {
+        ogpu_pr_free(p);
+        return -1;
+    }
     *out = p;
     return 0;
 }
@@ -1083,10 +1088,7 @@ int ogpu_pr_kernel_ms(ogpu_pr *p, double *total_ms, uint32_t *count)
 
 int ogpu_pr_ranks(ogpu_pr *p, float *host_out)
 {
-    if (og_hip_check(hipMemcpyAsync(host_out, p->out_old, (size_t)p->g->N * 4, hipMemcpyDeviceToHost,
-                                    og_stream()), "D2H ranks"))
-        return -1;
-    return og_hip_check(hipStreamSynchronize(og_stream()), "sync ranks");
+    return og_hip_check(og_download(host_out, p->out_old, (size_t)p->g->N * 4), "D2H ranks");
 }
 
 double ogpu_pr_bytes_per_iteration(const ogpu_pr *p)

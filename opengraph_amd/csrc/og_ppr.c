@@ -268,12 +268,10 @@ int ogpu_ppr_run(ogpu_ppr *p, ogpu_ppr_result *res)
 
 int ogpu_ppr_ranks(ogpu_ppr *p, float *x_out)
 {
-    hipStream_t s = og_stream();
     const size_t blk = (size_t)p->g->N * p->k * 4;
     if (!p->out && !(p->out = og_dalloc(blk))) return -1;
-    if (og_launch_ppr_out(&p->dev, p->out, s) ||
-        og_hip_check(hipMemcpyAsync(x_out, p->out, blk, hipMemcpyDeviceToHost, s), "D2H ranks") ||
-        og_hip_check(hipStreamSynchronize(s), "sync ranks"))
+    if (og_launch_ppr_out(&p->dev, p->out, og_stream()) ||
+        og_hip_check(og_download(x_out, p->out, blk), "D2H ranks"))
         return -1;
     return 0;
 }

@@ -7,6 +7,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <unistd.h>
 
 #include "og_internal.h"
 #include "og_learn.h"
@@ -22,6 +23,7 @@ static hipStream_t g_stream = NULL;
 static hipStream_t g_side = NULL;
 static hipEvent_t g_fork = NULL, g_join = NULL;
 static pthread_mutex_t g_ctx_lock = PTHREAD_MUTEX_INITIALIZER;
+static size_t g_pool_cap = 0;   /* bytes of freed device memory kept */
 
 void og_set_error(const char *fmt, ...)
 {
@@ -81,6 +83,7 @@ static int og_ctx_create(void)
     hipDeviceProp_t prop;
     if (og_hip_check(hipGetDeviceProperties(&prop, g_device), "hipGetDeviceProperties")) return -1;
     g_cus = prop.multiProcessorCount;
+    g_pool_cap = prop.totalGlobalMem / 64;
     if (og_hip_check(hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking), "hipStreamCreate") ||
         og_hip_check(hipStreamCreateWithFlags(&g_side, hipStreamNonBlocking), "hipStreamCreate (side)") ||
         og_hip_check(hipEventCreateWithFlags(&g_fork, hipEventDisableTiming), "hipEventCreate (fork)") ||
@@ -133,22 +136,220 @@ void og_trace_entry(const char *fn, uint32_t n_vertices, uint32_t n_edges)
             g_cus, n_vertices, n_edges);
 }
 
+/* ---- device memory ----
+ * A graph's build and a run's setup take dozens of short-lived buffers, and
+ * hipMalloc and hipFree (which waits for the device) of the large ones cost
+ * more than the kernels between them: 10 of 21 ms from a 67 M-edge list to its
+ * ranks.  Freed blocks are kept by size and handed out again.  All the
+ * library's work is on one stream (its side stream is joined to it), so what
+ * a block's next owner enqueues runs after what its last one did, and none of
+ * these pointers leaves the library.  Kept blocks are bounded by a 64th of the
+ * device's memory, the longest unused given back first, and all of them are
+ * given back before an allocation is allowed to fail. */
+typedef struct og_block
+{
+    void *p;
+    size_t bytes;
+    struct og_block *next;
+} og_block;
+
+#define OG_POOL_SLOTS 4096u
+static pthread_mutex_t g_pool_lock = PTHREAD_MUTEX_INITIALIZER;
+static og_block *g_pool_live[OG_POOL_SLOTS];   /* handed out, by address */
+static og_block *g_pool_free = NULL;           /* kept, the last freed first */
+static size_t g_pool_bytes = 0;
+
+static unsigned og_pool_slot(const void *p)
+{
+    return (unsigned)(((uintptr_t)p >> 8) * 0x9E3779B97F4A7C15ull >> 40) & (OG_POOL_SLOTS - 1);
+}
+
+/* Sizes are rounded up by at most an eighth, so that similar ones meet; a
+ * block that is never kept is not. */
+static size_t og_pool_size(size_t bytes)
+{
+    if (bytes <= 4096) return 4096;
+    if (bytes > g_pool_cap) return bytes;
+    size_t step = 512;
+    while (step * 16 <= bytes) step *= 2;
+    return (bytes + step - 1) / step * step;
+}
+
+/* Frees the kept blocks past `most` bytes, the longest unused first. */
+static void og_pool_trim(size_t most)
+{
+    while (g_pool_bytes > most && g_pool_free)
+    {
+        og_block **q = &g_pool_free;
+        while ((*q)->next) q = &(*q)->next;
+        og_block *b = *q;
+        *q = NULL;
+        g_pool_bytes -= b->bytes;
+        (void)hipFree(b->p);
+        free(b);
+    }
+}
+
 void *og_dalloc(size_t bytes)
 {
-    void *p = NULL;
-    if (bytes == 0) bytes = 256;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess)
+    const size_t size = og_pool_size(bytes);
+    pthread_mutex_lock(&g_pool_lock);
+    og_block *b = NULL;
+    for (og_block **q = &g_pool_free; *q; q = &(*q)->next)
+        if ((*q)->bytes == size)
+        {
+            b = *q;
+            *q = b->next;
+            g_pool_bytes -= size;
+            break;
+        }
+    if (!b)
     {
-        og_set_error("hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
-        return NULL;
+        hipError_t e = hipErrorOutOfMemory;
+        b = (og_block *)malloc(sizeof(og_block));
+        if (b)
+        {
+            b->bytes = size;
+            e = hipMalloc(&b->p, size);
+            if (e != hipSuccess)
+            {
+                (void)hipGetLastError();
+                og_pool_trim(0);
+                b->bytes = bytes ? bytes : 256;
+                e = hipMalloc(&b->p, b->bytes);
+            }
+        }
+        if (e != hipSuccess)
+        {
+            free(b);
+            pthread_mutex_unlock(&g_pool_lock);
+            og_set_error("hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+            return NULL;
+        }
     }
-    return p;
+    const unsigned k = og_pool_slot(b->p);
+    b->next = g_pool_live[k];
+    g_pool_live[k] = b;
+    pthread_mutex_unlock(&g_pool_lock);
+    return b->p;
 }
 
 void og_dfree(void *p)
 {
+    if (!p) return;
+    pthread_mutex_lock(&g_pool_lock);
+    og_block **q = &g_pool_live[og_pool_slot(p)];
+    while (*q && (*q)->p != p) q = &(*q)->next;
+    og_block *b = *q;
+    if (b)
+    {
+        *q = b->next;
+        if (b->bytes <= g_pool_cap)
+        {
+            b->next = g_pool_free;
+            g_pool_free = b;
+            g_pool_bytes += b->bytes;
+            og_pool_trim(g_pool_cap);
+            p = NULL;
+        }
+        else free(b);
+    }
+    pthread_mutex_unlock(&g_pool_lock);
     if (p) (void)hipFree(p);
+}
+
+/* ---- large results to the caller's memory ----
+ * The caller's buffer is ordinary, usually fresh memory: a plain copy into it
+ * stages and faults its pages on one thread (64 MB: 6 ms, 11 GB/s).  Here
+ * each of a few threads takes every n-th piece through a pinned buffer of its
+ * own, so that the copy engine serves one thread while the others move their
+ * pieces on (64 MB: 2 ms).  Below OG_STAGE_MIN a thread costs more than it
+ * saves. */
+#define OG_STAGE_BYTES ((size_t)1 << 20)
+#define OG_STAGE_THREADS 8u
+#define OG_STAGE_MIN ((size_t)4 << 20)
+static pthread_mutex_t g_stage_lock = PTHREAD_MUTEX_INITIALIZER;
+static char *g_stage = NULL;                    /* a piece per thread */
+static hipEvent_t g_stage_ev[OG_STAGE_THREADS];
+
+typedef struct og_stage_job
+{
+    char *dst;
+    const char *src;
+    size_t bytes;
+    uint32_t self, threads;
+    hipError_t err;
+} og_stage_job;
+
+static int og_stage_ready(void)
+{
+    if (g_stage) return 1;
+    void *p = NULL;
+    if (hipHostMalloc(&p, OG_STAGE_THREADS * OG_STAGE_BYTES, hipHostMallocDefault) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return 0;
+    }
+    for (uint32_t i = 0; i < OG_STAGE_THREADS; i++)
+        if (hipEventCreateWithFlags(&g_stage_ev[i], hipEventDisableTiming) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            while (i-- > 0) (void)hipEventDestroy(g_stage_ev[i]);
+            (void)hipHostFree(p);
+            return 0;
+        }
+    g_stage = (char *)p;
+    return 1;
+}
+
+static void *og_stage_run(void *arg)
+{
+    og_stage_job *j = (og_stage_job *)arg;
+    char *buf = g_stage + j->self * OG_STAGE_BYTES;
+    j->err = hipSetDevice(g_device);
+    for (size_t o = j->self * OG_STAGE_BYTES; o < j->bytes && j->err == hipSuccess; o += j->threads * OG_STAGE_BYTES)
+    {
+        const size_t k = j->bytes - o < OG_STAGE_BYTES ? j->bytes - o : OG_STAGE_BYTES;
+        j->err = hipMemcpyAsync(buf, j->src + o, k, hipMemcpyDeviceToHost, g_stream);
+        if (j->err == hipSuccess) j->err = hipEventRecord(g_stage_ev[j->self], g_stream);
+        if (j->err == hipSuccess) j->err = hipEventSynchronize(g_stage_ev[j->self]);
+        if (j->err == hipSuccess) memcpy(j->dst + o, buf, k);
+    }
+    return NULL;
+}
+
+hipError_t og_download(void *dst, const void *src, size_t bytes)
+{
+    hipPointerAttribute_t at;
+    memset(&at, 0, sizeof(at));
+    /* the caller's own pinned (or device) memory takes the copy directly */
+    int plain = bytes < OG_STAGE_MIN ||
+                (hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered);
+    if (bytes >= OG_STAGE_MIN) (void)hipGetLastError();   /* a pointer it does not know */
+    if (plain) return og_copy(dst, src, bytes, hipMemcpyDeviceToHost);
+    pthread_mutex_lock(&g_stage_lock);
+    if (!og_stage_ready())
+    {
+        pthread_mutex_unlock(&g_stage_lock);
+        return og_copy(dst, src, bytes, hipMemcpyDeviceToHost);
+    }
+    const long cpus = sysconf(_SC_NPROCESSORS_ONLN);
+    const uint32_t n = cpus > 0 && cpus < (long)OG_STAGE_THREADS ? (uint32_t)cpus : OG_STAGE_THREADS;
+    og_stage_job job[OG_STAGE_THREADS];
+    pthread_t th[OG_STAGE_THREADS];
+    int started[OG_STAGE_THREADS] = {0};
+    for (uint32_t i = 0; i < n; i++) job[i] = (og_stage_job){(char *)dst, (const char *)src, bytes, i, n, hipSuccess};
+    for (uint32_t i = 1; i < n; i++) started[i] = !pthread_create(&th[i], NULL, og_stage_run, &job[i]);
+    og_stage_run(&job[0]);
+    hipError_t e = job[0].err;
+    for (uint32_t i = 1; i < n; i++)
+    {
+        if (started[i]) pthread_join(th[i], NULL);
+        else og_stage_run(&job[i]);
+        if (e == hipSuccess) e = job[i].err;
+    }
+    pthread_mutex_unlock(&g_stage_lock);
+    return e;
 }
 
 void *og_host_alloc(size_t bytes)
@@ -194,9 +395,22 @@ int ogpu_device_info(char *name, size_t name_len, int *num_cus, size_t *total_me
 
 int ogpu_malloc(void **ptr, size_t bytes)
 {
+    /* (the caller's: not from the pool, whose reuse follows the library stream) */
     if (og_ctx_ensure()) return -1;
-    *ptr = og_dalloc(bytes);
-    return *ptr ? 0 : -1;
+    *ptr = NULL;
+    hipError_t e = hipMalloc(ptr, bytes ? bytes : 256);
+    if (e != hipSuccess)
+    {
+        (void)hipGetLastError();
+        pthread_mutex_lock(&g_pool_lock);
+        og_pool_trim(0);
+        pthread_mutex_unlock(&g_pool_lock);
+        e = hipMalloc(ptr, bytes ? bytes : 256);
+    }
+    if (e == hipSuccess) return 0;
+    *ptr = NULL;
+    og_set_error("hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    return -1;
 }
 
 int ogpu_free(void *ptr)

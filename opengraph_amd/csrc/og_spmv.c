@@ -237,10 +237,7 @@ int ogpu_spmv_iteration_seconds(ogpu_spmv *s, uint32_t i, double *seconds)
 
 int ogpu_spmv_output(ogpu_spmv *s, float *host_out)
 {
-    if (og_hip_check(hipMemcpyAsync(host_out, s->p->out_old, (size_t)s->p->g->N * 4, hipMemcpyDeviceToHost,
-                                    og_stream()), "D2H vector_output"))
-        return -1;
-    return og_hip_check(hipStreamSynchronize(og_stream()), "sync vector_output");
+    return og_hip_check(og_download(host_out, s->p->out_old, (size_t)s->p->g->N * 4), "D2H vector_output");
 }
 
 double ogpu_spmv_bytes_per_iteration(const ogpu_spmv *s)
