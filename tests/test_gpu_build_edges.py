@@ -38,6 +38,24 @@ def test_stable_sort_at_tile_edges(edges, ids):
     g.free()
 
 
+@pytest.mark.parametrize("edges", [1, 2, 3, 4, 5, 7, 8, 9, 4099, 300_002])
+@pytest.mark.parametrize("ids", [1, 3, 50_000])
+def test_mapping_at_quad_edges(edges, ids):
+    """Run starts and lengths of the sorted keys: runs within, across and
+    exactly of the four keys a thread reads, and no key at all."""
+    rng = np.random.default_rng(edges + ids)
+    s, d = (rng.integers(0, ids, edges).astype(np.uint32) for _ in range(2))
+    s[-1] = ids - 1
+    g = og.Graph.from_edges(s, d, 0)
+    n = g.num_vertices
+    for side, key in (("f", s), ("i", d)):
+        deg = np.bincount(key, minlength=n)
+        start = np.where(deg > 0, np.concatenate([[0], np.cumsum(deg)[:-1]]), 0)
+        assert np.array_equal(g.array(side + "_out_degree"), deg)
+        assert np.array_equal(g.array(side + "_edges_idx"), start)
+    g.free()
+
+
 @pytest.mark.parametrize("relabel", [0, 1, 2])
 @pytest.mark.parametrize("degrees", [[1], [16, 17], [511, 512, 513], [4095, 4096, 4097], [19968], [19969, 1],
                                      [19967, 1, 1, 40000]])
