@@ -117,8 +117,9 @@ typedef struct
                                edges), 1 on, 2 off -- one persistent block per CU that
                                serves the gathers of the lowest vertex ids (the hottest
                                after relabelling) from a 157 KB LDS copy; same results.
-                               push (variants 1, 3, 5): 0 default: partitioned -- the
-                               destinations in ranges of at most 16384 rows, one block
+                               push (variants 1, 3, 5): 0 default: variants 1 (with
+                               exact_above) and 3 as `binned` says, else partitioned
+                               -- the destinations in ranges of at most 16384 rows, one block
                                per range adds each in-edge's contribution to its
                                destination's accumulator with an LDS atomic (one running
                                sum per destination, as the reference's atomics) and runs
@@ -142,12 +143,16 @@ typedef struct
                                (the reference's source-ordered adds) and left out of the
                                atomic adds */
     uint32_t binned;        /* fp32 pull (variant 0, not personalized): 0 default (on),
-                               1 on, 2 off -- the binned pull: per iteration a gather pass
+                               1 on, 2 off; variants 1 (with exact_above), 2, 3, 4 and 9:
+                               0 on unless hub_threshold or hot_cache is given, else off
+                               -- the binned passes: per iteration a gather pass
                                writes each edge's contribution, source segment by source
                                segment from LDS, into an edge array grouped by destination
                                bins, and a sum pass adds every row from LDS in CSR order
-                               (rows longer than a bin by one block each).  Every row is
-                               the reference's running sum to the bit, and all global
+                               (rows longer than a bin by one block each); with 0 and up
+                               to 2^23 edges one launch runs all iterations instead,
+                               gathering through L2, with the same sums.  Every fp32 row
+                               is the reference's running sum to the bit, and all global
                                accesses stream.  hub_threshold, exact_above and hot_cache
                                then apply only to the learned start's feature pass */
     uint32_t warm_classes;  /* learned start (ogpu_pr_set_init_learned): the predicted
@@ -365,21 +370,22 @@ void ogpu_ppr_free(ogpu_ppr *p);
  *     reference's CSR order (bit-exact); with a hub_threshold, the gather
  *     pull: rows of at most hub_threshold in-edges bit-exact, longer rows
  *     add their fixed-tree sum to y (0xFFFFFFFF: every row bit-exact);
- *   1 push, fp32 atomics over the forward edges (unordered, as the
- *     reference's omp atomic), the hottest destinations summed per block
- *     in LDS first;
+ *   1 push, fp32 (unordered in the reference's omp atomic): by default each
+ *     destination's terms in CSR order, one of its orders; with a
+ *     hub_threshold or hot_cache by atomics;
  *   2 pull, Q16.16 inputs, u64 sums of (7 * x) >> 16 (bit-exact);
  *   3 push, Q32.32, u64 sums of (w * x) >> 32 (bit-exact): gathered over
- *     the in-edges by default, scattered with u64 atomics when scatter = 1. */
+ *     the in-edges by default, scattered with u64 atomics when scatter = 1.
+ * By default every code runs on the streaming passes (ogpu_pr_options.binned). */
 typedef struct ogpu_spmv ogpu_spmv;
 typedef struct
 {
     uint32_t code;           /* the reference's -p, 0..3 */
-    uint32_t hub_threshold;  /* 0 (default): -p 0 runs on the binned pull, every row's running
-                                y in the reference's order; otherwise -p 0 runs on the gather
-                                pull with this row-class threshold, as ogpu_pr_options */
-    uint32_t hot_cache;      /* as ogpu_pr_options: the pushes (-p 1, -p 3 scattered) are
-                                partitioned by destination range by default (0), 1 scatters
+    uint32_t hub_threshold;  /* 0 (default): the streaming passes, every fp32 row's running
+                                y in the reference's order; otherwise the gather pull with
+                                this row-class threshold, as ogpu_pr_options */
+    uint32_t hot_cache;      /* as ogpu_pr_options: the pushes off the streaming passes are
+                                partitioned by destination range (0), 1 scatters
                                 with LDS accumulators for the hottest destinations, 2 with
                                 plain atomics */
     uint32_t scatter;        /* code 3: 1 scatters with atomics instead of gathering */

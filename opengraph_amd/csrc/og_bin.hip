@@ -217,7 +217,7 @@ __device__ __forceinline__ void og_bin_put(const og_bin_dev &b, float *slot, con
  * split, left most of them idle: 400 us at R-MAT-22, now 128); then, while rows without in-edges still
  * change, every gridDim.x-th of their bins.  Bound by the streamed entries (6
  * bytes each); two blocks a CU, so that one's rows overlap the other's
- * entries.  R-MAT-24: 490 us = 3.6 TB/s (567 us beside a long-row kernel on
+ * entries.  R-MAT-24: 445 us = 4.0 TB/s (567 us beside a long-row kernel on
  * CUs of its own before); R-MAT-22: 117 us, where that kernel's longest row
  * took 158; R-MAT-16, whose wavefront rows bound it: 17 us against 33. */
 template <int MODE>
