@@ -281,11 +281,9 @@ typedef struct og_stage_job
     hipError_t err;
 } og_stage_job;
 
-static int og_stage_ready(void)
+static int og_stage_make(void **p)
 {
-    if (g_stage) return 1;
-    void *p = NULL;
-    if (hipHostMalloc(&p, OG_STAGE_THREADS * OG_STAGE_BYTES, hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc(p, OG_STAGE_THREADS * OG_STAGE_BYTES, hipHostMallocDefault) != hipSuccess)
     {
         (void)hipGetLastError();
         return 0;
@@ -295,18 +293,31 @@ static int og_stage_ready(void)
         {
             (void)hipGetLastError();
             while (i-- > 0) (void)hipEventDestroy(g_stage_ev[i]);
-            (void)hipHostFree(p);
+            (void)hipHostFree(*p);
             return 0;
         }
-    g_stage = (char *)p;
     return 1;
+}
+
+static int og_stage_ready(void)
+{
+    if (g_stage) return 1;
+    void *p = NULL;
+    int was = g_device;
+    (void)hipGetDevice(&was);
+    if (was != g_device && hipSetDevice(g_device) != hipSuccess) return 0;
+    const int ok = og_stage_make(&p);
+    if (was != g_device) (void)hipSetDevice(was);   /* the caller's choice stays */
+    if (ok) g_stage = (char *)p;
+    return ok;
 }
 
 static void *og_stage_run(void *arg)
 {
     og_stage_job *j = (og_stage_job *)arg;
     char *buf = g_stage + j->self * OG_STAGE_BYTES;
-    j->err = hipSetDevice(g_device);
+    /* (thread 0 is the caller's, whose current device stays) */
+    j->err = j->self ? hipSetDevice(g_device) : hipSuccess;
     for (size_t o = j->self * OG_STAGE_BYTES; o < j->bytes && j->err == hipSuccess; o += j->threads * OG_STAGE_BYTES)
     {
         const size_t k = j->bytes - o < OG_STAGE_BYTES ? j->bytes - o : OG_STAGE_BYTES;
@@ -345,7 +356,13 @@ hipError_t og_download(void *dst, const void *src, size_t bytes)
     for (uint32_t i = 1; i < n; i++)
     {
         if (started[i]) pthread_join(th[i], NULL);
-        else og_stage_run(&job[i]);
+        else
+        {
+            int was = g_device;
+            (void)hipGetDevice(&was);
+            og_stage_run(&job[i]);
+            if (was != g_device) (void)hipSetDevice(was);
+        }
         if (e == hipSuccess) e = job[i].err;
     }
     pthread_mutex_unlock(&g_stage_lock);
