@@ -199,6 +199,8 @@ __global__ __launch_bounds__(DT, 4) void og_dir_kernel(og_dir_dev b, og_pr_dev a
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const og_dir_bin d = b.bins[blockIdx.x];
     const bool piece = d.kind == OG_BIN_PIECE;
+    /* integer modes: a long row alone in its block is added by the whole block */
+    const bool alone = MODE != OG_MODE_F32 && d.kind != OG_BIN_THREAD_ROWS && d.row1 - d.row0 == 1;
     uint32_t id[DG];   /* the first DBATCH in-edges' */
     og_dir_ids(a.cols, d.pos0, 0, d.cnt, id);
     /* this thread's row (lane l of wavefront w: the wavefront's l-th) */
@@ -282,6 +284,28 @@ __global__ __launch_bounds__(DT, 4) void og_dir_kernel(og_dir_dev b, og_pr_dev a
                 if (mine)
                     r = update(v, og_row_by_thread<MODE>(slot, p0, p1, (A)(MODE == OG_MODE_F32 && a.spmv ? r : 0.0f)), r,
                                deg);
+            }
+            else if (alone)
+            {
+                /* every thread its share, added up at the row's end */
+                if constexpr (MODE != OG_MODE_F32)
+                {
+                    y += og_bin_int_strided<MODE>(slot, threadIdx.x, n, DT);
+                    if (q0 + n >= d.cnt)
+                    {
+                        for (int o = 32; o > 0; o >>= 1) y += __shfl_xor(y, o, 64);
+                        __syncthreads();   /* slot is read */
+                        if (lane == 0) ((A *)slot)[wave] = y;
+                        __syncthreads();
+                        if (threadIdx.x == 0)
+                        {
+                            y = 0;
+                            for (uint32_t w = 0; w < DW; w++) y += ((const A *)slot)[w];
+                            rp = r;
+                            r = update(v, y, r, deg);
+                        }
+                    }
+                }
             }
             else
             {
