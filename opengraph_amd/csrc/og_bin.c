@@ -431,7 +431,7 @@ static uint32_t og_bin_item_src(const uint32_t *seg_quads, uint32_t n_seg, uint3
     return (uint32_t)size;
 }
 
-int og_bin_plan_build(const og_plan *pl, int mode, og_bin_plan **out)
+int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, og_bin_plan **out)
 {
     *out = NULL;
     const uint32_t N = pl->N, E = pl->E, Z = pl->Z, H = pl->H;
@@ -459,6 +459,13 @@ int og_bin_plan_build(const og_plan *pl, int mode, og_bin_plan **out)
         goto done;
     }
     if (og_bin_list_runs(pl, &runs)) goto done;
+    if (og_bin_longest((const og_bin_run *)runs.p, runs.n) > max_row)
+    {
+        og_bin_plan_destroy(b);
+        b = NULL;
+        rc = 0;
+        goto done;
+    }
     {
         const uint32_t n_seg = (N + OG_BIN_SEG - 1) / OG_BIN_SEG;
         const uint32_t cus = og_num_cus() > 0 ? (uint32_t)og_num_cus() : 1;

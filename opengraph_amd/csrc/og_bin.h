@@ -124,10 +124,18 @@ typedef struct
 } og_bin_run;
 /* The runs of a plan's rows [0, Z), ascending (malloc'ed). */
 int og_bin_runs(const og_plan *pl, og_bin_run **runs, size_t *n);
+/* The longest row of the runs. */
+static inline uint32_t og_bin_longest(const og_bin_run *run, size_t n)
+{
+    uint32_t most = 0;
+    for (size_t i = 0; i < n; i++) most = run[i].deg > most ? run[i].deg : most;
+    return most;
+}
 
 /* Builds the binned layout of a plan whose rows keep the reference's
- * in-neighbour order (relabel 2 or 0). */
-int og_bin_plan_build(const og_plan *pl, int mode, og_bin_plan **out);
+ * in-neighbour order (relabel 2 or 0).  Not built (*out stays NULL, 0 is
+ * returned) where a row has more than max_row in-edges. */
+int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, og_bin_plan **out);
 void og_bin_plan_destroy(og_bin_plan *b);
 
 /* Arithmetic the binned and direct pulls run in: 32-bit gathered elements,

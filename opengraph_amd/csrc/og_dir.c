@@ -70,7 +70,7 @@ static uint32_t og_dir_pack(const og_bin_run *run, size_t n_runs, uint32_t Z, ui
     return n;
 }
 
-int og_dir_plan_build(const og_plan *pl, int mode, uint32_t max_edges, og_dir_plan **out)
+int og_dir_plan_build(const og_plan *pl, int mode, uint32_t max_edges, uint32_t max_row, og_dir_plan **out)
 {
     *out = NULL;
     const uint32_t E = pl->E, N = pl->N, Z = pl->Z;
@@ -90,7 +90,8 @@ int og_dir_plan_build(const og_plan *pl, int mode, uint32_t max_edges, og_dir_pl
     }
     if (og_bin_runs(pl, &run, &n_runs)) goto done;
     uint32_t n = most + 1;
-    for (uint64_t cap = OG_DIR_EDGES; n > most && cap <= OG_DIR_CAP; cap += cap / 4)
+    const int fits = og_bin_longest(run, n_runs) <= max_row;
+    for (uint64_t cap = OG_DIR_EDGES; fits && n > most && cap <= OG_DIR_CAP; cap += cap / 4)
         if ((uint64_t)E <= cap * most) n = og_dir_pack(run, n_runs, Z, (uint32_t)cap, mode == OG_MODE_F32 ? OG_DIR_WAVE_ROW : OG_DIR_WAVE_ROW_INT,
                             bins, most);
     if (n > most)

@@ -68,9 +68,10 @@ typedef struct og_dir_plan
     void *mem_bins, *mem_bar;
 } og_dir_plan;
 
-/* The bins of a plan in CSR order for at most max_edges in-edges; *out stays
- * NULL (and 0 is returned) where the graph does not fit. */
-int og_dir_plan_build(const og_plan *pl, int mode, uint32_t max_edges, og_dir_plan **out);
+/* The bins of a plan in CSR order for at most max_edges in-edges, max_row of
+ * them in a row; *out stays NULL (and 0 is returned) where the graph does not
+ * fit. */
+int og_dir_plan_build(const og_plan *pl, int mode, uint32_t max_edges, uint32_t max_row, og_dir_plan **out);
 void og_dir_plan_destroy(og_dir_plan *b);
 /* Blocks of the kernel the device holds at once. */
 uint32_t og_dir_resident(void);

@@ -30,6 +30,18 @@
  * (R-MAT-18, 4.2 M edges: 34 us an iteration direct, 42 binned; R-MAT-17 25 and
  * 33; uniform, 2 M: 18 and 23) */
 #define OG_DIR_MAX_EDGES (1u << 23)
+/* A streamed row is added by one block, 0.3 to 0.55 ns a term whatever its
+ * length; the integer variants' own pulls cut a long row into chunks for the
+ * whole device.  Longest row an integer pull streams: OG_ROW_ALWAYS terms, or
+ * this fraction of all of them.  us an iteration of the u64 / u32 pull by their
+ * own kernels and streamed, uniform sources: 1 M edges, a row of 33 k 37 / 25 and
+ * 28 / 23, of 66 k 37 / 25 and 43 / 35, of 210 k 37 / 25 and 118 / 91; 4 M edges, a row of
+ * 1/64th of them 69 / 61 and 54 / 47, of 1/32nd 68 / 60 and 80 / 66; 64 M edges, 1/64th
+ * 1185 / 1028 and 584 / 476, 1/16th 1137 / 998 and 1880 / 1403.  (The SpMV of
+ * the 33 k row loses, 18 and 21 us.  The u64 push adds a destination serially
+ * too and is slower at every length.) */
+#define OG_ROW_ALWAYS 24576u
+#define OG_ROW_FRACTION 64u
 /* Rows with more in-edges than this go to the chunk waves: 12..16 is the
  * fastest on R-MAT 24 (1.38-1.40 ms against 1.47 at 32 and 1.50 at 4) and
  * on Erdos-Renyi 24 (4.80-4.87 ms against 5.08 at 32). */
@@ -392,13 +404,16 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
         ogpu_pr_free(p);
         return -1;
     }
+    const uint32_t max_row = p->mode == OG_MODE_F32 || p->push ? 0xFFFFFFFFu
+                           : E / OG_ROW_FRACTION > OG_ROW_ALWAYS ? E / OG_ROW_FRACTION : OG_ROW_ALWAYS;
     /* a small graph's pull runs direct unless the binned one is asked for */
-    if (binned && opt->binned != 1 && !p->quant && og_dir_plan_build(p->plan, p->mode, OG_DIR_MAX_EDGES, &p->dir))
+    if (binned && opt->binned != 1 && !p->quant &&
+        og_dir_plan_build(p->plan, p->mode, OG_DIR_MAX_EDGES, max_row, &p->dir))
     {
         ogpu_pr_free(p);
         return -1;
     }
-    if (binned && !p->dir && og_bin_plan_build(p->plan, p->mode, &p->bins))
+    if (binned && !p->dir && og_bin_plan_build(p->plan, p->mode, max_row, &p->bins))
     {
         if (opt->binned == 1)
         {
@@ -411,7 +426,8 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     const int streamed = p->bins || p->dir;
     if (binned && !streamed && opt->variant != 0 && p->own_plan)
     {
-        /* no layout for this graph: the variant's own kernels and their plan */
+        /* no layout for this graph, or a slower one: the variant's own kernels
+         * and their plan */
         og_plan_destroy(p->plan);
         p->plan = NULL;
         if (og_plan_build(g, p->opt.relabel, p->opt.hub_threshold,

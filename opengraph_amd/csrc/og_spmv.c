@@ -252,7 +252,8 @@ double ogpu_spmv_bytes_per_iteration(const ogpu_spmv *s)
     case 1: return s->p->pp_v0 ? 10.0 * E + 8.0 * N : 16.0 * E + 4.0 * N;
     case 2: return 8.0 * E + 20.0 * N;   /* index + u32 term per edge; row_ptr, u64 y read + write */
     case 3:
-        return !s->scatter ? 12.0 * E + 20.0 * N   /* index + u64 term per edge */
+        return s->narrow ? 8.0 * E + 20.0 * N
+               : !s->scatter ? 12.0 * E + 20.0 * N   /* index + u64 term per edge */
                : s->p->pp_v0 ? 14.0 * E + 16.0 * N
                              : 24.0 * E + 8.0 * N;
     default: return 8.0 * E + 12.0 * N;  /* index + fp32 term per edge; row_ptr, y read + write */

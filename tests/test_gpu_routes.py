@@ -1,6 +1,8 @@
 """Rows and graphs at the lines where the integer variants and SpMV codes
 change between the direct, the binned and their own kernels: whole numbers, so
 every route is equal to the oracle to the bit."""
+import time
+
 import numpy as np
 import pytest
 
@@ -53,3 +55,70 @@ def _check(s, d, codes=(2, 3, 4, 9), spmv=(2, 3), relabel=1, iters=4):
     [CAP - 1, CAP, CAP + 1, CAP // 2], [CAP + 511, 1, 1], [2 * CAP, 2 * CAP + 1, 300] + [3] * 2000])
 def test_long_integer_rows_of_the_direct_pull(degrees):
     _check(*_rows(degrees, 30_011, sum(degrees)))
+
+
+def _best(f, n=7):
+    t = []
+    for _ in range(n):
+        a = time.perf_counter()
+        f()
+        t.append(time.perf_counter() - a)
+    return min(t)
+
+
+def _not_the_slower_form(s, d, codes, spmv, most=1.4):
+    """A default run takes at most `most` times what the variant's own kernels
+    take (binned = 2; SpMV: a hub_threshold); best of seven runs each, 20
+    iterations."""
+    g = og.Graph.from_edges(s, d, 0)
+    for code in codes:
+        t = []
+        for kw in (dict(), dict(binned=2)):
+            pr = og.PageRank(g, code, 20, 0.0, **kw)
+            pr.run()
+            t.append(_best(pr.run))
+            pr.free()
+        assert t[0] <= most * t[1], ("pagerank", code, t)
+    for code in spmv:
+        t = []
+        for kw in (dict(), dict(hub_threshold=16)):
+            sp = og.Spmv(g, code, **kw)
+            sp.run(20)
+            t.append(_best(lambda: sp.run(20)))
+            sp.free()
+        assert t[0] <= most * t[1], ("spmv", code, t)
+    g.free()
+
+
+def _hub(n, edges, hub, seed=3):
+    """A uniform graph, `hub` of whose in-edges are one vertex's."""
+    rng = np.random.default_rng(seed)
+    s, d = (rng.integers(0, n, edges).astype(np.uint32) for _ in range(2))
+    s[0] = n - 1
+    d[:] = np.where(d == 7, 8, d)
+    d[rng.permutation(edges)[:hub]] = 7
+    return s, d
+
+
+ROW = 24576      # an integer row that is always streamed; longer: a 64th of the in-edges
+
+
+@pytest.mark.parametrize("edges,hub", [(300_000, ROW - 1), (300_000, ROW), (300_000, ROW + 1),
+                                       (64 * ROW + 64, ROW + 1), (64 * ROW + 64, ROW + 2)])
+def test_integer_rows_at_the_longest_streamed(edges, hub):
+    s, d = _hub(20_000, edges, hub)
+    assert np.bincount(d).max() == hub
+    _check(s, d)
+    g = og.Graph.from_edges(s, d, 0)
+    pr = og.PageRank(g, 2, 2, 0.0)      # its bytes per iteration tell its passes
+    streamed = hub <= max(ROW, edges // 64)
+    n = g.num_vertices
+    assert pr.bytes_per_iteration() == (8 * edges + 20 * n if streamed else 12 * edges + 24 * n)
+    pr.free()
+    g.free()
+
+
+@pytest.mark.parametrize("n,edges,hub", [(1 << 20, 1 << 22, 1 << 21), (100_000, 1 << 20, 200_000),
+                                         (1 << 18, 1 << 22, 1 << 18)])
+def test_long_integer_rows_are_not_one_blocks_work(n, edges, hub):
+    _not_the_slower_form(*_hub(n, edges, hub), codes=(2, 4, 9), spmv=(2, 3))
