@@ -42,6 +42,13 @@
  * too and is slower at every length.) */
 #define OG_ROW_ALWAYS 24576u
 #define OG_ROW_FRACTION 64u
+/* Average in-degree past which an integer pull that does not run direct keeps
+ * its own kernel: its few contributions then all lie in the LDS copy, and 4
+ * bytes an edge beat the passes' 14 (u64 and u32 pull, own kernels and streamed:
+ * 20 k vertices, 64 M edges 173 / 134 and 205 / 194 us an iteration; 10 k, 64 M 125 / 113
+ * and 236 / 191; 2 k, 9 M 42 / 38 and 65 / 48; 10 k, 16 M 73 / 67 and 71 / 65; 40 k,
+ * 64 M 276 / 206 and 199 / 190). */
+#define OG_DENSE_DEGREE 2048u
 /* Rows with more in-edges than this go to the chunk waves: 12..16 is the
  * fastest on R-MAT 24 (1.38-1.40 ms against 1.47 at 32 and 1.50 at 4) and
  * on Erdos-Renyi 24 (4.80-4.87 ms against 5.08 at 32). */
@@ -413,7 +420,8 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
         ogpu_pr_free(p);
         return -1;
     }
-    if (binned && !p->dir && og_bin_plan_build(p->plan, p->mode, max_row, &p->bins))
+    const int dense = p->mode != OG_MODE_F32 && !p->push && E / OG_DENSE_DEGREE > N;
+    if (binned && !p->dir && !dense && og_bin_plan_build(p->plan, p->mode, max_row, &p->bins))
     {
         if (opt->binned == 1)
         {

@@ -122,3 +122,19 @@ def test_integer_rows_at_the_longest_streamed(edges, hub):
                                          (1 << 18, 1 << 22, 1 << 18)])
 def test_long_integer_rows_are_not_one_blocks_work(n, edges, hub):
     _not_the_slower_form(*_hub(n, edges, hub), codes=(2, 4, 9), spmv=(2, 3))
+
+
+@pytest.mark.parametrize("n,edges", [(4098, 4098 * 2048 + 2047), (4097, 4098 * 2048)])
+def test_integer_pulls_of_few_vertices(n, edges):
+    """Past 8 M edges (no direct pull) at and past 2048 in-edges a vertex."""
+    rng = np.random.default_rng(n)
+    s, d = (rng.integers(0, n, edges).astype(np.uint32) for _ in range(2))
+    s[0] = n - 1
+    _check(s, d, iters=3)
+    g = og.Graph.from_edges(s, d, 0)
+    pr = og.PageRank(g, 2, 2, 0.0)
+    assert pr.bytes_per_iteration() == (8 * edges + 20 * n if edges // 2048 <= n else 12 * edges + 24 * n)
+    pr.free()
+    g.free()
+    if n == 4097:
+        _not_the_slower_form(s, d, codes=(2, 4, 9), spmv=(2, 3), most=1.2)
