@@ -49,6 +49,12 @@
  * and 236 / 191; 2 k, 9 M 42 / 38 and 65 / 48; 10 k, 16 M 73 / 67 and 71 / 65; 40 k,
  * 64 M 276 / 206 and 199 / 190). */
 #define OG_DENSE_DEGREE 2048u
+/* In-edges from which the quantized pull streams (it has no direct form, whose
+ * one launch is what makes the others faster on small graphs): own kernels and
+ * streamed, us an iteration, R-MAT-14, 262 k edges 26 and 30; R-MAT-16, 1 M 28 and 33;
+ * R-MAT-17, 2 M 37 and 37; R-MAT-18, 3 M 54 and 37, 4 M 61 and 42; uniform, 1 M vertices,
+ * 2 M 48 and 44. */
+#define OG_QUANT_MIN_EDGES (1u << 21)
 /* Rows with more in-edges than this go to the chunk waves: 12..16 is the
  * fastest on R-MAT 24 (1.38-1.40 ms against 1.47 at 32 and 1.50 at 4) and
  * on Erdos-Renyi 24 (4.80-4.87 ms against 5.08 at 32). */
@@ -361,7 +367,8 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     if (!binned && (opt->variant == 1 || opt->variant == 2 || opt->variant == 3 || opt->variant == 4 ||
                     opt->variant == 9) &&
         opt->binned == 0 && !opt->hub_threshold && !opt->hot_cache && g->E > 0 &&
-        !(opt->variant == 1 && !opt->exact_above) && !(plan && plan->relabel == 1 && plan->H))
+        !(opt->variant == 1 && !opt->exact_above) && !(p->quant && E < OG_QUANT_MIN_EDGES) &&
+        !(plan && plan->relabel == 1 && plan->H))
         binned = 1;
     if (opt->binned == 1 && !binned)
     {

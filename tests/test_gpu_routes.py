@@ -57,7 +57,7 @@ def test_long_integer_rows_of_the_direct_pull(degrees):
     _check(*_rows(degrees, 30_011, sum(degrees)))
 
 
-def _best(f, n=7):
+def _best(f, n=15):
     t = []
     for _ in range(n):
         a = time.perf_counter()
@@ -68,7 +68,7 @@ def _best(f, n=7):
 
 def _not_the_slower_form(s, d, codes, spmv, most=1.4):
     """A default run takes at most `most` times what the variant's own kernels
-    take (binned = 2; SpMV: a hub_threshold); best of seven runs each, 20
+    take (binned = 2; SpMV: a hub_threshold); best of fifteen runs each, 20
     iterations."""
     g = og.Graph.from_edges(s, d, 0)
     for code in codes:
@@ -138,3 +138,13 @@ def test_integer_pulls_of_few_vertices(n, edges):
     g.free()
     if n == 4097:
         _not_the_slower_form(s, d, codes=(2, 4, 9), spmv=(2, 3), most=1.2)
+
+
+@pytest.mark.parametrize("edges", [(1 << 21) - 1, 1 << 21])
+def test_quantized_pull_at_its_first_streamed_size(edges):
+    _check(*og.rmat_host(17, edges, seed=8), codes=(4,), spmv=())
+
+
+@pytest.mark.parametrize("scale", [4, 12, 14, 16])
+def test_small_quantized_pull_is_not_the_slower_form(scale):
+    _not_the_slower_form(*og.rmat_host(scale, 16 << scale, seed=9), codes=(4,), spmv=(), most=1.1)
