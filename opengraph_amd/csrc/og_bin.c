@@ -431,7 +431,7 @@ static uint32_t og_bin_item_src(const uint32_t *seg_quads, uint32_t n_seg, uint3
     return (uint32_t)size;
 }
 
-int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, og_bin_plan **out)
+int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, uint64_t max_entries, og_bin_plan **out)
 {
     *out = NULL;
     const uint32_t N = pl->N, E = pl->E, Z = pl->Z, H = pl->H;
@@ -452,7 +452,7 @@ int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, og_bin_plan
     uint32_t *d_quads = NULL, *d_bin_quads = NULL, *d_seg = NULL;
     void *scratch = NULL;
     hipStream_t s = og_stream();
-    int rc = -1;
+    int rc = -1, unfit = 0;
     if (!b)
     {
         og_set_error("out of host memory");
@@ -461,8 +461,7 @@ int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, og_bin_plan
     if (og_bin_list_runs(pl, &runs)) goto done;
     if (og_bin_longest((const og_bin_run *)runs.p, runs.n) > max_row)
     {
-        og_bin_plan_destroy(b);
-        b = NULL;
+        unfit = 1;
         rc = 0;
         goto done;
     }
@@ -532,6 +531,12 @@ int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, og_bin_plan
             og_set_error("binned pull: graph too large for 32-bit entries");
             goto done;
         }
+        if (ent > max_entries)
+        {
+            unfit = 1;
+            rc = 0;
+            goto done;
+        }
         b->n_ent = ent + OG_BIN_SPARE;   /* spare entries past the last tile */
         b->d.n_ent = (uint32_t)ent;
         b->mem_src = og_dalloc(b->n_ent * 2);
@@ -595,7 +600,7 @@ done:
     og_dfree(d_quads); og_dfree(d_bin_quads); og_dfree(d_seg); og_dfree(scratch);
     og_dfree(d_order);
     free(runs.p); free(bins.p); free(items.p); free(order); free(blk); free(seg_src); free(rp);
-    if (rc) og_bin_plan_destroy(b);
+    if (rc || unfit) og_bin_plan_destroy(b);
     else *out = b;
     return rc;
 }

@@ -134,8 +134,9 @@ static inline uint32_t og_bin_longest(const og_bin_run *run, size_t n)
 
 /* Builds the binned layout of a plan whose rows keep the reference's
  * in-neighbour order (relabel 2 or 0).  Not built (*out stays NULL, 0 is
- * returned) where a row has more than max_row in-edges. */
-int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, og_bin_plan **out);
+ * returned) where a row has more than max_row in-edges or the tiles, padding
+ * included, more than max_entries entries. */
+int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, uint64_t max_entries, og_bin_plan **out);
 void og_bin_plan_destroy(og_bin_plan *b);
 
 /* Arithmetic the binned and direct pulls run in: 32-bit gathered elements,

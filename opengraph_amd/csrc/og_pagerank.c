@@ -49,6 +49,13 @@
  * and 236 / 191; 2 k, 9 M 42 / 38 and 65 / 48; 10 k, 16 M 73 / 67 and 71 / 65; 40 k,
  * 64 M 276 / 206 and 199 / 190). */
 #define OG_DENSE_DEGREE 2048u
+/* Entries an edge, padding included, up to which a variant with kernels of its
+ * own streams: where segments are many and rows short, few of a bin's edges
+ * share a tile, and every tile is padded to 16.  Own kernels and streamed, us
+ * an iteration of the u32 pull (random edges): 16 M vertices and 34 M edges, 4.9
+ * entries an edge 643 and 602, 25 M edges, 5.4 501 and 501, one in-edge each,
+ * 9.3 366 and 561; 24 M and 60 M, 6.0 1167 and 1282; 34 M and 34 M, 8.7 724 and 1059. */
+#define OG_ENTRIES_PER_EDGE 5.5
 /* In-edges from which the quantized pull streams (it has no direct form, whose
  * one launch is what makes the others faster on small graphs): own kernels and
  * streamed, us an iteration, R-MAT-14, 262 k edges 26 and 30; R-MAT-16, 1 M 28 and 33;
@@ -327,8 +334,12 @@ out:
     return rc;
 }
 
-/* Create a run on graph g.  plan may be supplied (borrowed) or built here. */
 int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, ogpu_pr **out)
+{
+    return og_pr_create_as(g, plan, opt, 0, out);
+}
+
+int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int only_streamed, ogpu_pr **out)
 {
     *out = NULL;
     if (og_ctx_ensure()) return -1;
@@ -428,7 +439,8 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
         return -1;
     }
     const int dense = p->mode != OG_MODE_F32 && !p->push && E / OG_DENSE_DEGREE > N;
-    if (binned && !p->dir && !dense && og_bin_plan_build(p->plan, p->mode, max_row, &p->bins))
+    const uint64_t max_entries = opt->variant ? (uint64_t)(OG_ENTRIES_PER_EDGE * E) : ~0ull;
+    if (binned && !p->dir && !dense && og_bin_plan_build(p->plan, p->mode, max_row, max_entries, &p->bins))
     {
         if (opt->binned == 1)
         {
@@ -439,6 +451,11 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     }
     if (p->bins) p->n_final_bin = og_final_blocks(p->bins->sum_grid, 0);
     const int streamed = p->bins || p->dir;
+    if (only_streamed && !streamed)
+    {
+        ogpu_pr_free(p);
+        return 0;
+    }
     if (binned && !streamed && opt->variant != 0 && p->own_plan)
     {
         /* no layout for this graph, or a slower one: the variant's own kernels

@@ -58,7 +58,8 @@ int ogpu_spmv_create(ogpu_graph *gg, const ogpu_spmv_options *opt_in, ogpu_spmv 
     return og_spmv_create_with((og_graph *)gg, NULL, opt_in, out);
 }
 
-int og_spmv_create_with(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt_in, ogpu_spmv **out)
+/* -p 1 on the streaming passes, or by its partitioned scatter (streamed = 0). */
+static int og_spmv_create_as(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt_in, int streamed, ogpu_spmv **out)
 {
     *out = NULL;
     ogpu_spmv_options o;
@@ -76,15 +77,14 @@ int og_spmv_create_with(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt
      * orders its atomics may land in, and u64 sums of the integer terms, all of
      * which fit 32 bits.  An option that asks for a row split, a hot copy or a
      * scatter selects the kernels it is about. */
-    const int streamed = !o.hub_threshold && !o.hot_cache && !(o.code == 3 && o.scatter) &&
-                         !(plan && plan->relabel == 1 && plan->H);
+    streamed = streamed && !o.hub_threshold && !o.hot_cache && !(o.code == 3 && o.scatter) &&
+               !(plan && plan->relabel == 1 && plan->H);
     s->scatter = (o.code == 1 && !streamed) || (o.code == 3 && o.scatter);
     s->mode = o.code < 2 ? OG_MODE_F32 : o.code == 2 || streamed ? OG_MODE_FX32 : OG_MODE_FX64;
     ogpu_pr_options po;
     ogpu_pr_default_options(&po);
     /* the PageRank variant whose plan, buffers and kernels the passes use */
-    po.variant = o.code == 0 || (o.code == 1 && streamed) ? 0 : o.code == 1 ? 1
-               : o.code == 2 || streamed ? 9 : (s->scatter ? 3 : 2);
+    po.variant = o.code < 2 ? o.code : o.code == 2 || streamed ? 9 : (s->scatter ? 3 : 2);
     po.max_iter = 1;
     po.hub_threshold = o.hub_threshold;
     /* the pushes (-p 1, -p 3 scattered) are partitioned by destination
@@ -95,10 +95,16 @@ int og_spmv_create_with(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt
      * PageRank push would gather its longest rows instead) */
     if (o.code == 1 && !streamed) po.exact_above = 0;
     po.binned = streamed || (o.code == 0 && !o.hub_threshold) ? 0 : 2;
-    if (og_pr_create_with(g, plan, &po, &s->p))
+    if (og_pr_create_as(g, plan, &po, o.code == 1 && streamed, &s->p))
     {
         free(s);
         return -1;
+    }
+    if (!s->p)
+    {
+        /* no layout for this graph, or a slower one */
+        free(s);
+        return og_spmv_create_as(g, plan, opt_in, 0, out);
     }
     s->narrow = o.code == 3 && streamed;
     s->terms = s->p->c[0];
@@ -109,6 +115,11 @@ int og_spmv_create_with(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt
     }
     *out = s;
     return 0;
+}
+
+int og_spmv_create_with(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt_in, ogpu_spmv **out)
+{
+    return og_spmv_create_as(g, plan, opt_in, 1, out);
 }
 
 int ogpu_spmv_reset(ogpu_spmv *s)

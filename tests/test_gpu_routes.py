@@ -148,3 +148,39 @@ def test_quantized_pull_at_its_first_streamed_size(edges):
 @pytest.mark.parametrize("scale", [4, 12, 14, 16])
 def test_small_quantized_pull_is_not_the_slower_form(scale):
     _not_the_slower_form(*og.rmat_host(scale, 16 << scale, seed=9), codes=(4,), spmv=(), most=1.1)
+
+
+def _permutation(n, seed=5):
+    s = np.arange(n, dtype=np.uint32)
+    return s, np.random.default_rng(seed).permutation(n).astype(np.uint32)
+
+
+def test_short_rows_over_many_segments():
+    """One in-edge a vertex from all over 2^24 others: 9 padded entries an edge."""
+    s, d = _permutation(1 << 24)
+    g = og.Graph.from_edges(s, d, 0)
+    pr = og.PageRank(g, 2, 2, 0.0)
+    assert pr.bytes_per_iteration() == 12.0 * len(s) + 24.0 * len(s)   # its own kernels
+    pr.free()
+    sp = og.Spmv(g, 1)
+    assert sp.bytes_per_iteration() == 10.0 * len(s) + 8.0 * len(s)
+    sp.free()
+    g.free()
+    _not_the_slower_form(s, d, codes=(1, 2, 3, 4, 9), spmv=(1, 2, 3), most=1.2)
+
+
+@pytest.mark.parametrize("n", [6_000_000, 9_000_000])   # below and above 5.5 entries an edge
+def test_short_rows_streamed_or_not(n):
+    s, d = _permutation(n)
+    _check(s, d, iters=2)
+    g = og.Graph.from_edges(s, d, 0)
+    pr = og.PageRank(g, 2, 2, 0.0)
+    assert pr.bytes_per_iteration() == ((8.0 + 20.0) * n if n == 6_000_000 else (12.0 + 24.0) * n)
+    pr.free()
+    # every sum has one term: the push is the oracle's pull to the bit
+    ref = po.pagerank(po.build_csr(s, d, 0, 8), 0, 0.0, 3, 8)["ranks"]
+    pr = og.PageRank(g, 1, 3, 0.0)
+    pr.run()
+    assert np.array_equal(pr.ranks().view(np.uint32), ref.view(np.uint32))
+    pr.free()
+    g.free()
