@@ -439,8 +439,14 @@ int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int 
         return -1;
     }
     const int dense = p->mode != OG_MODE_F32 && !p->push && E / OG_DENSE_DEGREE > N;
+    /* SpMV -p 1 (only_streamed): its scatter over rows of about one in-edge is
+     * one short launch (us a pass, scattered and binned: 1 M vertices on a ring 15
+     * and 23, 4 M 47 and 66, a random tree of 8 M 105 and 122; 1.6 in-edges a row, 1 M
+     * 19 and 16, 4 M 79 and 58; many more vertices than in-edges, whose y the scatter goes
+     * through, 50 and 32) */
+    const int ones = only_streamed && 2ull * E < 3ull * p->plan->Z && 2ull * E >= N;
     const uint64_t max_entries = opt->variant ? (uint64_t)(OG_ENTRIES_PER_EDGE * E) : ~0ull;
-    if (binned && !p->dir && !dense && og_bin_plan_build(p->plan, p->mode, max_row, max_entries, &p->bins))
+    if (binned && !p->dir && !dense && !ones && og_bin_plan_build(p->plan, p->mode, max_row, max_entries, &p->bins))
     {
         if (opt->binned == 1)
         {

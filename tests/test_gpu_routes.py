@@ -184,3 +184,20 @@ def test_short_rows_streamed_or_not(n):
     assert np.array_equal(pr.ranks().view(np.uint32), ref.view(np.uint32))
     pr.free()
     g.free()
+
+
+@pytest.mark.parametrize("kind", ["ring", "tree"])
+def test_spmv_push_over_rows_of_one_in_edge(kind):
+    n = 1 << 20
+    v = np.arange(1, n, dtype=np.uint32)
+    u = v - 1 if kind == "ring" else (np.random.default_rng(2).random(n - 1) * v).astype(np.uint32)
+    s, d = u.astype(np.uint32), v
+    g = og.Graph.from_edges(s, d, 0)
+    sp = og.Spmv(g, 1)
+    assert sp.bytes_per_iteration() == 10.0 * len(s) + 8.0 * n    # the partitioned scatter
+    sp.run(3)
+    want = po.spmv(po.build_csr(s, d, 0, 8), 0, 3)
+    assert np.array_equal(sp.output().view(np.uint32), want.view(np.uint32))   # one term a row
+    sp.free()
+    g.free()
+    _not_the_slower_form(s, d, codes=(), spmv=(1,), most=1.15)
