@@ -351,6 +351,17 @@ static uint32_t og_bin_cap(uint32_t E, uint32_t n_seg, uint32_t slots)
     return c > OG_BIN_CAP ? OG_BIN_CAP : (uint32_t)c;
 }
 
+/* fp32: rows of more in-edges are added by a wavefront: OG_BIN_WAVE_ROW, or a
+ * sixth of a bin where a small graph's bins are so small that a few such rows
+ * fill one, and the threads' long chains of adds would leave the rest of the
+ * block idle (10 k vertices, 16 M edges, bins of 8192, 1680 terms a row: SpMV 97 us a
+ * pass by threads, 62 by wavefronts; pull 103 and 78 us an iteration.  An eighth: 20 k
+ * vertices with 840 terms a row the same, R-MAT-18 with 10 M edges 3 % slower.) */
+static uint32_t og_bin_wave_row(uint32_t cap)
+{
+    return cap / 6 < OG_BIN_WAVE_ROW ? cap / 6 : OG_BIN_WAVE_ROW;
+}
+
 /* The sum pass's order: the bins dealt in their order (the long rows, the
  * longest ones, come first) to the block with the least so far, a long row's
  * pieces to one block.  order: the bins block by block; blk: where each
@@ -468,8 +479,8 @@ int og_bin_plan_build(const og_plan *pl, int mode, uint32_t max_row, uint64_t ma
     {
         const uint32_t n_seg = (N + OG_BIN_SEG - 1) / OG_BIN_SEG;
         const uint32_t cus = og_num_cus() > 0 ? (uint32_t)og_num_cus() : 1;
-        if (og_bin_pack(pl, &runs, og_bin_cap(E, n_seg, 2 * cus),
-                        mode == OG_MODE_F32 ? OG_BIN_WAVE_ROW : OG_BIN_CAP, &bins))
+        const uint32_t cap = og_bin_cap(E, n_seg, 2 * cus);
+        if (og_bin_pack(pl, &runs, cap, mode == OG_MODE_F32 ? og_bin_wave_row(cap) : OG_BIN_CAP, &bins))
         {
             og_set_error("out of host memory");
             goto done;

@@ -59,7 +59,7 @@ extern "C" {
 #define OG_BIN_CAP 19968u      /* in-edge values per bin: 78 KB of LDS, two bins per CU */
 #define OG_BIN_PAD 0xFFFFu     /* pos of a padding entry */
 /* rows with more in-edges are added by a wavefront (1024: 3 % slower at
- * R-MAT-24, the same at 20-22); the integer modes' bins take any number of
+ * R-MAT-24, the same at 20-22; fewer in small bins); the integer modes' bins take any number of
  * lanes per row instead */
 #define OG_BIN_WAVE_ROW 2048u
 #define OG_BIN_RPT 1u          /* rows per thread and bin: a bin holds at most RPT * THREADS rows */

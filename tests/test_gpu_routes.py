@@ -201,3 +201,36 @@ def test_spmv_push_over_rows_of_one_in_edge(kind):
     sp.free()
     g.free()
     _not_the_slower_form(s, d, codes=(), spmv=(1,), most=1.15)
+
+
+@pytest.mark.parametrize("relabel", [0, 1])
+@pytest.mark.parametrize("n,row", [(30_011, 4096 // 6), (8_000_000, 2048)])   # bins of 4096, and of more than 12288
+def test_wavefront_rows_of_the_binned_pull(n, row, relabel):
+    """Rows at the most in-edges that one thread adds, and at the steps of a wavefront's sum."""
+    deg = [row - 1, row, row + 1, row + 2, 64 + 64 * 36, 64 + 64 * 36 + 1, 64 + 64 * 12, 64 + 64 * 12 + 1, 3] + [1] * 700
+    s, d = _rows(deg, n, row)
+    o = po.build_csr(s, d, 0, 8)
+    ref = po.pagerank(o, 0, 0.0, 4, 8)["ranks"]
+    g = og.Graph.from_edges(s, d, 0)
+    pr = og.PageRank(g, 0, 4, 0.0, relabel=relabel, binned=1)
+    pr.run()
+    assert np.array_equal(pr.ranks().view(np.uint32), ref.view(np.uint32))
+    pr.free()
+    g.free()
+
+
+def test_long_rows_in_small_bins_are_not_a_threads():
+    """10 k rows of 900 terms, in bins of 4608: the SpMV's pass takes about what
+    its bytes take (half as long again when threads added them)."""
+    rng = np.random.default_rng(4)
+    n, e = 10_000, 9 << 20
+    s, d = (rng.integers(0, n, e).astype(np.uint32) for _ in range(2))
+    g = og.Graph.from_edges(s, d, 0)
+    t = []
+    for code in (0, 2):      # fp32 in order, and u64 sums over the same layout
+        sp = og.Spmv(g, code)
+        sp.run(20)
+        t.append(_best(lambda: sp.run(20)))
+        sp.free()
+    assert t[0] <= 1.3 * t[1], t
+    g.free()
