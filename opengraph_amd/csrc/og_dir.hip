@@ -48,6 +48,7 @@ template <typename T> __device__ __forceinline__ void og_dir_post(T *p, T x)
  * 512 blocks 60 us long; all blocks polling all flags took 8 us more than this
  * at 512.) */
 #define DGRP 32u
+#define DFAIL_EVERY 64u   /* polls between looks at FAIL (a look at each would lengthen every wait) */
 __device__ __forceinline__ bool og_dir_poll(const og_dir_dev &b, uint32_t word, uint32_t n, uint32_t it)
 {
     bool ok = true;
@@ -58,10 +59,12 @@ __device__ __forceinline__ bool og_dir_poll(const og_dir_dev &b, uint32_t word, 
         {
             __builtin_amdgcn_s_sleep(1);
             k++;
+            if (k % DFAIL_EVERY == DFAIL_EVERY / 2 && og_dir_peek(&b.bar[OG_DIR_FAIL])) k = b.spin;
         }
         ok = k < b.spin;
     }
-    /* the others are told to leave through FAIL, and the host */
+    /* those still waiting, and those that get a CU only now, leave too within
+     * DFAIL_EVERY polls; the host starts again */
     if (!ok) og_dir_post(&b.bar[OG_DIR_FAIL], 1u);
     return __syncthreads_and(ok);
 }
@@ -80,7 +83,8 @@ __device__ __forceinline__ void og_dir_done(const og_dir_dev &b, const og_pr_dev
     if (threadIdx.x == 0) og_dir_post(&b.bar[blockIdx.x], it + 1);
 }
 
-/* False: some block did not get here within b.spin polls; every block leaves. */
+/* False: some block did not get here within another's b.spin polls; every block
+ * leaves. */
 __device__ __forceinline__ bool og_dir_wait(const og_dir_dev &b, uint32_t it)
 {
     const uint32_t nb = gridDim.x;

@@ -26,6 +26,9 @@
 #define OG_CHECK_EVERY 8u
 /* iterations of one launch of the direct pull, which stops by itself */
 #define OG_DIR_CHECK_EVERY 256u
+/* runs that go one iteration a launch after the direct pull's blocks could not
+ * all be resident; then it is tried again */
+#define OG_DIR_SINGLE_RUNS 32u
 /* past this many in-edges the binned pull's streaming passes are as fast
  * (R-MAT-18, 4.2 M edges: 34 us an iteration direct, 42 binned; R-MAT-17 25 and
  * 33; uniform, 2 M: 18 and 23) */
@@ -981,7 +984,7 @@ static int64_t og_pr_solve(ogpu_pr *p)
             {
                 /* its blocks could not all be resident: from the start, one
                  * iteration a launch */
-                p->dir_single = 1;
+                p->dir_single = OG_DIR_SINGLE_RUNS;
                 if (og_pr_init_state(p)) return -1;
                 launched = 0;
                 continue;
@@ -1030,11 +1033,12 @@ int ogpu_pr_run(ogpu_pr *p, ogpu_pr_result *res)
     memset(res, 0, sizeof(*res));
     res->seconds_plan = p->seconds_plan;
     if (p->dd) return og_dd_run(p, res);
+    if (p->dir_single) p->dir_single--;
     if (p->report && !p->print_rows && !p->dir_single)
     {
         const int rc = og_pr_run_direct(p, res);
         if (rc <= 0) return rc;
-        p->dir_single = 1;
+        p->dir_single = OG_DIR_SINGLE_RUNS;
     }
     double t0 = og_now();
     int64_t launched = og_pr_solve(p);

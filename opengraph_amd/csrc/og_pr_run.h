@@ -65,7 +65,7 @@ struct ogpu_pr
     /* direct fp32 pull (og_dir.h): the iterations of a small graph in one
      * launch */
     struct og_dir_plan *dir;
-    int dir_single;           /* one iteration a launch */
+    uint32_t dir_single;      /* runs left to go one iteration a launch */
     og_pr_report *report;     /* host memory a whole run's results land in */
     /* partitioned push (og_push_part_kernel): destination ranges (device
      * n_pp + 1 row bounds), each inverse-CSR edge's offset in its range,

@@ -75,6 +75,23 @@ def test_blocks_that_do_not_wait(monkeypatch):
     _same(src, dst, 1e-5, 60)
 
 
+@pytest.mark.parametrize("spin", [1, 33, 64, 200])
+@pytest.mark.parametrize("iters", [60, 300])   # one launch, and launches of 256 iterations
+def test_blocks_that_give_up(monkeypatch, spin, iters):
+    """With a few polls some blocks give up at some barrier and the others leave
+    with them; the same bits, and so in later runs, which try again."""
+    monkeypatch.setenv("OG_DIR_SPIN", str(spin))
+    src, dst = og.rmat_host(15, 16 << 15, seed=5)
+    ref = po.pagerank(po.build_csr(src, dst, 0, 4), 0, 0.0, iters, 4)["ranks"].view(np.uint32)
+    g = og.Graph.from_edges(src, dst, 0)
+    pr = og.PageRank(g, 0, iters, 0.0)
+    for _ in range(70):
+        pr.run()
+        assert np.array_equal(pr.ranks().view(np.uint32), ref)
+    pr.free()
+    g.free()
+
+
 def test_enqueued_iterations_equal_a_run():
     src, dst = og.rmat_host(13, 16 << 13, seed=6)
     g = og.Graph.from_edges(src, dst, 0)
