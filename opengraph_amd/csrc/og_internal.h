@@ -35,6 +35,7 @@ hipEvent_t og_side_fork(void);
 hipEvent_t og_side_join(void);
 int og_num_cus(void);
 void og_trace_entry(const char *fn, uint32_t n_vertices, uint32_t n_edges);
+void og_trace_plan(const char *kind);
 /* Device memory from the library's pool (og_runtime.c), of any content;
  * og_dalloc returns NULL with the error set on failure. */
 void *og_dalloc(size_t bytes);

@@ -447,7 +447,7 @@ int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int 
      * and 23, 4 M 47 and 66, a random tree of 8 M 105 and 122; 1.6 in-edges a row, 1 M
      * 19 and 16, 4 M 79 and 58; many more vertices than in-edges, whose y the scatter goes
      * through, 50 and 32) */
-    const int ones = only_streamed && 2ull * E < 3ull * p->plan->Z && 2ull * E >= N;
+    const int ones = only_streamed && opt->variant == 1 && 2ull * E < 3ull * p->plan->Z && 2ull * E >= N;
     const uint64_t max_entries = opt->variant ? (uint64_t)(OG_ENTRIES_PER_EDGE * E) : ~0ull;
     if (binned && !p->dir && !dense && !ones && og_bin_plan_build(p->plan, p->mode, max_row, max_entries, &p->bins))
     {
@@ -1270,13 +1270,15 @@ static int og_dd_run(ogpu_pr *p, ogpu_pr_result *res)
 /* ===================================================================== */
 
 /* One cached device copy of the caller's GraphCSR (keyed by the struct and
- * array pointers, sizes and the sort mode) and its plan. */
+ * array pointers, sizes and the sort mode) and its plans, each built when a
+ * call first needs it. */
 static struct
 {
     const void *key[12];
     uint32_t N, E;
     og_graph *g;
-    og_plan *plan;
+    og_plan *plan;       /* for the gather pulls and pushes: long rows sorted by source */
+    og_plan *csr_plan;   /* for the direct and binned passes: rows in CSR order */
 } g_cache;
 
 static void og_fatal(const char *where)
@@ -1285,7 +1287,7 @@ static void og_fatal(const char *where)
     exit(EXIT_FAILURE);
 }
 
-int og_cache_graph(struct GraphCSR *graph, int need_forward, og_graph **g, og_plan **plan)
+int og_cache_graph(struct GraphCSR *graph, og_graph **g)
 {
     const void *key[12] = {graph,
                            graph->vertices ? graph->vertices->out_degree : NULL,
@@ -1302,17 +1304,11 @@ int og_cache_graph(struct GraphCSR *graph, int need_forward, og_graph **g, og_pl
     if (g_cache.g && memcmp(g_cache.key, key, sizeof(key)) == 0 && g_cache.N == graph->num_vertices &&
         g_cache.E == graph->num_edges)
     {
-        if (need_forward && !g_cache.plan->push_src)
-        {
-            og_plan_destroy(g_cache.plan);
-            g_cache.plan = NULL;
-            if (og_plan_build(g_cache.g, 1, OG_DEFAULT_SEQ_T, OG_DEFAULT_EXACT_ABOVE, 1, &g_cache.plan)) return -1;
-        }
         *g = g_cache.g;
-        *plan = g_cache.plan;
         return 0;
     }
     og_plan_destroy(g_cache.plan);
+    og_plan_destroy(g_cache.csr_plan);
     og_graph_destroy(g_cache.g);
     memset(&g_cache, 0, sizeof(g_cache));
     if (!graph->vertices || !graph->inverse_vertices || !graph->sorted_edges_array ||
@@ -1329,19 +1325,38 @@ int og_cache_graph(struct GraphCSR *graph, int need_forward, og_graph **g, og_pl
         graph->inverse_vertices->in_degree, graph->inverse_vertices->edges_idx};
     ogpu_graph *gg = NULL;
     if (ogpu_graph_from_arrays(graph->num_vertices, graph->num_edges, arrays, &gg)) return -1;
-    og_plan *pl = NULL;
-    if (og_plan_build((og_graph *)gg, 1, OG_DEFAULT_SEQ_T, 0, need_forward, &pl))
-    {
-        ogpu_graph_free(gg);
-        return -1;
-    }
     memcpy(g_cache.key, key, sizeof(key));
     g_cache.N = graph->num_vertices;
     g_cache.E = graph->num_edges;
     g_cache.g = (og_graph *)gg;
-    g_cache.plan = pl;
     *g = g_cache.g;
-    *plan = pl;
+    return 0;
+}
+
+int og_cache_plan(int need_forward, og_plan **plan)
+{
+    if (!g_cache.plan || (need_forward && !g_cache.plan->push_src))
+    {
+        /* (a push that follows a pull of the same graph gathers its longest rows
+         * in CSR order) */
+        const uint32_t chain_t = need_forward && (g_cache.plan || g_cache.csr_plan) ? OG_DEFAULT_EXACT_ABOVE : 0;
+        og_plan_destroy(g_cache.plan);
+        g_cache.plan = NULL;
+        og_trace_plan("gather");
+        if (og_plan_build(g_cache.g, 1, OG_DEFAULT_SEQ_T, chain_t, need_forward, &g_cache.plan)) return -1;
+    }
+    *plan = g_cache.plan;
+    return 0;
+}
+
+int og_cache_csr_plan(og_plan **plan)
+{
+    if (!g_cache.csr_plan)
+    {
+        og_trace_plan("CSR order");
+        if (og_plan_build(g_cache.g, 2, OG_DEFAULT_SEQ_T, OG_CH, 0, &g_cache.csr_plan)) return -1;
+    }
+    *plan = g_cache.csr_plan;
     return 0;
 }
 
@@ -1409,12 +1424,15 @@ static struct PageRankStats *og_dropin(struct Arguments *arguments, struct Graph
     og_variant_mode(variant, &mode, &push, &quant, &dd);
     og_graph *g = NULL;
     og_plan *plan = NULL;
-    if (og_cache_graph(graph, push || dd, &g, &plan)) og_fatal("graph upload");
+    if (og_cache_graph(graph, &g)) og_fatal("graph upload");
     og_trace_entry("pageRankGraphCSR", g->N, g->E);
     ogpu_pr *pr = NULL;
-    /* the fp32 pull runs binned, on a plan of its own that keeps every row
-     * in CSR order (the cached plan sorts long rows for the gather pulls) */
-    if (og_pr_create_with(g, variant == 0 ? NULL : plan, &o, &pr)) og_fatal("pagerank setup");
+    /* the fp32 pull runs on the direct or binned passes, whose plan keeps every
+     * row in CSR order; the others on the plan of the gather pulls and pushes,
+     * whose long rows, sorted by source, rule those passes out */
+    if ((variant == 0 ? og_cache_csr_plan(&plan) : og_cache_plan(push || dd, &plan)) ||
+        og_pr_create_with(g, plan, &o, &pr))
+        og_fatal("pagerank setup");
 
     struct PageRankStats *stats = newPageRankStatsGraphCSR(graph);
     const char *title = og_variant_title(variant);

@@ -91,12 +91,19 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
 int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int only_streamed, ogpu_pr **out);
 /* Grow an event array to `need` created events. */
 int og_pr_events(hipEvent_t **arr, uint32_t *have, uint32_t need);
-/* The drop-ins' device copy of a caller's GraphCSR and its default plan,
- * cached by pointer and array identity (forward edges when need_forward). */
+/* The drop-ins' device copy of a caller's GraphCSR, cached by pointer and array
+ * identity, and its cached plans: og_plan_build's relabel 1 (with forward edges
+ * when need_forward), and relabel 2 with the rows of more than OG_CH in-edges
+ * first (longest first), as the direct and binned passes build theirs. */
 struct GraphCSR;
-int og_cache_graph(struct GraphCSR *graph, int need_forward, og_graph **g, og_plan **plan);
-/* An SpMV run on graph g over a borrowed plan (NULL: built here). */
-int og_spmv_create_with(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt, ogpu_spmv **out);
+int og_cache_graph(struct GraphCSR *graph, og_graph **g);
+int og_cache_plan(int need_forward, og_plan **plan);
+int og_cache_csr_plan(og_plan **plan);
+/* An SpMV run on graph g over a borrowed plan (NULL: built here).  streamed 0: by
+ * the code's own kernels; otherwise, unless its options or the plan ask for
+ * those, on the direct or binned passes, and where -p 1 to 3 are not faster there
+ * *out stays NULL and 0 is returned. */
+int og_spmv_create_as(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt, int streamed, ogpu_spmv **out);
 
 #ifdef __cplusplus
 }

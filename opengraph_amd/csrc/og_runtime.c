@@ -136,6 +136,13 @@ void og_trace_entry(const char *fn, uint32_t n_vertices, uint32_t n_edges)
             g_cus, n_vertices, n_edges);
 }
 
+/* With OGPU_TRACE, the plans the drop-in entry points build (a later call on the
+ * same graph uses them again). */
+void og_trace_plan(const char *kind)
+{
+    if (getenv("OGPU_TRACE")) fprintf(stderr, "opengraph_amd: plan built (%s)\n", kind);
+}
+
 /* ---- device memory ----
  * A graph's build and a run's setup take dozens of short-lived buffers, and
  * hipMalloc and hipFree (which waits for the device) of the large ones cost

@@ -55,11 +55,12 @@ void ogpu_spmv_free(ogpu_spmv *s)
 
 int ogpu_spmv_create(ogpu_graph *gg, const ogpu_spmv_options *opt_in, ogpu_spmv **out)
 {
-    return og_spmv_create_with((og_graph *)gg, NULL, opt_in, out);
+    const int rc = og_spmv_create_as((og_graph *)gg, NULL, opt_in, 1, out);
+    /* no layout for this graph, or a slower one */
+    return rc || *out ? rc : og_spmv_create_as((og_graph *)gg, NULL, opt_in, 0, out);
 }
 
-/* -p 1 on the streaming passes, or by its partitioned scatter (streamed = 0). */
-static int og_spmv_create_as(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt_in, int streamed, ogpu_spmv **out)
+int og_spmv_create_as(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt_in, int streamed, ogpu_spmv **out)
 {
     *out = NULL;
     ogpu_spmv_options o;
@@ -77,14 +78,15 @@ static int og_spmv_create_as(og_graph *g, og_plan *plan, const ogpu_spmv_options
      * orders its atomics may land in, and u64 sums of the integer terms, all of
      * which fit 32 bits.  An option that asks for a row split, a hot copy or a
      * scatter selects the kernels it is about. */
-    streamed = streamed && !o.hub_threshold && !o.hot_cache && !(o.code == 3 && o.scatter) &&
-               !(plan && plan->relabel == 1 && plan->H);
+    const int plain = !o.hub_threshold && !o.hot_cache && !(o.code == 3 && o.scatter);
+    streamed = streamed && plain && !(plan && plan->relabel == 1 && plan->H);
     s->scatter = (o.code == 1 && !streamed) || (o.code == 3 && o.scatter);
-    s->mode = o.code < 2 ? OG_MODE_F32 : o.code == 2 || streamed ? OG_MODE_FX32 : OG_MODE_FX64;
+    s->narrow = o.code == 3 && plain;
+    s->mode = o.code < 2 ? OG_MODE_F32 : o.code == 2 || s->narrow ? OG_MODE_FX32 : OG_MODE_FX64;
     ogpu_pr_options po;
     ogpu_pr_default_options(&po);
     /* the PageRank variant whose plan, buffers and kernels the passes use */
-    po.variant = o.code < 2 ? o.code : o.code == 2 || streamed ? 9 : (s->scatter ? 3 : 2);
+    po.variant = o.code < 2 ? o.code : o.code == 2 || s->narrow ? 9 : (s->scatter ? 3 : 2);
     po.max_iter = 1;
     po.hub_threshold = o.hub_threshold;
     /* the pushes (-p 1, -p 3 scattered) are partitioned by destination
@@ -95,18 +97,16 @@ static int og_spmv_create_as(og_graph *g, og_plan *plan, const ogpu_spmv_options
      * PageRank push would gather its longest rows instead) */
     if (o.code == 1 && !streamed) po.exact_above = 0;
     po.binned = streamed || (o.code == 0 && !o.hub_threshold) ? 0 : 2;
-    if (og_pr_create_as(g, plan, &po, o.code == 1 && streamed, &s->p))
+    if (og_pr_create_as(g, plan, &po, o.code && streamed, &s->p))
     {
         free(s);
         return -1;
     }
     if (!s->p)
     {
-        /* no layout for this graph, or a slower one */
         free(s);
-        return og_spmv_create_as(g, plan, opt_in, 0, out);
+        return 0;
     }
-    s->narrow = o.code == 3 && streamed;
     s->terms = s->p->c[0];
     if (o.code >= 2)
     {
@@ -321,16 +321,14 @@ static struct SPMVStats *og_spmv_dropin(struct Arguments *arguments, struct Grap
 {
     og_graph *g = NULL;
     og_plan *plan = NULL;
-    if (og_cache_graph(graph, 0, &g, &plan)) og_spmv_fatal("graph upload");
+    if (og_cache_graph(graph, &g)) og_spmv_fatal("graph upload");
     og_trace_entry("SPMVGraphCSR", g->N, g->E);
     ogpu_spmv_options o;
     ogpu_spmv_default_options(&o);
     o.code = code;
     ogpu_spmv *s = NULL;
-    /* on a plan of its own that keeps every row in CSR order (the cached plan
-     * sorts long rows for the gather pulls) */
-    (void)plan;
-    if (og_spmv_create_with(g, NULL, &o, &s)) og_spmv_fatal("spmv setup");
+    if (og_cache_csr_plan(&plan) || og_spmv_create_as(g, plan, &o, 1, &s)) og_spmv_fatal("spmv setup");
+    if (!s && (og_cache_plan(code == 1, &plan) || og_spmv_create_as(g, plan, &o, 0, &s))) og_spmv_fatal("spmv setup");
     struct SPMVStats *stats = newSPMVStatsGraphCSR(graph);
     stats->arguments = arguments;
     /* SPMV.c:663-669: the input vector the passes use */

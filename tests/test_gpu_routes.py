@@ -234,3 +234,44 @@ def test_long_rows_in_small_bins_are_not_a_threads():
         sp.free()
     assert t[0] <= 1.3 * t[1], t
     g.free()
+
+
+@pytest.mark.parametrize("kind", ["rmat", "hub", "tree"])
+def test_dropin_calls_share_their_plans(kind, monkeypatch, capfd):
+    """The drop-in entry points on one graph: each of the two plans is built by
+    the first call that needs it and by no later one."""
+    monkeypatch.setenv("OGPU_TRACE", "1")
+    if kind == "rmat":
+        s, d = og.rmat_host(13, 16 << 13, seed=7)
+    elif kind == "hub":      # -p 2 and 3 by their own kernels
+        s, d = _hub(20_000, 300_000, ROW + 1)
+    else:                    # -p 1 scatters
+        d = np.arange(1, 400_000, dtype=np.uint32)
+        s = (np.random.default_rng(2).random(len(d)) * d).astype(np.uint32)
+    o = po.build_csr(s, d, 0, 8)
+    host = og.HostGraphCSR(o.a)
+
+    def built():
+        return capfd.readouterr().err.count("plan built")
+
+    own = {"rmat": (), "hub": (2, 3), "tree": (1,)}[kind]
+    built()
+    plans = 0
+    for code in (0, 1, 2, 3, 0, 1, 2, 3):
+        y = og.spmv_graph_csr(host, code, 3)[0]
+        if code == 1:
+            np.testing.assert_allclose(y, po.spmv(o, 0, 3), rtol=1e-4)
+        else:
+            assert np.array_equal(y.view(np.uint32), po.spmv(o, code, 3).view(np.uint32)), code
+        plans += built()
+    assert plans == 1 + (1 if own else 0)
+    ranks = og.pagerank_graph_csr(host, 0, 5, 0.0)[0]
+    assert np.array_equal(ranks.view(np.uint32), po.pagerank(o, 0, 0.0, 5, 8)["ranks"].view(np.uint32))
+    assert built() == 0
+    for first in (True, False):
+        for code in (1, 2, 3, 9):
+            ranks = og.pagerank_graph_csr(host, code, 5, 0.0)[0]
+            want = po.pagerank(o, 0 if code == 1 else code, 0.0, 5, 8)["ranks"]
+            np.testing.assert_allclose(ranks, want, rtol=1e-5 if code == 1 else 0, atol=0)
+        n = built()
+        assert n == 0 or (first and n == 1)
