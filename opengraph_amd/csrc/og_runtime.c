@@ -152,7 +152,8 @@ void og_trace_plan(const char *kind)
  * a block's next owner enqueues runs after what its last one did, and none of
  * these pointers leaves the library.  Kept blocks are bounded by a 64th of the
  * device's memory, the longest unused given back first, and all of them are
- * given back before an allocation is allowed to fail. */
+ * given back before an allocation is allowed to fail.  Every block is the library's device's, whichever the
+ * calling thread has chosen: another thread may get it next. */
 typedef struct og_block
 {
     void *p;
@@ -197,6 +198,17 @@ static void og_pool_trim(size_t most)
     }
 }
 
+static hipError_t og_device_malloc(void **p, size_t bytes)
+{
+    int was = g_device;
+    (void)hipGetDevice(&was);
+    hipError_t e = was == g_device ? hipSuccess : hipSetDevice(g_device);
+    if (e == hipSuccess) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();   /* reported by og_dalloc */
+    if (was != g_device) (void)hipSetDevice(was);
+    return e;
+}
+
 void *og_dalloc(size_t bytes)
 {
     const size_t size = og_pool_size(bytes);
@@ -217,13 +229,12 @@ void *og_dalloc(size_t bytes)
         if (b)
         {
             b->bytes = size;
-            e = hipMalloc(&b->p, size);
+            e = og_device_malloc(&b->p, size);
             if (e != hipSuccess)
             {
-                (void)hipGetLastError();
                 og_pool_trim(0);
                 b->bytes = bytes ? bytes : 256;
-                e = hipMalloc(&b->p, b->bytes);
+                e = og_device_malloc(&b->p, b->bytes);
             }
         }
         if (e != hipSuccess)
