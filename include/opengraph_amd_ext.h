@@ -32,6 +32,9 @@ int ogpu_free(void *d_ptr);
 int ogpu_memcpy_h2d(void *d_dst, const void *src, size_t bytes);
 int ogpu_memcpy_d2h(void *dst, const void *d_src, size_t bytes);
 int ogpu_synchronize(void);
+/* Freed device memory is kept for the library's next objects, up to a 64th of
+ * the device's; this gives it back (to other allocators of the process, say). */
+int ogpu_release_memory(void);
 /* Device-to-device copy by a plain streaming kernel (bytes % 16 == 0); the
  * reference point for memory-traffic counters. */
 int ogpu_device_copy(void *d_dst, const void *d_src, size_t bytes);

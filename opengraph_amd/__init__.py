@@ -202,6 +202,7 @@ SIGNATURES = {
     "ogpu_memcpy_h2d": (C.c_int, [_VP, _VP, C.c_size_t]),
     "ogpu_memcpy_d2h": (C.c_int, [_VP, _VP, C.c_size_t]),
     "ogpu_synchronize": (C.c_int, []),
+    "ogpu_release_memory": (C.c_int, []),
     "ogpu_device_copy": (C.c_int, [_VP, _VP, C.c_size_t]),
     "ogpu_rmat_device": (C.c_int, [u32, C.c_uint64, C.c_double, C.c_double, C.c_double, C.c_uint64, C.c_int, _VP, _VP]),
     "ogpu_rmat_host": (C.c_int, [u32, C.c_uint64, C.c_double, C.c_double, C.c_double, C.c_uint64, C.c_int, _VP, _VP]),
@@ -810,6 +811,11 @@ class Spmv:
 
 def synchronize():
     check(load().ogpu_synchronize())
+
+
+def release_memory():
+    """Gives the device memory that the library keeps from freed objects back."""
+    check(load().ogpu_release_memory())
 
 
 def device_copy(dst: DeviceArray, src: DeviceArray, nbytes: int):

@@ -152,7 +152,8 @@ void og_trace_plan(const char *kind)
  * a block's next owner enqueues runs after what its last one did, and none of
  * these pointers leaves the library.  Kept blocks are bounded by a 64th of the
  * device's memory, the longest unused given back first, and all of them are
- * given back before an allocation is allowed to fail.  Every block is the library's device's, whichever the
+ * given back before an allocation is allowed to fail, or when the caller says so
+ * (ogpu_release_memory).  Every block is the library's device's, whichever the
  * calling thread has chosen: another thread may get it next. */
 typedef struct og_block
 {
@@ -446,6 +447,14 @@ int ogpu_malloc(void **ptr, size_t bytes)
     *ptr = NULL;
     og_set_error("hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
     return -1;
+}
+
+int ogpu_release_memory(void)
+{
+    pthread_mutex_lock(&g_pool_lock);
+    og_pool_trim(0);
+    pthread_mutex_unlock(&g_pool_lock);
+    return 0;
 }
 
 int ogpu_free(void *ptr)

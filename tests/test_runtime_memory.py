@@ -53,6 +53,19 @@ def test_blocks_are_the_librarys_devices(lib):
     assert lib.stub_device_of(b) == 1
 
 
+def test_kept_memory_is_bounded_and_given_back(lib):
+    p = [lib.og_dalloc(300_000) for _ in range(10)]
+    for x in p:
+        lib.og_dfree(x)
+    assert 0 < lib.stub_used() <= CAP
+    lib.og_dfree(lib.og_dalloc(2 * MB))      # larger than all that is kept: never kept
+    assert lib.stub_used() <= CAP
+    live = lib.og_dalloc(300_000)
+    assert lib.ogpu_release_memory() == 0
+    assert lib.stub_used() == lib.stub_size_of(live)
+    lib.og_dfree(live)
+
+
 def test_an_allocation_fails_only_without_kept_memory(lib):
     for x in [lib.og_dalloc(300_000) for _ in range(3)]:
         lib.og_dfree(x)
