@@ -350,12 +350,17 @@ static void *og_stage_run(void *arg)
 
 hipError_t og_download(void *dst, const void *src, size_t bytes)
 {
-    hipPointerAttribute_t at;
-    memset(&at, 0, sizeof(at));
-    /* the caller's own pinned (or device) memory takes the copy directly */
-    int plain = bytes < OG_STAGE_MIN ||
-                (hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered);
-    if (bytes >= OG_STAGE_MIN) (void)hipGetLastError();   /* a pointer it does not know */
+    /* the caller's own pinned (or device) memory takes the copy directly; so does
+     * a thread with an error pending, which asking about an unknown pointer
+     * could replace */
+    int plain = bytes < OG_STAGE_MIN || hipPeekAtLastError() != hipSuccess;
+    if (!plain)
+    {
+        hipPointerAttribute_t at;
+        memset(&at, 0, sizeof(at));
+        if (hipPointerGetAttributes(&at, dst) == hipSuccess) plain = at.type != hipMemoryTypeUnregistered;
+        else (void)hipGetLastError();
+    }
     if (plain) return og_copy(dst, src, bytes, hipMemcpyDeviceToHost);
     pthread_mutex_lock(&g_stage_lock);
     if (!og_stage_ready())

@@ -76,3 +76,20 @@ def test_an_allocation_fails_only_without_kept_memory(lib):
     assert lib.stub_last() == 0              # reported, not left for another call to find
     lib.og_dfree(a)
     assert lib.og_dalloc(1)
+
+
+@pytest.mark.parametrize("known", [0, 1])
+@pytest.mark.parametrize("words", [1, MB - 1, MB, 9 * MB // 4 + 3])
+def test_download_leaves_the_threads_state(lib, known, words):
+    """Data whole, the thread's device and its pending error as they were."""
+    lib.stub_known(known)
+    src = (C.c_uint32 * words)(*([0] * 7)) if words >= 7 else (C.c_uint32 * words)()
+    for i in range(0, words, 4099):
+        src[i] = i * 2654435761 % (1 << 32)
+    src[words - 1] = 77
+    for device, error in ((0, 0), (1, 0), (0, 1), (1, 719)):
+        dst = (C.c_uint32 * words)()
+        lib.stub_set(device, error)
+        assert lib.og_download(dst, src, words * 4) == 0
+        assert (lib.stub_current(), lib.stub_last()) == (device, error)
+        assert bytes(dst) == bytes(src)
