@@ -1,5 +1,6 @@
-"""The wavefront sums of the binned pull (og_bin.hip, og_bin_wave_step)
-restated on the CPU: T consecutive terms per lane, each lane's run as the
+"""The wavefront sums of the binned and direct pulls (og_rowsum.h,
+og_bin_wave_step) restated on the CPU: T consecutive terms per lane (36 in the
+binned pull's steps, 28 in the direct one's, 12 in a short last one), each lane's run as the
 moves of an even and of an odd running sum, the runs composed in lane order,
 the first lane that leaves the binade added term by term.  Bar: the bits of
 the sequential fp32 sum, by brute force.  Two planted mistakes -- one move per
@@ -75,13 +76,13 @@ KINDS = ["few bits", "ranks", "power law", "equal", "zeros"]
 
 
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("n", [1, 27, 28, 29, 1791, 1792, 1793, 6000])
+@pytest.mark.parametrize("n", [1, 27, 28, 29, 36, 37, 63, 64, 65, 1791, 1792, 1793, 2303, 2304, 2305, 6000])
 def test_equal_to_the_sequential_sum(kind, n):
     rng = np.random.default_rng(n)
     x = terms(kind, n, rng)
     for y0 in (0.0, 0.3, 1e-5, 7.99999):
         want = seq(y0, x)
-        for T, lanes in ((28, 64), (12, 64), (4, 8)):
+        for T, lanes in ((36, 64), (28, 64), (12, 64), (4, 8)):
             assert bits(wave_sum(x, y0, T, lanes)) == bits(want), (kind, n, y0, T)
 
 
@@ -101,3 +102,18 @@ def test_terms_that_are_not_positive_and_finite():
         y[at] = a
         got, want = wave_sum(y, 0.0, 28, 64), seq(0.0, y)
         assert bits(got) == bits(want) or (np.isnan(got) and np.isnan(want))
+
+
+def test_zeros_and_leading_zeros():
+    x = np.zeros(3000, F)
+    for T in (36, 28, 12):
+        assert bits(wave_sum(x, 0.0, T, 64)) == 0
+    x[1500:] = F(1e-3)
+    for T in (36, 28, 12):
+        assert bits(wave_sum(x, 0.0, T, 64)) == bits(seq(0.0, x))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_long_rows(kind):
+    x = terms(kind, 40_000, np.random.default_rng(40))
+    assert bits(wave_sum(x, 0.0, 36, 64)) == bits(seq(0.0, x))

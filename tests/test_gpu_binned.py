@@ -6,7 +6,7 @@ Bar: bit-exact.  Every row is the reference's running fp32 sum over its
 in-edges in CSR order (pageRank.c:998-1011): thread rows add from LDS one
 term at a time; wavefront rows and rows longer than a bin (cut into pieces,
 added by one block) use the exact binade fast-forward, pinned on the CPU by
-tests/test_bin_scan.py.  Cases: every golden fp32-pull case; a graph with
+tests/test_bin_moves.py.  Cases: every golden fp32-pull case; a graph with
 hubs just under, at and well over the bin capacity whose in-neighbours have
 small out-degrees (few-bit contributions: many half-ulp ties in the long
 sums); R-MAT scales 18 and 20; Erdos-Renyi with a vertex count that is

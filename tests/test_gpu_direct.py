@@ -51,9 +51,10 @@ def _same(src, dst, eps, iters, **kw):
     [1], [1, 1, 1], [3] * 512, [3] * 513, [511, 512, 513, 514], [64, 65, 575, 1344, 2368, 2369],
     [EDGES - 1, EDGES, EDGES + 1], [BATCH - 1, BATCH, BATCH + 1, 2 * BATCH + 1], [CAP - 1, CAP, CAP + 1],
     [5 * CAP // 2, 7], [8] * 20_000, [40] * 3000 + [2] * 9000])
-def test_row_and_block_edges(degrees):
+@pytest.mark.parametrize("relabel", [1, 0])   # by in-degree, and in the caller's order
+def test_row_and_block_edges(degrees, relabel):
     src, dst = _graph(30_011, degrees, sum(degrees))
-    _same(src, dst, 0.0, 7)
+    _same(src, dst, 0.0, 7, relabel=relabel)
 
 
 @pytest.mark.parametrize("edges", [32 * EDGES, 64 * EDGES - 5, 65 * EDGES, 300_000])

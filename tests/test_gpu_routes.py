@@ -53,8 +53,15 @@ def _check(s, d, codes=(2, 3, 4, 9), spmv=(2, 3), relabel=1, iters=4):
 @pytest.mark.parametrize("degrees", [
     [WAVE - 1, WAVE, WAVE + 1], [WAVE + 1], [EDGES - 1, EDGES, EDGES + 1], [EDGES // 2] * 3, [511, 512, 513, 575],
     [CAP - 1, CAP, CAP + 1, CAP // 2], [CAP + 511, 1, 1], [2 * CAP, 2 * CAP + 1, 300] + [3] * 2000])
-def test_long_integer_rows_of_the_direct_pull(degrees):
-    _check(*_rows(degrees, 30_011, sum(degrees)))
+@pytest.mark.parametrize("relabel", [1, 0])
+def test_long_integer_rows_of_the_direct_pull(degrees, relabel):
+    _check(*_rows(degrees, 30_011, sum(degrees)), spmv=(2, 3) if relabel else (), relabel=relabel)
+
+
+@pytest.mark.parametrize("relabel", [1, 0])
+def test_integer_modes_past_the_direct_pull(relabel):
+    s, d = og.rmat_host(18, 9_000_000, seed=3)
+    _check(s, d, spmv=(), relabel=relabel, iters=3)
 
 
 def _best(f, n=15):

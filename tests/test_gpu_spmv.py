@@ -100,11 +100,13 @@ def test_default_rows_and_push_within_bound(golden, gname):
             y = _run(g, 0, 20, hub_threshold=16, hot_cache=hot)
             assert np.array_equal(y[short].view(np.uint32), ref[short].view(np.uint32)), hot
             assert np.all(np.abs(y.astype(np.float64) - want) <= bound), hot
-        for hot in (0, 2):          # LDS accumulators (default for -p 1) and plain atomics
-            y = _run(g, 1, 20, hot_cache=hot)
-            assert np.all(np.abs(y.astype(np.float64) - want) <= bound), ("push", hot)
+        # -p 1: the streaming passes (default), the partitioned scatter's LDS
+        # accumulators (any hub_threshold), the scatter's, and plain atomics
+        for kw in (dict(), dict(hub_threshold=16), dict(hot_cache=1), dict(hot_cache=2)):
+            y = _run(g, 1, 20, **kw)
+            assert np.all(np.abs(y.astype(np.float64) - want) <= bound), ("push", kw)
             # the reference's (single-thread) output obeys the same bound
-            assert np.all(np.abs(y.astype(np.float64) - ref) <= 2 * bound), ("push", hot)
+            assert np.all(np.abs(y.astype(np.float64) - ref) <= 2 * bound), ("push", kw)
     finally:
         g.free()
 
@@ -168,8 +170,9 @@ def test_scale20_fp32(rmat20):
     assert np.all(np.abs(y.astype(np.float64) - want) <= bound)
     y = _run(g, 0, 8, hub_threshold=ALL_EXACT)
     assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
-    y = _run(g, 1, 8)
-    assert np.all(np.abs(y.astype(np.float64) - want) <= bound)
+    for kw in (dict(), dict(hub_threshold=16)):
+        y = _run(g, 1, 8, **kw)
+        assert np.all(np.abs(y.astype(np.float64) - want) <= bound), kw
 
 
 def test_dropin_spmv_graph_csr(golden):

@@ -2,7 +2,9 @@
 bit-exact against the oracle, the fp32 push within the reference's own spread
 (1e-5) -- and, since its destinations add in source order here, equal to the
 sequential pull.  Sizes: the direct pull's and, past 8 M edges, the binned
-one's; rows at the edges of a thread's, a wavefront's and a bin's."""
+one's ("large", and "binned edges" with rows at its bins' and pieces' ends);
+rows at the edges of a thread's, a wavefront's and a block's in the direct
+one."""
 import numpy as np
 import pytest
 
@@ -11,7 +13,8 @@ from oracle import pyoracle as po
 
 pytestmark = pytest.mark.gpu
 
-CAP, WAVE = 19968, 192
+CAP = 19968      # in-edge values of a block's LDS
+WAVES = [127, 128, 129, 511, 512, 513]   # the direct pull's thread rows: up to 128 integers, 512 fp32
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -29,13 +32,16 @@ def _rows(seed, degrees, n):
 
 def _graph(kind):
     if kind == "edges":
-        return _rows(1, [CAP - 1, CAP, CAP + 1, 2 * CAP + 5, WAVE - 1, WAVE, WAVE + 1] + [7] * 600 + [1] * 900, 20_003)
+        return _rows(1, [CAP - 1, CAP, CAP + 1, 2 * CAP + 5] + WAVES + [7] * 600 + [1] * 900, 20_003)
     if kind == "small":
         return og.rmat_host(12, 50_000, seed=4)
+    if kind == "binned edges":    # bins of 4.6 k in-edges
+        deg = [CAP - 1, CAP, CAP + 1, 2 * CAP, 2 * CAP + 1, 4600, 2300, 2301, 513] + WAVES
+        return _rows(2, deg + [9] * 900_000 + [1] * 900_000, 2_000_003)
     return og.rmat_host(19, 9_000_000, seed=7)
 
 
-@pytest.mark.parametrize("kind", ["edges", "small", "large"])
+@pytest.mark.parametrize("kind", ["edges", "small", "large", "binned edges"])
 def test_variants_against_the_oracle(kind):
     s, d = _graph(kind)
     g = og.Graph.from_edges(s, d, 0)
@@ -54,7 +60,7 @@ def test_variants_against_the_oracle(kind):
     g.free()
 
 
-@pytest.mark.parametrize("kind", ["edges", "small", "large"])
+@pytest.mark.parametrize("kind", ["edges", "small", "large", "binned edges"])
 def test_spmv_codes_against_the_oracle(kind):
     s, d = _graph(kind)
     g = og.Graph.from_edges(s, d, 0)
