@@ -29,10 +29,19 @@
 /* runs that go one iteration a launch after the direct pull's blocks could not
  * all be resident; then it is tried again */
 #define OG_DIR_SINGLE_RUNS 32u
-/* past this many in-edges the binned pull's streaming passes are as fast
- * (R-MAT-18, 4.2 M edges: 34 us an iteration direct, 42 binned; R-MAT-17 25 and
- * 33; uniform, 2 M: 18 and 23) */
+/* In-edges up to which the direct pull is the faster one: as many as its blocks
+ * hold where the gathered array is within the L1s' reach (2^14 vertices) or the sums are
+ * serial (fp32), fewer where its gathers from L2 are what counts, fewest in a
+ * SpMV, which has no final reduction whose launch the direct form saves.  us an
+ * iteration or pass, binned and direct.  u64 pull: 8 k vertices, 8 M edges 49 and
+ * 28; 50 k, 4 M 33 and 31, 6 M 43 and 42, 8 M 50 and 56; 250 k, 6 M 42 and 40, 8 M 48 and
+ * 49; R-MAT-17, 6 M 55 and 44, 8 M 66 and 68.  fp32 pull: 50 k, 8 M 47 and 42; 250 k,
+ * 8 M 46 and 48; R-MAT-17, 8 M 74 and 74.  SpMV -p 0: 8 k, 8 M 44 and 31; 3 M at 50 k
+ * 23 and 21, at 250 k 23 and 23; 4 M 25 and 25, 25 and 28; 8 M 41 and 43, 39 and 48. */
 #define OG_DIR_MAX_EDGES (1u << 23)
+#define OG_DIR_MAX_EDGES_INT (6u << 20)
+#define OG_DIR_MAX_EDGES_SPMV (3u << 20)
+#define OG_DIR_NEAR (1u << 14)
 /* A streamed row is added by one block, 0.3 to 0.55 ns a term whatever its
  * length; the integer variants' own pulls cut a long row into chunks for the
  * whole device.  Longest row an integer pull streams: OG_ROW_ALWAYS terms, or
@@ -342,7 +351,7 @@ int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, og
     return og_pr_create_as(g, plan, opt, 0, out);
 }
 
-int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int only_streamed, ogpu_pr **out)
+int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int spmv, ogpu_pr **out)
 {
     *out = NULL;
     if (og_ctx_ensure()) return -1;
@@ -434,20 +443,22 @@ int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int 
     }
     const uint32_t max_row = p->mode == OG_MODE_F32 || p->push ? 0xFFFFFFFFu
                            : E / OG_ROW_FRACTION > OG_ROW_ALWAYS ? E / OG_ROW_FRACTION : OG_ROW_ALWAYS;
+    const uint32_t dir_edges = N <= OG_DIR_NEAR ? OG_DIR_MAX_EDGES : spmv ? OG_DIR_MAX_EDGES_SPMV
+                             : p->mode != OG_MODE_F32 ? OG_DIR_MAX_EDGES_INT : OG_DIR_MAX_EDGES;
     /* a small graph's pull runs direct unless the binned one is asked for */
     if (binned && opt->binned != 1 && !p->quant &&
-        og_dir_plan_build(p->plan, p->mode, OG_DIR_MAX_EDGES, max_row, &p->dir))
+        og_dir_plan_build(p->plan, p->mode, dir_edges, max_row, &p->dir))
     {
         ogpu_pr_free(p);
         return -1;
     }
     const int dense = p->mode != OG_MODE_F32 && !p->push && E / OG_DENSE_DEGREE > N;
-    /* SpMV -p 1 (only_streamed): its scatter over rows of about one in-edge is
+    /* SpMV -p 1: its scatter over rows of about one in-edge is
      * one short launch (us a pass, scattered and binned: 1 M vertices on a ring 15
      * and 23, 4 M 47 and 66, a random tree of 8 M 105 and 122; 1.6 in-edges a row, 1 M
      * 19 and 16, 4 M 79 and 58; many more vertices than in-edges, whose y the scatter goes
      * through, 50 and 32) */
-    const int ones = only_streamed && opt->variant == 1 && 2ull * E < 3ull * p->plan->Z && 2ull * E >= N;
+    const int ones = spmv && opt->variant == 1 && 2ull * E < 3ull * p->plan->Z && 2ull * E >= N;
     const uint64_t max_entries = opt->variant ? (uint64_t)(OG_ENTRIES_PER_EDGE * E) : ~0ull;
     if (binned && !p->dir && !dense && !ones && og_bin_plan_build(p->plan, p->mode, max_row, max_entries, &p->bins))
     {
@@ -460,7 +471,7 @@ int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int 
     }
     if (p->bins) p->n_final_bin = og_final_blocks(p->bins->sum_grid, 0);
     const int streamed = p->bins || p->dir;
-    if (only_streamed && !streamed)
+    if (spmv && opt->variant && !streamed)
     {
         ogpu_pr_free(p);
         return 0;

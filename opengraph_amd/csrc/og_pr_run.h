@@ -86,9 +86,9 @@ struct ogpu_pr
 /* Create a run of opt->variant on graph g; plan may be supplied (borrowed)
  * or is built here.  Buffers are allocated, the state is not initialized. */
 int og_pr_create_with(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, ogpu_pr **out);
-/* The same; only_streamed: *out stays NULL (and 0 is returned) where the run
- * would not be on the direct or binned passes. */
-int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int only_streamed, ogpu_pr **out);
+/* The same; spmv: for SpMV passes on the direct or binned passes.  Where a
+ * variant other than 0 would not be on them *out stays NULL (and 0 is returned). */
+int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int spmv, ogpu_pr **out);
 /* Grow an event array to `need` created events. */
 int og_pr_events(hipEvent_t **arr, uint32_t *have, uint32_t need);
 /* The drop-ins' device copy of a caller's GraphCSR, cached by pointer and array

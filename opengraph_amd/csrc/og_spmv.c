@@ -97,7 +97,7 @@ int og_spmv_create_as(og_graph *g, og_plan *plan, const ogpu_spmv_options *opt_i
      * PageRank push would gather its longest rows instead) */
     if (o.code == 1 && !streamed) po.exact_above = 0;
     po.binned = streamed || (o.code == 0 && !o.hub_threshold) ? 0 : 2;
-    if (og_pr_create_as(g, plan, &po, o.code && streamed, &s->p))
+    if (og_pr_create_as(g, plan, &po, streamed, &s->p))
     {
         free(s);
         return -1;

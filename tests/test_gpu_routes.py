@@ -282,3 +282,13 @@ def test_dropin_calls_share_their_plans(kind, monkeypatch, capfd):
             np.testing.assert_allclose(ranks, want, rtol=1e-5 if code == 1 else 0, atol=0)
         n = built()
         assert n == 0 or (first and n == 1)
+
+
+@pytest.mark.parametrize("n", [1 << 14, (1 << 14) + 1])
+@pytest.mark.parametrize("edges", [3 << 20, (3 << 20) + 1, 6 << 20, (6 << 20) + 1, 8 << 20, (8 << 20) + 1])
+def test_largest_direct_graphs(n, edges):
+    """Sizes around the direct pull's limits, SpMV's and the pulls', near and far."""
+    rng = np.random.default_rng(edges)
+    s, d = (rng.integers(0, n, edges).astype(np.uint32) for _ in range(2))
+    s[0] = n - 1
+    _check(s, d, codes=(2,) if edges <= (3 << 20) + 1 else (0, 9), spmv=(0, 2) if edges <= (3 << 20) + 1 else (), iters=2)
