@@ -387,8 +387,7 @@ int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int 
      * R-MAT-22, 377 us by the hot-cache gather, 235 streamed (the partitioned
      * u64 push likewise); fp32 push, R-MAT-20, 243 us by ranges with their
      * chains beside them, 80 streamed. */
-    if (!binned && (opt->variant == 1 || opt->variant == 2 || opt->variant == 3 || opt->variant == 4 ||
-                    opt->variant == 9) &&
+    if (opt->variant && og_bin_mode(p->mode) && !p->dd &&
         opt->binned == 0 && !opt->hub_threshold && !opt->hot_cache && g->E > 0 &&
         !(opt->variant == 1 && !opt->exact_above) && !(p->quant && E < OG_QUANT_MIN_EDGES) &&
         !(plan && plan->relabel == 1 && plan->H))
