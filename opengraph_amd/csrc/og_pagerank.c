@@ -48,12 +48,13 @@
  * this fraction of all of them.  us an iteration of the u64 / u32 pull by their
  * own kernels and streamed, uniform sources: 1 M edges, a row of 33 k 37 / 25 and
  * 28 / 23, of 66 k 37 / 25 and 43 / 35, of 210 k 37 / 25 and 118 / 91; 4 M edges, a row of
- * 1/64th of them 69 / 61 and 54 / 47, of 1/32nd 68 / 60 and 80 / 66; 64 M edges, 1/64th
- * 1185 / 1028 and 584 / 476, 1/16th 1137 / 998 and 1880 / 1403.  (The SpMV of
- * the 33 k row loses, 18 and 21 us.  The u64 push adds a destination serially
- * too and is slower at every length.) */
+ * a 64th of them 69 / 61 and 54 / 47, a 40th 69 / 61 and 69 / 57, a 32nd 68 / 60 and
+ * 80 / 66; 64 M edges, a 40th 1186 / 1031 and 825 / 650, a 32nd 1174 / 1020 and 1016 /
+ * 784, a 16th 1137 / 998 and 1880 / 1403.  (The SpMV of the 33 k row loses, 18 and
+ * 21 us.  The u64 push adds a destination serially too and is slower at every
+ * length.) */
 #define OG_ROW_ALWAYS 24576u
-#define OG_ROW_FRACTION 64u
+#define OG_ROW_FRACTION 40u
 /* Average in-degree past which an integer pull that does not run direct keeps
  * its own kernel: its few contributions then all lie in the LDS copy, and 4
  * bytes an edge beat the passes' 14 (u64 and u32 pull, own kernels and streamed:

@@ -107,18 +107,18 @@ def _hub(n, edges, hub, seed=3):
     return s, d
 
 
-ROW = 24576      # an integer row that is always streamed; longer: a 64th of the in-edges
+ROW = 24576      # an integer row that is always streamed; longer: a 40th of the in-edges
 
 
 @pytest.mark.parametrize("edges,hub", [(300_000, ROW - 1), (300_000, ROW), (300_000, ROW + 1),
-                                       (64 * ROW + 64, ROW + 1), (64 * ROW + 64, ROW + 2)])
+                                       (40 * ROW + 40, ROW + 1), (40 * ROW + 40, ROW + 2)])
 def test_integer_rows_at_the_longest_streamed(edges, hub):
     s, d = _hub(20_000, edges, hub)
     assert np.bincount(d).max() == hub
     _check(s, d)
     g = og.Graph.from_edges(s, d, 0)
     pr = og.PageRank(g, 2, 2, 0.0)      # its bytes per iteration tell its passes
-    streamed = hub <= max(ROW, edges // 64)
+    streamed = hub <= max(ROW, edges // 40)
     n = g.num_vertices
     assert pr.bytes_per_iteration() == (8 * edges + 20 * n if streamed else 12 * edges + 24 * n)
     pr.free()
