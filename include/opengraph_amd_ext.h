@@ -147,14 +147,21 @@ typedef struct
                                atomic adds */
     uint32_t binned;        /* fp32 pull (variant 0, not personalized): 0 default (on),
                                1 on, 2 off; variants 1 (with exact_above), 2, 3, 4 and 9:
-                               0 on unless hub_threshold or hot_cache is given, else off
+                               0 on unless hub_threshold or hot_cache is given, else off;
+                               but off where the variant's own kernels are faster (2, 4, 9:
+                               a row of more than a 40th of the in-edges and 24576, more
+                               than 2048 in-edges a vertex past the direct sizes; 4: less
+                               than 2^21 in-edges; all: short rows over so many segments
+                               that padding takes the layout past 5.5 entries an edge)
                                -- the binned passes: per iteration a gather pass
                                writes each edge's contribution, source segment by source
                                segment from LDS, into an edge array grouped by destination
                                bins, and a sum pass adds every row from LDS in CSR order
-                               (rows longer than a bin by one block each); with 0 and up
-                               to 2^23 edges one launch runs all iterations instead,
-                               gathering through L2, with the same sums.  Every fp32 row
+                               (rows longer than a bin by one block each); with 0 and a
+                               small graph (variants 0 to 3 and 9; at most 262,144 rows
+                               with in-edges, and 2^23 in-edges, 6 x 2^20 in the integer
+                               variants past 2^14 vertices) one launch runs all iterations
+                               instead, gathering through L2, with the same sums.  Every fp32 row
                                is the reference's running sum to the bit, and all global
                                accesses stream.  hub_threshold, exact_above and hot_cache
                                then apply only to the learned start's feature pass */
@@ -379,7 +386,10 @@ void ogpu_ppr_free(ogpu_ppr *p);
  *   2 pull, Q16.16 inputs, u64 sums of (7 * x) >> 16 (bit-exact);
  *   3 push, Q32.32, u64 sums of (w * x) >> 32 (bit-exact): gathered over
  *     the in-edges by default, scattered with u64 atomics when scatter = 1.
- * By default every code runs on the streaming passes (ogpu_pr_options.binned). */
+ * By default every code runs on the streaming passes (ogpu_pr_options.binned;
+ * direct up to 3 x 2^20 in-edges, 2^23 at up to 2^14 vertices), codes 1 to 3
+ * where they are the faster ones: 2 and 3 as the integer variants, 1 by its
+ * scatter on rows of about one in-edge and past 5.5 entries an edge. */
 typedef struct ogpu_spmv ogpu_spmv;
 typedef struct
 {

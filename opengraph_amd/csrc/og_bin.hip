@@ -214,11 +214,12 @@ __device__ __forceinline__ void og_bin_put(const og_bin_dev &b, float *slot, con
 /* Block i takes the bins sched[blk[i], blk[i + 1]) in that order (a long
  * row's pieces one after the other); integer modes put all the block's
  * threads on a bin's rows, a power of two each (a thread per row, the fp32
- * split, left most of them idle: 400 us at R-MAT-22, now 128); then, while rows without in-edges still
- * change, every gridDim.x-th of their bins.  Bound by the streamed entries (6
- * bytes each); two blocks a CU, so that one's rows overlap the other's
- * entries.  R-MAT-24: 445 us = 4.0 TB/s (567 us beside a long-row kernel on
- * CUs of its own before); R-MAT-22: 117 us, where that kernel's longest row
+ * split, left most of them idle: 400 us at R-MAT-22, now 128); then, while rows
+ * without in-edges still change, every gridDim.x-th of their bins.  Bound by the
+ * streamed entries (6 bytes each), at smaller sizes by the wavefront rows; two
+ * blocks a CU, so that one's rows overlap the other's entries.  R-MAT-24: 449 us
+ * = 4.7 TB/s by the HBM counters, as the gather pass (567 us beside a long-row
+ * kernel on CUs of its own before); R-MAT-22: 117 us, where that kernel's longest row
  * took 158; R-MAT-16, whose wavefront rows bound it: 17 us against 33. */
 template <int MODE>
 __global__ __launch_bounds__(BT, 4) void og_bin_sum_kernel(og_bin_dev b, og_pr_dev a)
