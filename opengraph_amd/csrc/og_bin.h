@@ -1,5 +1,5 @@
 /*
- * og_bin.h -- the binned fp32 pull (og_bin.hip, og_bin.c): pageRank.c:998-1011
+ * og_bin.h -- the binned pull (og_bin.hip, og_bin.c): pageRank.c:998-1011
  * as two streaming passes over an edge layout built once per graph.
  *
  * Rows (new ids, the plan's CSR order kept) are packed into bins whose

@@ -1,5 +1,5 @@
 /*
- * og_bin.hip -- gfx950 kernels of the binned fp32 pull (layout and passes
+ * og_bin.hip -- gfx950 kernels of the binned pull (layout and passes
  * described in og_bin.h) and of its one-time layout build.
  *
  * Row sums and their exactness: og_rowsum.h.

@@ -59,10 +59,10 @@ struct ogpu_pr
     double *lscratch;
     /* every-row-exact fp32 pull: rows [0, C) longest first (device) */
     uint32_t *chain_rows;
-    /* binned fp32 pull (og_bin.h): layout, blocks of its final reduction */
+    /* binned pull (og_bin.h): layout, blocks of its final reduction */
     struct og_bin_plan *bins;
     uint32_t n_final_bin;
-    /* direct fp32 pull (og_dir.h): the iterations of a small graph in one
+    /* direct pull (og_dir.h): the iterations of a small graph in one
      * launch */
     struct og_dir_plan *dir;
     uint32_t dir_single;      /* runs left to go one iteration a launch */

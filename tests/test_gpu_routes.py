@@ -154,7 +154,7 @@ def test_quantized_pull_at_its_first_streamed_size(edges):
 
 @pytest.mark.parametrize("scale", [4, 12, 14, 16])
 def test_small_quantized_pull_is_not_the_slower_form(scale):
-    _not_the_slower_form(*og.rmat_host(scale, 16 << scale, seed=9), codes=(4,), spmv=(), most=1.15)
+    _not_the_slower_form(*og.rmat_host(scale, 16 << scale, seed=9), codes=(4,), spmv=(), most=1.2)
 
 
 def _permutation(n, seed=5):
