@@ -150,8 +150,8 @@ typedef struct
                                0 on unless hub_threshold or hot_cache is given, else off;
                                but off where the variant's own kernels are faster (2, 4, 9:
                                a row of more than a 40th of the in-edges and 24576, more
-                               than 2048 in-edges a vertex past the direct sizes; 4: less
-                               than 2^21 in-edges; all: short rows over so many segments
+                               than 2048 in-edges a vertex past the direct sizes; 4, and 2
+                               with relabel 0: less than 2^21 in-edges; all: short rows over so many segments
                                that padding takes the layout past 5.5 entries an edge)
                                -- the binned passes: per iteration a gather pass
                                writes each edge's contribution, source segment by source

@@ -17,7 +17,7 @@
  * block adds a row that is alone in it (every row of more than OG_DIR_EDGES is):
  * u64 pull, R-MAT-17 with 6 M edges 92 us an iteration by one wavefront, now
  * 39; one row of 210 k among 1 M edges 317 and 118. */
-#define OG_DIR_WAVE_ROW 512u
+#define OG_DIR_WAVE_ROW OG_CH
 #define OG_DIR_WAVE_ROW_INT 128u
 
 void og_dir_plan_destroy(og_dir_plan *b)
@@ -90,10 +90,16 @@ int og_dir_plan_build(const og_plan *pl, int mode, uint32_t max_edges, uint32_t 
     }
     if (og_bin_runs(pl, &run, &n_runs)) goto done;
     uint32_t n = most + 1;
+    /* A plan in the caller's order groups its rows at OG_CH only, a bin holds one
+     * kind, and another line cuts one at every other row: u32 pull, R-MAT-16, 28 us
+     * an iteration with the integer line, 15 without; a thread takes long over a
+     * u64 row, so small graphs keep it there (R-MAT-12 14 and 25, R-MAT-17 50
+     * and 32). */
+    const int by_degree_line = pl->relabel || (mode == OG_MODE_FX64 && E < (1u << 21));
+    const uint32_t wave_row = mode != OG_MODE_F32 && by_degree_line ? OG_DIR_WAVE_ROW_INT : OG_DIR_WAVE_ROW;
     const int fits = og_bin_longest(run, n_runs) <= max_row;
     for (uint64_t cap = OG_DIR_EDGES; fits && n > most && cap <= OG_DIR_CAP; cap += cap / 4)
-        if ((uint64_t)E <= cap * most) n = og_dir_pack(run, n_runs, Z, (uint32_t)cap, mode == OG_MODE_F32 ? OG_DIR_WAVE_ROW : OG_DIR_WAVE_ROW_INT,
-                            bins, most);
+        if ((uint64_t)E <= cap * most) n = og_dir_pack(run, n_runs, Z, (uint32_t)cap, wave_row, bins, most);
     if (n > most)
     {
         rc = 0;

@@ -75,6 +75,9 @@
  * R-MAT-17, 2 M 37 and 37; R-MAT-18, 3 M 54 and 37, 4 M 61 and 42; uniform, 1 M vertices,
  * 2 M 48 and 44. */
 #define OG_QUANT_MIN_EDGES (1u << 21)
+/* The same for the u64 pull over rows in the caller's order (relabel 0), whose
+ * kinds of rows alternate: R-MAT-14 22 and 26, R-MAT-16 26 and 38, R-MAT-17 46 and 32. */
+#define OG_UNSORTED_MIN_EDGES (1u << 21)
 /* Rows with more in-edges than this go to the chunk waves: 12..16 is the
  * fastest on R-MAT 24 (1.38-1.40 ms against 1.47 at 32 and 1.50 at 4) and
  * on Erdos-Renyi 24 (4.80-4.87 ms against 5.08 at 32). */
@@ -391,6 +394,7 @@ int og_pr_create_as(og_graph *g, og_plan *plan, const ogpu_pr_options *opt, int 
     if (opt->variant && og_bin_mode(p->mode) && !p->dd &&
         opt->binned == 0 && !opt->hub_threshold && !opt->hot_cache && g->E > 0 &&
         !(opt->variant == 1 && !opt->exact_above) && !(p->quant && E < OG_QUANT_MIN_EDGES) &&
+        !(opt->variant == 2 && !plan && !opt->relabel && E < OG_UNSORTED_MIN_EDGES) &&
         !(plan && plan->relabel == 1 && plan->H))
         binned = 1;
     if (opt->binned == 1 && !binned)

@@ -73,7 +73,7 @@ def _best(f, n=15):
     return min(t)
 
 
-def _not_the_slower_form(s, d, codes, spmv, most=1.4):
+def _not_the_slower_form(s, d, codes, spmv, most=1.4, **opt):
     """A default run takes at most `most` times what the variant's own kernels
     take (binned = 2; SpMV: a hub_threshold); best of fifteen runs each, 20
     iterations."""
@@ -81,7 +81,7 @@ def _not_the_slower_form(s, d, codes, spmv, most=1.4):
     for code in codes:
         t = []
         for kw in (dict(), dict(binned=2)):
-            pr = og.PageRank(g, code, 20, 0.0, **kw)
+            pr = og.PageRank(g, code, 20, 0.0, **opt, **kw)
             pr.run()
             t.append(_best(pr.run))
             pr.free()
@@ -292,3 +292,8 @@ def test_largest_direct_graphs(n, edges):
     s, d = (rng.integers(0, n, edges).astype(np.uint32) for _ in range(2))
     s[0] = n - 1
     _check(s, d, codes=(2,) if edges <= (3 << 20) + 1 else (0, 9), spmv=(0, 2) if edges <= (3 << 20) + 1 else (), iters=2)
+
+
+@pytest.mark.parametrize("scale", [14, 16])
+def test_integer_pulls_in_the_callers_order(scale):
+    _not_the_slower_form(*og.rmat_host(scale, 16 << scale, seed=9), codes=(2, 9), spmv=(), most=1.2, relabel=0)
