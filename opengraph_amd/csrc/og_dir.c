@@ -108,10 +108,11 @@ int og_dir_plan_build(const og_plan *pl, int mode, uint32_t max_edges, uint32_t 
         goto done;
     }
     b->d.n_bins = n;
-    /* polls of the barrier before a block gives up: a poll takes about 0.7 us and
-     * an iteration microseconds, or up to 0.55 ns per in-edge of its longest block,
-     * so 11 ms and five times the latter (OG_DIR_SPIN: another limit, small ones
-     * for tests of the fallback) */
+    /* polls of the barrier before a block gives up: a poll (64 cycles of sleep and
+     * a round trip to memory) takes upwards of half a microsecond, an iteration
+     * microseconds, or up to 0.55 ns per in-edge of its longest block, so some 10
+     * ms and a few times the latter (OG_DIR_SPIN: another limit, small ones for
+     * tests of the fallback) */
     uint32_t most_edges = 0;
     for (uint32_t i = 0; i < n; i++) most_edges = bins[i].cnt > most_edges ? bins[i].cnt : most_edges;
     const char *spin = getenv("OG_DIR_SPIN");
